@@ -21,8 +21,16 @@ namespace
 {
 
 constexpr int kBlock = 256;
-constexpr int kLanes = 4;                      // lanes per row (P1 rows ~15)
-constexpr int kRowsPerChunk = kBlock / kLanes; // rows per chunk / workgroup
+constexpr int kLanes = 4;                // lanes per row (P1 rows ~15)
+constexpr int kSteps = 4;                // entries per lane loaded together
+constexpr int kRowsPerPass = kBlock / kLanes;
+// Rows per chunk. A chunk is the unit of the reductions (one partial per
+// chunk), so its size fixes how many partials every workgroup re-sums: with
+// 64 rows the 117,649 rows of a 48^3 mesh had 1,839 partials re-summed for
+// every chunk, and 64 of the 256 threads had a row in the vector phases
+// (update 33 us, direction 31 us for sixteen systems of 8^3 to 48^3); with
+// 256 rows every thread has one and a workgroup sums 460 partials once.
+constexpr int kRowsPerChunk = 256;
 
 /// Device view of one system (FP64).
 struct SysDesc
@@ -36,6 +44,7 @@ struct SysDesc
   double* p;
   double* q;
   double* dinv;
+  double2* zp; // per row (z, previous p): what the next SpMV gathers
   const std::int32_t* diag; // CSR position of each row's diagonal (-1: none)
   std::int32_t nrows;
   std::int32_t chunk0; // first chunk of the system
@@ -43,15 +52,21 @@ struct SysDesc
   std::int32_t pad;
 };
 
-/// Per-system CG scalars. iter is read by the phase kernels and advanced
-/// from iter_next by the first chunk of the next SpMV (never in a kernel
-/// that reads it).
+/// Per-system CG scalars. The SpMV phase of iteration k reads k from
+/// iter_next and writes iter, the update phase reads iter and writes
+/// iter_next, so no kernel writes what another of its workgroups reads
+/// (done excepted: it is only ever set by the workgroup whose decision the
+/// others reach from the same sums).
 struct SysState
 {
   double rz[2];
   double rr0, rr, tol2;
   std::int32_t iter, iter_next, done, max_it;
-  std::int32_t active, converged, pad0, pad1;
+  std::int32_t active, converged;
+  // iteration whose stop test and rz are in the state already (set at the
+  // start and after the last iteration of a step: the partials move when
+  // systems join or leave between steps)
+  std::int32_t tested, pad;
 };
 
 struct ChunkDesc
@@ -59,20 +74,67 @@ struct ChunkDesc
   std::int32_t sys, row0, row1, first; // first: chunk is the system's first
 };
 
-__device__ inline double sum_range(const double* partials, int c0, int n)
+/// Sums of the system's NV partial arrays (c0 .. c0 + n of each), by the
+/// whole block in a fixed order; the results are returned to every thread.
+template <int NV>
+__device__ inline void sum_ranges(const double* const (&partials)[NV], int c0, int n,
+                                  double (&out)[NV])
 {
-  __shared__ double lds[4];
-  __shared__ double total;
-  double a = 0;
-  for (int i = threadIdx.x; i < n; i += kBlock)
-    a += partials[c0 + i];
-  const double s = block_sum_256(a, lds);
-  if (threadIdx.x == 0)
-    total = s;
+  __shared__ double lds[NV][kBlock / 64];
+#pragma unroll
+  for (int k = 0; k < NV; ++k)
+  {
+    double a = 0;
+    for (int i = threadIdx.x; i < n; i += kBlock)
+      a += partials[k][c0 + i];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1)
+      a += __shfl_down(a, off, 64);
+    if ((threadIdx.x & 63) == 0)
+      lds[k][threadIdx.x >> 6] = a;
+  }
   __syncthreads();
-  const double t = total;
+#pragma unroll
+  for (int k = 0; k < NV; ++k)
+    out[k] = (lds[k][0] + lds[k][1]) + (lds[k][2] + lds[k][3]);
   __syncthreads();
-  return t;
+}
+
+/// Block sums of NV values, stored at partials[k][slot].
+template <int NV>
+__device__ inline void store_block_sums(const double (&v)[NV], double* const (&partials)[NV],
+                                        int slot)
+{
+  __shared__ double lds[NV][kBlock / 64];
+#pragma unroll
+  for (int k = 0; k < NV; ++k)
+  {
+    double a = v[k];
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1)
+      a += __shfl_down(a, off, 64);
+    if ((threadIdx.x & 63) == 0)
+      lds[k][threadIdx.x >> 6] = a;
+  }
+  __syncthreads();
+  if (threadIdx.x < NV)
+  {
+    const int k = threadIdx.x;
+    partials[k][slot] = (lds[k][0] + lds[k][1]) + (lds[k][2] + lds[k][3]);
+  }
+  __syncthreads();
+}
+
+/// Chunks of one workgroup: a contiguous range, and contiguous over the
+/// workgroups of an XCD, so that a system's partials are summed once per
+/// workgroup (not once per chunk) and both phases find their rows in the
+/// same L2.
+__device__ inline int2 chunk_range(int nch)
+{
+  const int nb = gridDim.x;
+  const int l = xcd_contiguous(blockIdx.x, nb);
+  return {static_cast<int>(static_cast<long long>(nch) * l / nb),
+          static_cast<int>(static_cast<long long>(nch) * (l + 1) / nb)};
 }
 
 /// Whether a system takes no part in this phase, read once per block so that
@@ -91,160 +153,270 @@ __device__ inline bool block_skip(const SysState& S)
   return r;
 }
 
-/// Block sum of one value, stored by thread 0 at partials[slot].
-__device__ inline void store_block_sum(double v, double* partials, int slot)
+/// Stop test of a system before iteration k (k >= 1) from the reductions of
+/// the iterations so far.
+__device__ inline bool stop_test(const SysState& S, int k, double rr, bool& conv)
 {
-  __shared__ double lds[4];
-  const double s = block_sum_256(v, lds);
-  if (threadIdx.x == 0)
-    partials[slot] = s;
+  conv = rr / S.rr0 < S.tol2;
+  return conv || k >= S.max_it;
 }
 
+/// First phase of iteration k: stop test and beta from the last update's
+/// sums, p = z + beta p formed where it is gathered (each row's z and
+/// previous p are one 16-byte load), q = A p and the partial sums of p . q.
+/// Two kernels per iteration instead of three (SpMV, update, direction): the
+/// bytes are the same (the direction kernel's reads of r, dinv and p became
+/// the pair), a launch and a pass of latency are gone. Four lanes per row,
+/// the first 4 x kSteps entries of two rows per thread loaded before their
+/// gathers. Sixteen systems of 8^3 to 48^3 (618,000 rows, 8.8 M entries,
+/// 106 MB of matrix: it stays in the on-package cache): 41 us per iteration
+/// (31 here, 10 in the update) against 99.5 us of the three kernels; the
+/// whole wave of requests 14.8 ms against 27.0 ms.
 __global__ void __launch_bounds__(kBlock)
     bcg_spmv_k(const int* nchunk, const ChunkDesc* chunks, const SysDesc* sys, SysState* st,
-               double* p_pq)
+               double* p_pq, const double* p_rz, const double* p_rr)
 {
-  const int nch = *nchunk;
-  for (int t = blockIdx.x; t < nch; t += gridDim.x)
+  const int2 range = chunk_range(*nchunk);
+  int cur = -1;
+  bool skip = false;
+  double beta = 0;
+  for (int t = range.x; t < range.y; ++t)
   {
     const ChunkDesc ch = chunks[t];
-    SysState& S = st[ch.sys];
-    if (ch.first && threadIdx.x == 0)
-      S.iter = S.iter_next;
-    if (block_skip(S))
-      continue;
     const SysDesc& D = sys[ch.sys];
-    const std::int32_t row = ch.row0 + threadIdx.x / kLanes;
+    if (ch.sys != cur)
+    {
+      cur = ch.sys;
+      SysState& S = st[cur];
+      skip = block_skip(S);
+      if (!skip)
+      {
+        const int k = S.iter_next;
+        if (S.tested == k)
+          beta = k > 0 ? S.rz[k & 1] / S.rz[(k - 1) & 1] : 0.0;
+        else
+        {
+          double sums[2];
+          sum_ranges<2>({p_rz, p_rr}, D.chunk0, D.nchunks, sums);
+          bool conv;
+          skip = stop_test(S, k, sums[1], conv);
+          beta = sums[0] / S.rz[(k - 1) & 1];
+          if (ch.first && threadIdx.x == 0)
+          {
+            S.rz[k & 1] = sums[0];
+            S.rr = sums[1];
+            if (skip)
+            {
+              S.converged = conv ? 1 : 0;
+              __hip_atomic_store(&S.done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            }
+          }
+        }
+        if (ch.first && threadIdx.x == 0)
+          S.iter = k;
+      }
+    }
+    if (skip)
+      continue;
     const int lane = threadIdx.x % kLanes;
-    double s = 0;
-    if (row < ch.row1)
-    {
-      const std::int32_t e = D.rp[row + 1];
-      for (std::int32_t j = D.rp[row] + lane; j < e; j += kLanes)
-        s += D.v[j] * D.p[D.ci[j]];
-    }
-#pragma unroll
-    for (int off = kLanes / 2; off > 0; off >>= 1)
-      s += __shfl_down(s, off, kLanes);
+    const std::int32_t* __restrict__ ci = D.ci;
+    const double* __restrict__ v = D.v;
+    const double2* __restrict__ zp = D.zp;
     double d = 0;
-    if (lane == 0 && row < ch.row1)
+#pragma unroll
+    for (int half = 0; half < kRowsPerChunk / kRowsPerPass; half += 2)
     {
-      D.q[row] = s;
-      d = s * D.p[row];
+      std::int32_t row[2], e[2], c[2][kSteps];
+      std::int32_t j[2];
+      double a[2][kSteps];
+      double2 own[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+      {
+        row[h] = ch.row0 + (half + h) * kRowsPerPass + threadIdx.x / kLanes;
+        const std::int32_t rr = min(row[h], ch.row1 - 1);
+        j[h] = D.rp[rr] + lane;
+        e[h] = D.rp[rr + 1];
+        own[h] = zp[rr];
+      }
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int i = 0; i < kSteps; ++i)
+        {
+          // past the row's end: its last entry again, added as zero
+          const std::int32_t jj = max(min(j[h] + i * kLanes, e[h] - 1), 0);
+          c[h][i] = ci[jj];
+          a[h][i] = v[jj];
+        }
+      double s[2] = {0, 0};
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int i = 0; i < kSteps; ++i)
+        {
+          const double2 g = zp[c[h][i]];
+          if (j[h] + i * kLanes < e[h])
+            s[h] += a[h][i] * __builtin_fma(beta, g.y, g.x);
+        }
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+      {
+        for (std::int32_t q = j[h] + kSteps * kLanes; q < e[h]; q += kLanes)
+        {
+          const double2 g = zp[ci[q]];
+          s[h] += v[q] * __builtin_fma(beta, g.y, g.x);
+        }
+#pragma unroll
+        for (int off = kLanes / 2; off > 0; off >>= 1)
+          s[h] += __shfl_down(s[h], off, kLanes);
+        if (lane == 0 && row[h] < ch.row1)
+        {
+          const double p = __builtin_fma(beta, own[h].y, own[h].x);
+          D.p[row[h]] = p;
+          D.q[row[h]] = s[h];
+          d += s[h] * p;
+        }
+      }
     }
-    store_block_sum(d, p_pq, t);
+    store_block_sums<1>({d}, {p_pq}, t);
   }
 }
 
+/// Second phase: x += alpha p, r -= alpha q, the pairs (dinv r, p) that the
+/// next SpMV gathers, and the partial sums of r . z and r . r.
 __global__ void __launch_bounds__(kBlock)
-    bcg_update_k(const int* nchunk, const ChunkDesc* chunks, const SysDesc* sys,
-                 const SysState* st, const double* p_pq, double* p_rz, double* p_rr)
+    bcg_update_k(const int* nchunk, const ChunkDesc* chunks, const SysDesc* sys, SysState* st,
+                 const double* p_pq, double* p_rz, double* p_rr)
 {
-  const int nch = *nchunk;
-  for (int t = blockIdx.x; t < nch; t += gridDim.x)
+  const int2 range = chunk_range(*nchunk);
+  int cur = -1;
+  bool skip = false;
+  double alpha = 0;
+  for (int t = range.x; t < range.y; ++t)
   {
     const ChunkDesc ch = chunks[t];
-    const SysState& S = st[ch.sys];
-    if (block_skip(S))
-      continue;
     const SysDesc& D = sys[ch.sys];
-    const double pq = sum_range(p_pq, D.chunk0, D.nchunks);
-    const double alpha = S.rz[S.iter & 1] / pq;
-    double srz = 0, srr = 0;
-    for (std::int32_t i = ch.row0 + threadIdx.x; i < ch.row1; i += kBlock)
+    if (ch.sys != cur)
     {
-      D.x[i] += alpha * D.p[i];
+      cur = ch.sys;
+      SysState& S = st[cur];
+      skip = block_skip(S);
+      if (!skip)
+      {
+        double pq[1];
+        sum_ranges<1>({p_pq}, D.chunk0, D.nchunks, pq);
+        const int k = S.iter;
+        alpha = S.rz[k & 1] / pq[0];
+        if (ch.first && threadIdx.x == 0)
+          S.iter_next = k + 1;
+      }
+    }
+    if (skip)
+      continue;
+    double sums[2] = {0, 0};
+    const std::int32_t i = ch.row0 + threadIdx.x;
+    if (i < ch.row1)
+    {
+      const double p = D.p[i], di = D.dinv[i];
+      D.x[i] += alpha * p;
       const double ri = D.r[i] - alpha * D.q[i];
       D.r[i] = ri;
-      srz += ri * D.dinv[i] * ri;
-      srr += ri * ri;
+      const double z = di * ri;
+      D.zp[i] = make_double2(z, p);
+      sums[0] = z * ri;
+      sums[1] = ri * ri;
     }
-    store_block_sum(srz, p_rz, t);
-    store_block_sum(srr, p_rr, t);
+    store_block_sums<2>(sums, {p_rz, p_rr}, t);
   }
 }
 
+/// After the last iteration of a step: the stop test and r . z that the next
+/// SpMV would take from the partials, so that the status read then is that of
+/// every iteration done and the partials are free to move.
 __global__ void __launch_bounds__(kBlock)
-    bcg_direction_k(const int* nchunk, const ChunkDesc* chunks, const SysDesc* sys,
-                    SysState* st, const double* p_rz, const double* p_rr)
+    bcg_finish_k(int nsys, const SysDesc* sys, SysState* st, const double* p_rz,
+                 const double* p_rr)
 {
-  const int nch = *nchunk;
-  for (int t = blockIdx.x; t < nch; t += gridDim.x)
+  for (int s = blockIdx.x; s < nsys; s += gridDim.x)
   {
-    const ChunkDesc ch = chunks[t];
-    SysState& S = st[ch.sys];
-    if (block_skip(S))
+    SysState& S = st[s];
+    if (block_skip(S) || S.tested == S.iter_next)
       continue;
-    const SysDesc& D = sys[ch.sys];
-    const double rz = sum_range(p_rz, D.chunk0, D.nchunks);
-    const double rr = sum_range(p_rr, D.chunk0, D.nchunks);
-    const int k = S.iter;
-    const bool conv = rr / S.rr0 < S.tol2;
-    const bool stop = conv || k + 1 >= S.max_it;
-    const double beta = rz / S.rz[k & 1];
-    __syncthreads(); // every thread has read the scalars before the writes
-    if (ch.first && threadIdx.x == 0)
+    const SysDesc& D = sys[s];
+    double sums[2];
+    sum_ranges<2>({p_rz, p_rr}, D.chunk0, D.nchunks, sums); // ends with a barrier
+    if (threadIdx.x == 0)
     {
-      S.rz[(k + 1) & 1] = rz;
-      S.rr = rr;
-      S.iter_next = k + 1;
-      if (stop)
+      bool conv;
+      const int k = S.iter_next;
+      S.rz[k & 1] = sums[0];
+      S.rr = sums[1];
+      S.tested = k;
+      if (stop_test(S, k, sums[1], conv))
       {
         S.converged = conv ? 1 : 0;
         S.done = 1;
       }
     }
-    if (stop)
-      continue;
-    for (std::int32_t i = ch.row0 + threadIdx.x; i < ch.row1; i += kBlock)
-      D.p[i] = D.dinv[i] * D.r[i] + beta * D.p[i];
+    __syncthreads();
   }
 }
 
-/// Start of a system's solve from x = 0: r = b, p = z = dinv b, partial
-/// sums of (r.z, r.r); dinv from the CSR diagonal.
+/// First residual of one row: r = b, z = dinv b, x = 0 (dinv from the CSR
+/// diagonal); adds its r . z and r . r to sums.
+__device__ inline void start_row(const SysDesc& D, const std::int32_t* diag, std::int32_t i,
+                                 double (&sums)[2])
+{
+  const std::int32_t pd = diag[i];
+  const double a = pd >= 0 ? D.v[pd] : 0.0;
+  const double di = a != 0.0 ? 1.0 / a : 1.0;
+  const double bi = D.b[i];
+  D.dinv[i] = di;
+  D.x[i] = 0.0;
+  D.r[i] = bi;
+  const double z = di * bi;
+  D.zp[i] = make_double2(z, 0.0);
+  sums[0] += z * bi;
+  sums[1] += bi * bi;
+}
+
+/// Start of a system's solve from x = 0: start_row and the partial sums.
 __global__ void __launch_bounds__(kBlock)
     bcg_start_k(SysDesc D, const std::int32_t* diag, int c0, double* p_rz, double* p_rr)
 {
-  const std::int32_t row0 = blockIdx.x * kRowsPerChunk;
-  const std::int32_t row1 = min(row0 + kRowsPerChunk, D.nrows);
-  double srz = 0, srr = 0;
-  for (std::int32_t i = row0 + threadIdx.x; i < row1; i += kBlock)
-  {
-    const std::int32_t pd = diag[i];
-    const double a = pd >= 0 ? D.v[pd] : 0.0;
-    const double di = a != 0.0 ? 1.0 / a : 1.0;
-    D.dinv[i] = di;
-    const double bi = D.b[i];
-    D.x[i] = 0.0;
-    D.r[i] = bi;
-    D.p[i] = di * bi;
-    srz += bi * di * bi;
-    srr += bi * bi;
-  }
-  store_block_sum(srz, p_rz, c0 + blockIdx.x);
-  store_block_sum(srr, p_rr, c0 + blockIdx.x);
+  const std::int32_t i = blockIdx.x * kRowsPerChunk + threadIdx.x;
+  double sums[2] = {0, 0};
+  if (i < D.nrows)
+    start_row(D, diag, i, sums);
+  store_block_sums<2>(sums, {p_rz, p_rr}, c0 + blockIdx.x);
+}
+
+__device__ inline void start_state(SysState& S, const double (&sums)[2])
+{
+  S.rz[0] = sums[0];
+  S.rz[1] = 0;
+  S.rr0 = sums[1];
+  S.rr = sums[1];
+  S.iter = 0;
+  S.iter_next = 0;
+  S.tested = 0;
+  S.converged = sums[1] == 0.0 ? 1 : 0;
+  S.done = (sums[1] == 0.0 || S.max_it <= 0) ? 1 : 0;
 }
 
 __global__ void __launch_bounds__(kBlock)
     bcg_start_finish_k(const double* p_rz, const double* p_rr, int c0, int n, SysState* S,
                        double tol2, int max_it)
 {
-  const double rz = sum_range(p_rz, c0, n);
-  const double rr = sum_range(p_rr, c0, n);
+  double sums[2];
+  sum_ranges<2>({p_rz, p_rr}, c0, n, sums);
   if (threadIdx.x == 0)
   {
-    S->rz[0] = rz;
-    S->rz[1] = 0;
-    S->rr0 = rr;
-    S->rr = rr;
     S->tol2 = tol2;
-    S->iter = 0;
-    S->iter_next = 0;
     S->max_it = max_it;
     S->active = 1;
-    S->converged = rr == 0.0 ? 1 : 0;
-    S->done = (rr == 0.0 || max_it <= 0) ? 1 : 0;
+    start_state(*S, sums);
   }
 }
 
@@ -254,29 +426,18 @@ __global__ void __launch_bounds__(kBlock)
     bcg_restart_k(const int* nchunk, const ChunkDesc* chunks, const SysDesc* sys,
                   const SysState* st, double* p_rz, double* p_rr)
 {
-  const int nch = *nchunk;
-  for (int t = blockIdx.x; t < nch; t += gridDim.x)
+  const int2 range = chunk_range(*nchunk);
+  for (int t = range.x; t < range.y; ++t)
   {
     const ChunkDesc ch = chunks[t];
     if (st[ch.sys].active == 0)
       continue;
     const SysDesc& D = sys[ch.sys];
-    double srz = 0, srr = 0;
-    for (std::int32_t i = ch.row0 + threadIdx.x; i < ch.row1; i += kBlock)
-    {
-      const std::int32_t pd = D.diag[i];
-      const double a = pd >= 0 ? D.v[pd] : 0.0;
-      const double di = a != 0.0 ? 1.0 / a : 1.0;
-      D.dinv[i] = di;
-      const double bi = D.b[i];
-      D.x[i] = 0.0;
-      D.r[i] = bi;
-      D.p[i] = di * bi;
-      srz += bi * di * bi;
-      srr += bi * bi;
-    }
-    store_block_sum(srz, p_rz, t);
-    store_block_sum(srr, p_rr, t);
+    double sums[2] = {0, 0};
+    const std::int32_t i = ch.row0 + threadIdx.x;
+    if (i < ch.row1)
+      start_row(D, D.diag, i, sums);
+    store_block_sums<2>(sums, {p_rz, p_rr}, t);
   }
 }
 
@@ -292,19 +453,10 @@ __global__ void __launch_bounds__(kBlock)
     if (S.active == 0)
       continue;
     const SysDesc& D = sys[s];
-    const double rz = sum_range(p_rz, D.chunk0, D.nchunks);
-    const double rr = sum_range(p_rr, D.chunk0, D.nchunks);
+    double sums[2];
+    sum_ranges<2>({p_rz, p_rr}, D.chunk0, D.nchunks, sums);
     if (threadIdx.x == 0)
-    {
-      S.rz[0] = rz;
-      S.rz[1] = 0;
-      S.rr0 = rr;
-      S.rr = rr;
-      S.iter = 0;
-      S.iter_next = 0;
-      S.converged = rr == 0.0 ? 1 : 0;
-      S.done = (rr == 0.0 || S.max_it <= 0) ? 1 : 0;
-    }
+      start_state(S, sums);
     __syncthreads();
   }
 }
@@ -332,13 +484,13 @@ struct dfx_batch
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   int graph_iters = 0;
-  // work vectors (r, p, q, diag^-1) of systems that left, kept by row count
+  // work vectors (r, p, q, diag^-1, (z, p) pairs) of systems that left, kept by row count
   // for the next system of that size (no device allocation or free, and so
   // no device-wide synchronisation, while serving)
   struct Work
   {
     std::int64_t n;
-    double* v[4];
+    double* v[5];
   };
   std::vector<Work> pool;
 };
@@ -374,7 +526,7 @@ void batch_rebuild_chunks(dfx_batch& B)
 /// stays valid) striding over the live chunks.
 int phase_grid(const dfx_batch& B)
 {
-  return std::max(1, std::min(B.max_chunks, ctx().num_cu * 4));
+  return std::max(1, std::min(B.max_chunks, ctx().num_cu * 8));
 }
 
 void launch_iterations(dfx_batch& B, int iters)
@@ -383,10 +535,11 @@ void launch_iterations(dfx_batch& B, int iters)
   const int g = phase_grid(B);
   for (int i = 0; i < iters; ++i)
   {
-    bcg_spmv_k<<<g, kBlock, 0, s>>>(B.nchunk, B.chunks, B.sys, B.st, B.p_pq);
+    bcg_spmv_k<<<g, kBlock, 0, s>>>(B.nchunk, B.chunks, B.sys, B.st, B.p_pq, B.p_rz, B.p_rr);
     bcg_update_k<<<g, kBlock, 0, s>>>(B.nchunk, B.chunks, B.sys, B.st, B.p_pq, B.p_rz, B.p_rr);
-    bcg_direction_k<<<g, kBlock, 0, s>>>(B.nchunk, B.chunks, B.sys, B.st, B.p_rz, B.p_rr);
   }
+  bcg_finish_k<<<std::min(B.max_sys, 1024), kBlock, 0, s>>>(B.max_sys, B.sys, B.st, B.p_rz,
+                                                           B.p_rr);
 }
 
 } // namespace
@@ -433,6 +586,7 @@ dfx_status dfx_batch_destroy(dfx_batch* B)
         dfree(B->hsys[s].p);
         dfree(B->hsys[s].q);
         dfree(B->hsys[s].dinv);
+        dfree(B->hsys[s].zp);
       }
     for (auto& w : B->pool)
       for (double* v : w.v)
@@ -486,6 +640,7 @@ dfx_status dfx_batch_add(dfx_batch* B, const dfx_csr* A, const dfx_vec* b, dfx_v
           d.p = it->v[1];
           d.q = it->v[2];
           d.dinv = it->v[3];
+          d.zp = reinterpret_cast<double2*>(it->v[4]);
           B->pool.erase(it);
         }
         else
@@ -494,6 +649,13 @@ dfx_status dfx_batch_add(dfx_batch* B, const dfx_csr* A, const dfx_vec* b, dfx_v
           d.p = static_cast<double*>(dmalloc(sizeof(double) * n));
           d.q = static_cast<double*>(dmalloc(sizeof(double) * n));
           d.dinv = static_cast<double*>(dmalloc(sizeof(double) * n));
+          d.zp = static_cast<double2*>(dmalloc(sizeof(double2) * n));
+        }
+        if (A->nnz == 0)
+        {
+          // the SpMV loads (and drops) entry 0 for an empty row: give it one
+          d.ci = A->row_ptr;
+          d.v = d.dinv;
         }
         B->hsys[s] = d;
         B->slot_used[s] = 1;
@@ -508,6 +670,7 @@ dfx_status dfx_batch_add(dfx_batch* B, const dfx_csr* A, const dfx_vec* b, dfx_v
           dfree(d.p);
           dfree(d.q);
           dfree(d.dinv);
+          dfree(d.zp);
           throw;
         }
         const SysDesc& dd = B->hsys[s];
@@ -530,7 +693,7 @@ dfx_status dfx_batch_remove(dfx_batch* B, int32_t slot)
         SysDesc& d = B->hsys[slot];
         // queued work of this system precedes any later use of its vectors
         // in stream order, so they go back to the pool at once
-        B->pool.push_back({std::max<std::int64_t>(d.nrows, 1), {d.r, d.p, d.q, d.dinv}});
+        B->pool.push_back({std::max<std::int64_t>(d.nrows, 1), {d.r, d.p, d.q, d.dinv, reinterpret_cast<double*>(d.zp)}});
         d = SysDesc{};
         B->slot_used[slot] = 0;
         SysState zero{};

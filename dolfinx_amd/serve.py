@@ -118,8 +118,8 @@ class MeshTemplate:
 
     def footprint(self) -> int:
         """HBM bytes a resident request needs: matrix values, b, x and the
-        CG work vectors r, p, q, diag^-1."""
-        return 8 * self.nnz + 6 * 8 * self.N
+        CG work vectors r, p, q, diag^-1 and the (z, p) pairs."""
+        return 8 * self.nnz + 8 * 8 * self.N
 
     def matrix(self) -> la.MatrixCSR:
         return la.MatrixCSR.shared(self.pattern, np.float64)
