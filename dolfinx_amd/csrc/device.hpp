@@ -191,6 +191,13 @@ struct dfx_csr
   // (row, entry) pairs.
   std::int32_t* rblk = nullptr;
   std::int32_t nblk = 0;
+  // 16-bit columns (bs = 1; nnz + 2 places). Row-lane SpMV: window and
+  // offset in the windows of the row's 64-row group (win, int4 per group);
+  // otherwise (win null) offsets from the first column of the row block
+  // (rbase per row block, -1 where they do not fit).
+  void* win = nullptr;
+  std::int32_t* rbase = nullptr;
+  std::uint16_t* cols16 = nullptr;
   // pattern arrays borrowed from another matrix (not freed by this one)
   const dfx_csr* pattern_owner = nullptr;
   // Sliced-ELL copy used inside the solvers (bs = 1), refreshed from the CSR

@@ -239,83 +239,161 @@ constexpr int stream_chunk()
   return 16384 / static_cast<int>(sizeof(T));
 }
 
+/// Entries a row block of the scalar stream SpMV may hold: its entries are
+/// loaded in aligned pairs, so the pair before an odd first entry takes one
+/// place of the chunk.
+template <typename T>
+constexpr int stream_entries()
+{
+  return stream_chunk<T>() - 1;
+}
+
+/// 16-bit columns of the stream SpMV: workgroup b finds the smallest column
+/// of row block b and, if the block's columns span less than 2^16, writes
+/// them as offsets from it (base[b]); base[b] = -1 keeps the 32-bit columns.
+__global__ void __launch_bounds__(kBlock)
+    stream_cols_k(const int2* __restrict__ rbj, const std::int32_t* __restrict__ rp,
+                  const std::int32_t* __restrict__ ci, std::int32_t* __restrict__ base,
+                  std::uint16_t* __restrict__ c16)
+{
+  __shared__ std::int32_t ends[2];
+  const int2 lo = rbj[blockIdx.x], hi = rbj[blockIdx.x + 1];
+  if (threadIdx.x == 0)
+  {
+    ends[0] = 0x7fffffff;
+    ends[1] = -1;
+  }
+  __syncthreads();
+  for (std::int32_t r = lo.x + threadIdx.x; r < hi.x; r += kBlock)
+  {
+    const std::int32_t j0 = rp[r], j1 = rp[r + 1];
+    if (j1 > j0)
+    {
+      atomicMin(&ends[0], ci[j0]); // columns are sorted in a row
+      atomicMax(&ends[1], ci[j1 - 1]);
+    }
+  }
+  __syncthreads();
+  const std::int32_t first = ends[0], last = ends[1];
+  const bool narrow = last >= first && last - first < 65536;
+  if (threadIdx.x == 0)
+    base[blockIdx.x] = narrow ? first : -1;
+  if (narrow)
+    for (std::int32_t j = lo.y + threadIdx.x; j < hi.y; j += kBlock)
+      c16[j] = static_cast<std::uint16_t>(ci[j] - first);
+}
+
+/// Two consecutive values, aligned to their size.
+template <typename T>
+using Pair = T __attribute__((ext_vector_type(2)));
+
 /// Stream CSR SpMV, y (+)= A x. Each row block (consecutive rows whose
 /// entries fit one chunk) is processed by one workgroup: the products
 /// v_j x[c_j] of the block's contiguous entry range are formed with fully
-/// coalesced loads into LDS, then one thread per row sums its products left
-/// to right, the order of the reference's row-serial loop. Row blocks are
-/// given as (first row, first entry) pairs (rbj, nblk + 1 of them), so a
+/// coalesced loads (aligned pairs of entries, 16-bit columns from the block's
+/// first column where they fit) into LDS, then 2^lg threads per row (as many
+/// as the workgroup has for the block's rows) sum its products. Row blocks
+/// are given as (first row, first entry) pairs (rbj, nblk + 1 of them), so a
 /// block's bounds are one load. While the rows of the current block are
 /// summed, the next block's entries and its rows' positions (and y, dotv)
 /// are in flight, and the bounds of the block after it: each block waits
 /// for one memory round trip (its x gather) instead of a chain of them. A
 /// block holding a single longer row is reduced with a strided sum. With
-/// dotv, partial sums of y.dotv go to partials.
+/// dotv, partial sums of y.dotv go to partials. P3 on 24^3 tetrahedra (18.4 M
+/// entries, 47 per row: 43 rows in a chunk) 36 us; with one thread per row
+/// the sums, 47 LDS reads one after the other in 43 of the 256 threads, took
+/// longer than the loads and the product 72 us.
 template <typename T>
 __global__ void __launch_bounds__(kBlock)
     spmv_stream_k(std::int32_t nblk, const int2* __restrict__ rbj,
-                  const std::int32_t* __restrict__ rp, const std::int32_t* __restrict__ ci,
-                  const T* __restrict__ v, const T* __restrict__ x, T* __restrict__ y,
-                  int accumulate, const T* __restrict__ dotv, double* partials,
-                  const int* stop)
+                  const std::int32_t* __restrict__ rbase, const std::int32_t* __restrict__ rp,
+                  const std::int32_t* __restrict__ ci, const std::uint16_t* __restrict__ c16,
+                  std::int32_t ncols, const T* __restrict__ v, const T* __restrict__ x,
+                  T* __restrict__ y, int accumulate, const T* __restrict__ dotv,
+                  double* partials, const int* stop)
 {
   if (stop && block_flag(stop))
     return;
   constexpr int NC = stream_chunk<T>();
-  constexpr int U = NC / kBlock;
-  __shared__ T prod[NC];
+  constexpr int U = NC / (2 * kBlock); // pairs per thread
+  __shared__ Pair<T> prod2[NC / 2];
   __shared__ double red[4];
+  const T* prod = reinterpret_cast<const T*>(prod2);
   double d[1] = {0.0};
   struct Bounds
   {
-    std::int32_t r0, r1, j0, j1;
+    std::int32_t r0, r1, j0, j1, base;
   };
-  // this thread's row of a block: its products [kb, ke) in the chunk, and
-  // y and dotv at the row
+  // this thread's row of a block: its products [kb, ke) in the chunk (lane
+  // of 2^lg threads), and y and dotv at the row
   struct Row
   {
-    std::int32_t kb, ke;
+    std::int32_t r, kb, ke;
+    int lg;
     T yold, dv;
   };
   auto bounds = [&](int b) -> Bounds
   {
     const int2 lo = rbj[b], hi = rbj[b + 1];
-    return {lo.x, hi.x, lo.y, hi.y};
+    return {lo.x, hi.x, lo.y, hi.y, rbase[b]};
   };
   auto row_of = [&](const Bounds& B) -> Row
   {
-    Row w{0, 0, T(0), T(0)};
-    const std::int32_t r = B.r0 + static_cast<std::int32_t>(threadIdx.x);
-    if (r < B.r1)
+    int lg = 0;
+    while (lg < 6 && (static_cast<std::uint32_t>(B.r1 - B.r0) << (lg + 1)) <= kBlock)
+      ++lg;
+    Row w{B.r0 + static_cast<std::int32_t>(threadIdx.x >> lg), 0, 0, lg, T(0), T(0)};
+    if (w.r < B.r1)
     {
-      w.kb = rp[r] - B.j0;
-      w.ke = rp[r + 1] - B.j0;
+      const std::int32_t j00 = B.j0 & ~1;
+      w.kb = rp[w.r] - j00;
+      w.ke = rp[w.r + 1] - j00;
       if (accumulate)
-        w.yold = y[r];
+        w.yold = y[w.r];
       if (dotv)
-        w.dv = dotv[r];
+        w.dv = dotv[w.r];
     }
     return w;
   };
-  T vv[U];
-  std::int32_t cc[U];
+  Pair<T> vv[U];
+  std::int32_t cc[U][2];
 #pragma unroll
   for (int u = 0; u < U; ++u)
   {
-    vv[u] = T(0);
-    cc[u] = 0;
+    vv[u] = Pair<T>(T(0));
+    cc[u][0] = cc[u][1] = 0;
   }
   // unconditional loads at clamped positions (no branch around a load, so
-  // all of them are in flight together); entries past j1 are not used
+  // all of them are in flight together); entries outside [j0, j1) are not
+  // used. The pair after the last entry may reach one place past nnz (the
+  // arrays hold it); a neighbouring block's 16-bit offset is clamped to the
+  // matrix's columns.
   auto stage = [&](const Bounds& B)
   {
-    const std::int32_t last = max(B.j1 - 1, B.j0);
-#pragma unroll
-    for (int u = 0; u < U; ++u)
+    const std::int32_t lastp = (B.j1 - 1) & ~1;
+    const std::int32_t j00 = B.j0 & ~1;
+    if (B.base >= 0)
     {
-      const std::int32_t j = min(B.j0 + static_cast<std::int32_t>(threadIdx.x) + u * kBlock, last);
-      vv[u] = v[j];
-      cc[u] = ci[j];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+      {
+        const std::int32_t j = min(j00 + 2 * static_cast<std::int32_t>(threadIdx.x + u * kBlock), lastp);
+        vv[u] = *reinterpret_cast<const Pair<T>*>(v + j);
+        const std::uint32_t c = *reinterpret_cast<const std::uint32_t*>(c16 + j);
+        cc[u][0] = min(B.base + static_cast<std::int32_t>(c & 0xffffu), ncols - 1);
+        cc[u][1] = min(B.base + static_cast<std::int32_t>(c >> 16), ncols - 1);
+      }
+    }
+    else
+    {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+      {
+        const std::int32_t j = min(j00 + 2 * static_cast<std::int32_t>(threadIdx.x + u * kBlock), lastp);
+        vv[u] = *reinterpret_cast<const Pair<T>*>(v + j);
+        cc[u][0] = ci[j];
+        cc[u][1] = ci[min(j + 1, B.j1 - 1)];
+      }
     }
   };
   const XcdRange xr = xcd_range(nblk);
@@ -323,53 +401,63 @@ __global__ void __launch_bounds__(kBlock)
   if (bi < xr.end)
   {
     Bounds cur = bounds(bi);
-    const bool cur_short = cur.j1 - cur.j0 <= NC;
-    if (cur_short && cur.j1 > cur.j0)
+    auto is_short = [](const Bounds& B) { return B.j1 - B.j0 <= stream_entries<T>(); };
+    if (is_short(cur) && cur.j1 > cur.j0)
       stage(cur);
     Row row = row_of(cur);
     int nbi = bi + xr.step;
-    Bounds nxt = nbi < xr.end ? bounds(nbi) : Bounds{0, 0, 0, 0};
+    Bounds nxt = nbi < xr.end ? bounds(nbi) : Bounds{0, 0, 0, 0, 0};
     for (;;)
     {
       const bool more = nbi < xr.end;
       const int nnbi = nbi + xr.step;
-      Row nrow{0, 0, T(0), T(0)};
-      Bounds nnxt{0, 0, 0, 0};
-      if (cur.j1 - cur.j0 <= NC)
+      Row nrow{0, 0, 0, 0, T(0), T(0)};
+      Bounds nnxt{0, 0, 0, 0, 0};
+      if (is_short(cur))
       {
         if (cur.j1 > cur.j0)
         {
-          T xv[U];
-#pragma unroll
-          for (int u = 0; u < U; ++u)
-            xv[u] = x[cc[u]];
+          T xv[U][2];
 #pragma unroll
           for (int u = 0; u < U; ++u)
           {
-            const std::int32_t j = cur.j0 + threadIdx.x + u * kBlock;
-            if (j < cur.j1)
-              prod[j - cur.j0] = vv[u] * xv[u];
+            xv[u][0] = x[cc[u][0]];
+            xv[u][1] = x[cc[u][1]];
           }
+#pragma unroll
+          for (int u = 0; u < U; ++u)
+            prod2[threadIdx.x + u * kBlock] = Pair<T>{vv[u].x * xv[u][0], vv[u].y * xv[u][1]};
         }
         lds_barrier();
-        // the next block's loads go out before the sums (a row block has
-        // at most kBlock rows: one row per thread)
+        // the next block's loads go out before the sums
         if (more)
         {
-          if (nxt.j1 - nxt.j0 <= NC && nxt.j1 > nxt.j0)
+          if (is_short(nxt) && nxt.j1 > nxt.j0)
             stage(nxt);
           nrow = row_of(nxt);
           if (nnbi < xr.end)
             nnxt = bounds(nnbi);
         }
-        const std::int32_t r = cur.r0 + threadIdx.x;
-        if (r < cur.r1)
+        T sum = 0;
+        const int step = 1 << row.lg, lane = threadIdx.x & (step - 1);
+        std::int32_t k = row.kb + lane;
+        for (; k + 3 * step < row.ke; k += 4 * step)
         {
-          T sum = 0;
-          for (std::int32_t k = row.kb; k < row.ke; ++k)
-            sum += prod[k];
+          const T p0 = prod[k], p1 = prod[k + step], p2 = prod[k + 2 * step],
+                  p3 = prod[k + 3 * step];
+          sum += p0;
+          sum += p1;
+          sum += p2;
+          sum += p3;
+        }
+        for (; k < row.ke; k += step)
+          sum += prod[k];
+        for (int off = step >> 1; off > 0; off >>= 1)
+          sum += __shfl_xor(sum, off, 64);
+        if (lane == 0 && row.r < cur.r1)
+        {
           const T yr = accumulate ? row.yold + sum : sum;
-          y[r] = yr;
+          y[row.r] = yr;
           if (dotv)
             d[0] += double(yr) * double(row.dv);
         }
@@ -390,7 +478,7 @@ __global__ void __launch_bounds__(kBlock)
         }
         if (more)
         {
-          if (nxt.j1 - nxt.j0 <= NC && nxt.j1 > nxt.j0)
+          if (is_short(nxt) && nxt.j1 > nxt.j0)
             stage(nxt);
           nrow = row_of(nxt);
           if (nnbi < xr.end)
@@ -407,6 +495,191 @@ __global__ void __launch_bounds__(kBlock)
   }
   if (partials)
     block_partials<1>(d, partials);
+}
+
+/// Rows of a wavefront in the row-lane SpMV, and its longest row.
+constexpr int kRowGroup = 64;
+constexpr int kRowLaneMax = 32;
+/// Rows from which a matrix of short rows is served by the row-lane SpMV. It
+/// needs many groups per resident wavefront (8 per CU at FP64): measured
+/// against the stream SpMV, FP64 27-entry rows 146 against 179 us at 2.1 M
+/// rows, but 33.9 against 30.7 us at 523,000 and 24.5 against 19.8 us at
+/// 300,000 (the matrix is then in the on-package cache and the gathers hide
+/// behind five times as many wavefronts); FP64 15-entry rows 14.8 against
+/// 16.5 us at 358,000; FP32 27-entry rows 96 against 146 us at 2.1 M and 16.0
+/// against 17.7 us at 275,000.
+inline std::int32_t row_lane_min_rows(int dtype, std::int32_t max_row)
+{
+  return dtype == DFX_F64 && max_row > 16 ? 1 << 20 : 1 << 18;
+}
+
+/// 16-bit columns of the row-lane SpMV: the wavefront of 64-row group g
+/// covers the group's columns by up to four windows of 2^14 columns, each
+/// from the first column that the windows before it leave out (win[g]), and
+/// writes every column as its window and its offset in it. The rows of an RCM
+/// ordering couple a few narrow bands (the breadth-first levels) far apart:
+/// of the 64-row groups of the 128^3 hexahedral matrix 43 % span more than
+/// 2^16 columns, and all are covered by the windows. *wide is set when a
+/// group needs more.
+__global__ void __launch_bounds__(kBlock)
+    row_windows_k(std::int32_t nrows, std::int32_t ngroups, const std::int32_t* __restrict__ rp,
+                  const std::int32_t* __restrict__ ci, int4* __restrict__ win,
+                  std::uint16_t* __restrict__ c16, int* wide)
+{
+  const std::int32_t g = blockIdx.x * (kBlock / kRowGroup) + threadIdx.x / kRowGroup;
+  if (g >= ngroups)
+    return;
+  const int lane = threadIdx.x % kRowGroup;
+  const std::int32_t j0 = rp[g * kRowGroup], j1 = rp[min((g + 1) * kRowGroup, nrows)];
+  std::int32_t base[4], from = 0;
+#pragma unroll
+  for (int w = 0; w < 4; ++w)
+  {
+    std::int32_t lo = 0x7fffffff;
+    for (std::int32_t j = j0 + lane; j < j1; j += kRowGroup)
+    {
+      const std::int32_t c = ci[j];
+      if (c >= from)
+        lo = min(lo, c);
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1)
+      lo = min(lo, __shfl_xor(lo, o, 64));
+    base[w] = lo;
+    from = lo < 0x7fffffff - 16384 ? lo + 16384 : 0x7fffffff;
+  }
+  bool out = false;
+  for (std::int32_t j = j0 + lane; j < j1; j += kRowGroup)
+  {
+    const std::int32_t c = ci[j];
+    const int w = (c >= base[1]) + (c >= base[2]) + (c >= base[3]);
+    const std::int32_t o = c - (w & 2 ? (w & 1 ? base[3] : base[2]) : (w & 1 ? base[1] : base[0]));
+    out |= o >= 16384;
+    c16[j] = static_cast<std::uint16_t>(w << 14 | (o & 16383));
+  }
+  if (out)
+    *wide = 1;
+  if (lane == 0)
+    win[g] = make_int4(base[0], base[1], base[2], base[3]);
+}
+
+/// Row-lane SpMV for matrices of short rows (at most NI entries), y (+)= A x.
+/// A wavefront takes 64 consecutive rows: their entries are loaded in aligned
+/// pairs with coalesced loads, turned over in LDS, and lane l then walks row
+/// l. Neighbouring rows have neighbouring columns, so the x gathers of one
+/// step touch few cache lines; in entry order (spmv_stream_k) nearly every
+/// lane of a gather has a line of its own, and a CU serves about one line per
+/// cycle. The wavefronts are independent (no workgroup barrier); the gathers
+/// of a group are issued before the loads of the next one, and waited for
+/// behind them. 128^3 hexahedra (57 M entries) FP64 146 us = 4.4 TB/s of its
+/// 640 MB (176 us with the stream kernel and 32-bit columns), FP32 96 us
+/// (133 us).
+template <typename T, int NI>
+__global__ void __launch_bounds__(2 * kRowGroup)
+    spmv_rows_k(std::int32_t nrows, std::int32_t ngroups, const int4* __restrict__ win,
+                const std::int32_t* __restrict__ rp, const std::uint16_t* __restrict__ c16,
+                std::int32_t ncols, const T* __restrict__ v, const T* __restrict__ x,
+                T* __restrict__ y, int accumulate, const T* __restrict__ dotv, double* partials,
+                const int* stop)
+{
+  constexpr int NP = (kRowGroup * NI + 1 + 2 * kRowGroup - 1) / (2 * kRowGroup); // pairs per lane
+  __shared__ Pair<T> sval[2][NP * kRowGroup];
+  __shared__ std::uint32_t scol[2][NP * kRowGroup];
+  __shared__ double red[2];
+  const int wave = threadIdx.x / kRowGroup, lane = threadIdx.x % kRowGroup;
+  const T* val = reinterpret_cast<const T*>(sval[wave]);
+  const std::uint16_t* col = reinterpret_cast<const std::uint16_t*>(scol[wave]);
+  double d = 0.0;
+  const int stopped
+      = stop ? __hip_atomic_load(stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+  if (stopped)
+    return; // set by an earlier kernel: the same for every wavefront
+  Pair<T> vv[NP];
+  std::uint32_t cc[NP];
+  std::int32_t kb = 0, len = 0;
+  int4 w{0, 0, 0, 0};
+  T yold = T(0), dv = T(0);
+  // clamped positions: no load behind a branch; the pair after the last entry
+  // may reach one place past nnz (the arrays hold it)
+  auto stage = [&](std::int32_t g)
+  {
+    const std::int32_t r0 = g * kRowGroup, r1 = min(r0 + kRowGroup, nrows);
+    const std::int32_t j0 = rp[r0], j1 = rp[r1];
+    const std::int32_t j00 = j0 & ~1, lastp = max(j1 - 1, j0) & ~1;
+#pragma unroll
+    for (int u = 0; u < NP; ++u)
+    {
+      const std::int32_t j = min(j00 + 2 * (lane + u * kRowGroup), lastp);
+      vv[u] = *reinterpret_cast<const Pair<T>*>(v + j);
+      cc[u] = *reinterpret_cast<const std::uint32_t*>(c16 + j);
+    }
+    const std::int32_t r = min(r0 + lane, r1 - 1);
+    kb = rp[r] - j00;
+    len = rp[r + 1] - j00 - kb;
+    w = win[g];
+    if (accumulate)
+      yold = y[r];
+    if (dotv)
+      dv = dotv[r];
+  };
+  const std::int32_t npair = (ngroups + 1) / 2;
+  const XcdRange xr = xcd_range(npair);
+  std::int32_t it = xr.first;
+  if (it < xr.end && 2 * it + wave < ngroups)
+    stage(2 * it + wave);
+  for (; it < xr.end; it += xr.step)
+  {
+    const std::int32_t g = 2 * it + wave;
+    if (g >= ngroups)
+      break; // the last pair's second half
+#pragma unroll
+    for (int u = 0; u < NP; ++u)
+    {
+      sval[wave][lane + u * kRowGroup] = vv[u];
+      scol[wave][lane + u * kRowGroup] = cc[u];
+    }
+    const std::int32_t r = g * kRowGroup + lane, n = len, k0 = kb;
+    const int4 b = w;
+    const T y0 = yold, d0 = dv;
+    __builtin_amdgcn_wave_barrier();
+    T xv[NI];
+#pragma unroll
+    for (int k = 0; k < NI; ++k)
+    {
+      const std::uint32_t c = col[max(min(k0 + k, k0 + n - 1), 0)];
+      const std::int32_t base = c & 0x8000u ? (c & 0x4000u ? b.w : b.z) : (c & 0x4000u ? b.y : b.x);
+      xv[k] = x[max(min(base + static_cast<std::int32_t>(c & 0x3fffu), ncols - 1), 0)];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const std::int32_t ng = 2 * (it + xr.step) + wave;
+    if (it + xr.step < xr.end && ng < ngroups)
+      stage(ng);
+    __builtin_amdgcn_sched_barrier(0);
+    T sum = T(0);
+#pragma unroll
+    for (int k = 0; k < NI; ++k)
+      if (k < n)
+        sum += val[k0 + k] * xv[k];
+    if (r < nrows)
+    {
+      const T yr = accumulate ? y0 + sum : sum;
+      y[r] = yr;
+      if (dotv)
+        d += double(yr) * double(d0);
+    }
+    __builtin_amdgcn_wave_barrier();
+  }
+  if (partials)
+  {
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1)
+      d += __shfl_down(d, off, 64);
+    if (lane == 0)
+      red[wave] = d;
+    __syncthreads();
+    if (threadIdx.x == 0)
+      partials[blockIdx.x] = red[0] + red[1];
+  }
 }
 
 /// Rows per slice of the sliced-ELL solver copy (one wavefront).
@@ -775,8 +1048,8 @@ int lanes_per_row(const dfx_csr& A)
     return 1; // sliced-ELL snapshot: one lane per row
   if (A.lanes)
     return A.lanes;
-  if (A.nblk > 0)
-    return 1; // stream kernel
+  if (A.nblk > 0 || A.win)
+    return 1; // row-lane or stream kernel
   const double mean = A.nrows ? double(A.nnz) / A.nrows : 1.0;
   int G = 2;
   while (G < 64 && G * 6 < mean)
@@ -821,6 +1094,8 @@ void prime_stream_grids()
 }
 
 constexpr int kMaxPartials = 2048;
+/// Bytes after the last value: the stream SpMV loads values in pairs.
+constexpr std::size_t kValuePad = 16;
 
 /// y (+)= A x through the sliced-ELL copy of A (its values as last
 /// copied), with the partial sums of y . dotv into partials when given.
@@ -857,6 +1132,32 @@ int launch_sell(const dfx_csr& A, const T* x, T* y, int accumulate, const T* dot
   return nb;
 }
 
+/// Whether the row-lane SpMV serves A (rows of at most kRowLaneMax entries
+/// whose groups' columns fit the windows), and its launch.
+inline bool use_rows(const dfx_csr& A) { return A.win && (A.lanes == 0 || A.lanes == 1); }
+
+template <typename T>
+int launch_rows(const dfx_csr& A, const T* x, T* y, int accumulate, const T* dotv,
+                double* partials, const int* stop)
+{
+  const std::int32_t ng = (A.nrows + kRowGroup - 1) / kRowGroup;
+  auto go = [&](auto kern)
+  {
+    const int nb = std::max(
+        1, std::min({(ng + 1) / 2,
+                     resident_blocks(reinterpret_cast<const void*>(kern), 2 * kRowGroup, 0),
+                     kMaxPartials}));
+    kern<<<nb, 2 * kRowGroup, 0, stream()>>>(A.nrows, ng, reinterpret_cast<const int4*>(A.win),
+                                             A.row_ptr, A.cols16, A.ncols,
+                                             static_cast<const T*>(A.values), x, y, accumulate,
+                                             dotv, partials, stop);
+    return nb;
+  };
+  return A.max_row <= 16   ? go(spmv_rows_k<T, 16>)
+         : A.max_row <= 27 ? go(spmv_rows_k<T, 27>)
+                           : go(spmv_rows_k<T, kRowLaneMax>);
+}
+
 template <typename T>
 void launch_spmv(const dfx_csr& A, const T* x, T* y, bool accumulate)
 {
@@ -868,14 +1169,16 @@ void launch_spmv(const dfx_csr& A, const T* x, T* y, bool accumulate)
     launch_sell<T>(A, x, y, accumulate ? 1 : 0, nullptr, nullptr, nullptr);
     return;
   }
-  if (A.bs == 1 && lanes_per_row(A) == 1)
+  if (use_rows(A))
+    launch_rows<T>(A, x, y, accumulate ? 1 : 0, nullptr, nullptr, nullptr);
+  else if (A.bs == 1 && lanes_per_row(A) == 1)
   {
     const int nb = std::max(
         1, std::min(A.nblk, resident_blocks(reinterpret_cast<const void*>(spmv_stream_k<T>),
                                             kBlock, 0)));
-    spmv_stream_k<T><<<nb, kBlock, 0, s>>>(A.nblk, row_blocks(A), A.row_ptr, A.cols,
-                                           static_cast<const T*>(A.values), x, y,
-                                           accumulate, nullptr, nullptr, nullptr);
+    spmv_stream_k<T><<<nb, kBlock, 0, s>>>(A.nblk, row_blocks(A), A.rbase, A.row_ptr, A.cols,
+                                           A.cols16, A.ncols, static_cast<const T*>(A.values), x,
+                                           y, accumulate, nullptr, nullptr, nullptr);
   }
   else if (A.bs == 1)
   {
@@ -1607,14 +1910,17 @@ int launch_cg_spmv(const dfx_csr& A, const T* p, T* q, CGState* st, bool sell)
   const T* v = static_cast<const T*>(A.values);
   if (sell)
     return launch_sell<T>(A, p, q, 0, p, st->partials, &st->done);
+  if (use_rows(A))
+    return launch_rows<T>(A, p, q, 0, p, st->partials, &st->done);
   if (A.bs == 1 && lanes_per_row(A) == 1)
   {
     const int nb = std::max(
         1, std::min({A.nblk,
                      resident_blocks(reinterpret_cast<const void*>(spmv_stream_k<T>), kBlock, 0),
                      kMaxPartials}));
-    spmv_stream_k<T><<<nb, kBlock, 0, s>>>(A.nblk, row_blocks(A), A.row_ptr, A.cols, v, p, q, 0, p,
-                                           st->partials, &st->done);
+    spmv_stream_k<T><<<nb, kBlock, 0, s>>>(A.nblk, row_blocks(A), A.rbase, A.row_ptr, A.cols,
+                                           A.cols16, A.ncols, v, p, q, 0, p, st->partials,
+                                           &st->done);
     return nb;
   }
   if (A.bs == 1)
@@ -2147,10 +2453,11 @@ dfx_status dfx_csr_create(const int64_t* row_ptr, const int32_t* cols, int32_t n
         A->cols = static_cast<std::int32_t*>(dmalloc(sizeof(std::int32_t) * std::max<std::int64_t>(nnz, 1)));
         A->diag = static_cast<std::int32_t*>(dmalloc(sizeof(std::int32_t) * std::max(nrows, 1)));
         const std::size_t vb = dtype_size(dtype) * std::size_t(nnz) * bs * bs;
-        A->values = dmalloc(std::max<std::size_t>(vb, 8));
+        A->values = dmalloc(vb + kValuePad);
         h2d(A->row_ptr, rp32.data(), sizeof(std::int32_t) * (nrows + 1));
         const std::int32_t chunk
-            = (dtype == DFX_F64 ? stream_chunk<double>() : stream_chunk<float>()) / bs;
+            = bs == 1 ? (dtype == DFX_F64 ? stream_entries<double>() : stream_entries<float>())
+                      : (dtype == DFX_F64 ? stream_chunk<double>() : stream_chunk<float>()) / bs;
         if (bs == 1 || (bs <= 3 && maxrow <= chunk))
         {
           // row blocks of the stream SpMV: greedy, at most kBlock / bs rows
@@ -2175,6 +2482,36 @@ dfx_status dfx_csr_create(const int64_t* row_ptr, const int32_t* cols, int32_t n
         }
         h2d(A->cols, cols, sizeof(std::int32_t) * nnz);
         DFX_HIP(hipMemsetAsync(A->values, 0, vb, stream()));
+        if (bs == 1 && nnz > 0)
+        {
+          A->cols16 = static_cast<std::uint16_t*>(dmalloc(sizeof(std::uint16_t) * (nnz + 2)));
+          // the place past an odd nnz is loaded (and its product dropped)
+          DFX_HIP(hipMemsetAsync(A->cols16 + nnz, 0, 2 * sizeof(std::uint16_t), stream()));
+          if (maxrow <= kRowLaneMax && nrows >= row_lane_min_rows(dtype, maxrow))
+          {
+            const std::int32_t ng = (nrows + kRowGroup - 1) / kRowGroup;
+            int4* win = static_cast<int4*>(dmalloc(sizeof(int4) * ng + sizeof(int)));
+            int* wide = reinterpret_cast<int*>(win + ng);
+            DFX_HIP(hipMemsetAsync(wide, 0, sizeof(int), stream()));
+            row_windows_k<<<(ng + 3) / 4, kBlock, 0, stream()>>>(nrows, ng, A->row_ptr, A->cols,
+                                                                win, A->cols16, wide);
+            check_launch("row_windows");
+            int h = 0;
+            d2h(&h, wide, sizeof(int));
+            A->win = win;
+            if (h)
+            {
+              dfree(win);
+              A->win = nullptr;
+            }
+          }
+          if (!A->win)
+          {
+            A->rbase = static_cast<std::int32_t*>(dmalloc(sizeof(std::int32_t) * A->nblk));
+            stream_cols_k<<<A->nblk, kBlock, 0, stream()>>>(row_blocks(*A), A->row_ptr, A->cols,
+                                                            A->rbase, A->cols16);
+          }
+        }
         if (nrows > 0)
           diag_pos_k<<<(nrows + kBlock - 1) / kBlock, kBlock, 0, stream()>>>(nrows, A->row_ptr, A->cols, A->diag);
         check_launch("csr_create");
@@ -2210,9 +2547,12 @@ dfx_status dfx_csr_create_shared(const dfx_csr* P, int dtype, dfx_csr** out)
           // the stream SpMV row blocks depend on the value size
           A->rblk = nullptr;
           A->nblk = 0;
+          A->rbase = nullptr;
+          if (!A->win)
+            A->cols16 = nullptr;
         }
         const std::size_t vb = dtype_size(dtype) * std::size_t(A->nnz) * A->bs * A->bs;
-        A->values = dmalloc(std::max<std::size_t>(vb, 8));
+        A->values = dmalloc(vb + kValuePad);
         // zeros stored when first read (an assembly overwrites them all)
         A->zeroed = true;
         A->zero_pending = true;
@@ -2228,6 +2568,9 @@ dfx_status dfx_csr_destroy(dfx_csr* A)
     {
       dfree(A->row_ptr);
       dfree(A->rblk);
+      dfree(A->rbase);
+      dfree(A->win);
+      dfree(A->cols16);
       dfree(A->cols);
       dfree(A->diag);
     }
