@@ -74,57 +74,6 @@ struct ChunkDesc
   std::int32_t sys, row0, row1, first; // first: chunk is the system's first
 };
 
-/// Sums of the system's NV partial arrays (c0 .. c0 + n of each), by the
-/// whole block in a fixed order; the results are returned to every thread.
-template <int NV>
-__device__ inline void sum_ranges(const double* const (&partials)[NV], int c0, int n,
-                                  double (&out)[NV])
-{
-  __shared__ double lds[NV][kBlock / 64];
-#pragma unroll
-  for (int k = 0; k < NV; ++k)
-  {
-    double a = 0;
-    for (int i = threadIdx.x; i < n; i += kBlock)
-      a += partials[k][c0 + i];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1)
-      a += __shfl_down(a, off, 64);
-    if ((threadIdx.x & 63) == 0)
-      lds[k][threadIdx.x >> 6] = a;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < NV; ++k)
-    out[k] = (lds[k][0] + lds[k][1]) + (lds[k][2] + lds[k][3]);
-  __syncthreads();
-}
-
-/// Block sums of NV values, stored at partials[k][slot].
-template <int NV>
-__device__ inline void store_block_sums(const double (&v)[NV], double* const (&partials)[NV],
-                                        int slot)
-{
-  __shared__ double lds[NV][kBlock / 64];
-#pragma unroll
-  for (int k = 0; k < NV; ++k)
-  {
-    double a = v[k];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1)
-      a += __shfl_down(a, off, 64);
-    if ((threadIdx.x & 63) == 0)
-      lds[k][threadIdx.x >> 6] = a;
-  }
-  __syncthreads();
-  if (threadIdx.x < NV)
-  {
-    const int k = threadIdx.x;
-    partials[k][slot] = (lds[k][0] + lds[k][1]) + (lds[k][2] + lds[k][3]);
-  }
-  __syncthreads();
-}
-
 /// Chunks of one workgroup: a contiguous range, and contiguous over the
 /// workgroups of an XCD, so that a system's partials are summed once per
 /// workgroup (not once per chunk) and both phases find their rows in the

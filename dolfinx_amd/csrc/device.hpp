@@ -101,15 +101,40 @@ __device__ inline XcdRange xcd_range(int n)
   return {lo + (b >> 3), hi, (nb - x + 7) >> 3};
 }
 
+/// One step of wave_sum: the value of the lane that DPP control C names
+/// (zero where there is none), added.
+template <int C, int ROWS>
+__device__ inline double dpp_add(double v)
+{
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(b), C, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(b >> 32), C, ROWS, 0xf, false);
+  return v + __hiloint2double(hi, lo);
+}
+
+/// Sum over a wavefront in a fixed order, valid in lane 63. Data moves
+/// between lanes in the vector pipeline (row shifts of 1, 2, 4 and 8 lanes
+/// inside rows of 16, then broadcasts of lanes 15 and 31): six dependent adds
+/// without the LDS round trip that each shuffle takes, in reductions that sit
+/// alone on the path of every CG iteration.
+__device__ inline double wave_sum(double v)
+{
+  v = dpp_add<0x111, 0xf>(v);
+  v = dpp_add<0x112, 0xf>(v);
+  v = dpp_add<0x114, 0xf>(v);
+  v = dpp_add<0x118, 0xf>(v);
+  v = dpp_add<0x142, 0xa>(v);
+  v = dpp_add<0x143, 0xc>(v);
+  return v;
+}
+
 /// Sum over a 256-thread block (4 wavefronts of 64); result valid in
 /// thread 0. Fixed order, so deterministic.
 __device__ inline double block_sum_256(double v, double* lds /*[4]*/)
 {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1)
-    v += __shfl_down(v, off, 64);
+  v = wave_sum(v);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  if (lane == 0)
+  if (lane == 63)
     lds[wave] = v;
   __syncthreads();
   double s = 0;
@@ -165,6 +190,54 @@ __device__ inline double sum_partials(const double* partials, int n)
   const double t = total;
   __syncthreads();
   return t;
+}
+
+/// Sums of n values from c0 of each of NV partial arrays, by a 256-thread
+/// block in a fixed order; the results are returned to every thread (two
+/// barriers whatever NV is).
+template <int NV>
+__device__ inline void sum_ranges(const double* const (&partials)[NV], int c0, int n,
+                                  double (&out)[NV])
+{
+  __shared__ double lds[NV][4];
+#pragma unroll
+  for (int k = 0; k < NV; ++k)
+  {
+    double a = 0;
+    for (int i = threadIdx.x; i < n; i += 256)
+      a += partials[k][c0 + i];
+    a = wave_sum(a);
+    if ((threadIdx.x & 63) == 63)
+      lds[k][threadIdx.x >> 6] = a;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < NV; ++k)
+    out[k] = (lds[k][0] + lds[k][1]) + (lds[k][2] + lds[k][3]);
+  __syncthreads();
+}
+
+/// Sums of NV values over a 256-thread block, stored at partials[k][slot].
+template <int NV>
+__device__ inline void store_block_sums(const double (&v)[NV], double* const (&partials)[NV],
+                                        int slot)
+{
+  __shared__ double lds[NV][4];
+#pragma unroll
+  for (int k = 0; k < NV; ++k)
+  {
+    double a = v[k];
+    a = wave_sum(a);
+    if ((threadIdx.x & 63) == 63)
+      lds[k][threadIdx.x >> 6] = a;
+  }
+  __syncthreads();
+  if (threadIdx.x < NV)
+  {
+    const int k = threadIdx.x;
+    partials[k][slot] = (lds[k][0] + lds[k][1]) + (lds[k][2] + lds[k][3]);
+  }
+  __syncthreads();
 }
 
 } // namespace dfx

@@ -232,6 +232,99 @@ __device__ inline void lds_barrier()
   __builtin_amdgcn_s_barrier();
 }
 
+constexpr int kMaxPartials = 2048;
+
+struct CGState
+{
+  double rz[2];
+  double rr0, rr, tol2;
+  std::int32_t iter, done, max_it;
+  std::int32_t kd; // iteration the direction kernel completes (set by the update
+                   // kernel); two-kernel iteration: iterations done
+  std::int32_t tested, pad; // two-kernel iteration: see cg_begin
+  double partials[3 * kMaxPartials];
+};
+
+/// Two consecutive values, aligned to their size.
+template <typename T>
+using Pair = T __attribute__((ext_vector_type(2)));
+
+/// What the SpMV of the two-kernel CG iteration forms its vector from: per
+/// entry the pair (z, previous p), p = z + beta p; p is stored too.
+template <typename T>
+struct DirArgs
+{
+  const Pair<T>* zp;
+  T* p;
+  int nb_upd; // partials of the update kernel
+  CGState* st;
+};
+
+template <typename T>
+__device__ inline T dir_of(Pair<T> g, T beta)
+{
+  return __builtin_fma(beta, g.y, g.x);
+}
+
+/// Start of the SpMV of iteration k: the stop test ||r||^2/||r0||^2 < rtol^2
+/// or max_it and beta = rz_k / rz_{k-1} from the partials of the last update
+/// (or from the state, where cg_start_finish_k or cg_finish_k already put
+/// them: tested = k). Every workgroup reaches the same decision; workgroup 0
+/// records it. Nothing that another workgroup reads here is written here
+/// but done, which is read once per workgroup. False: stopped.
+template <typename T>
+__device__ inline bool cg_begin(const DirArgs<T>& dir, T& beta)
+{
+  __shared__ double lds[2][4];
+  __shared__ int done;
+  CGState* st = dir.st;
+  const int k = st->kd;
+  const bool known = st->tested == k;
+  if (threadIdx.x == 0)
+    done = __hip_atomic_load(&st->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  double s[2] = {0.0, 0.0};
+  if (!known)
+  {
+    const double* pr = st->partials + kMaxPartials;
+    for (int i = threadIdx.x; i < dir.nb_upd; i += 256)
+    {
+      s[0] += pr[i];
+      s[1] += pr[dir.nb_upd + i];
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < 2; ++q)
+  {
+    s[q] = wave_sum(s[q]);
+    if ((threadIdx.x & 63) == 63)
+      lds[q][threadIdx.x >> 6] = s[q];
+  }
+  __syncthreads();
+  if (done)
+    return false;
+  const bool writer = blockIdx.x == 0 && threadIdx.x == 0;
+  if (known)
+  {
+    beta = k > 0 ? static_cast<T>(st->rz[k & 1] / st->rz[(k - 1) & 1]) : T(0);
+    if (writer)
+      st->iter = k;
+    return true;
+  }
+  const double rz = (lds[0][0] + lds[0][1]) + (lds[0][2] + lds[0][3]);
+  const double rr = (lds[1][0] + lds[1][1]) + (lds[1][2] + lds[1][3]);
+  const bool stop = rr / st->rr0 < st->tol2 || k >= st->max_it;
+  if (writer)
+  {
+    st->rz[k & 1] = rz;
+    st->rr = rr;
+    st->iter = k;
+    if (stop)
+      __hip_atomic_store(&st->done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  beta = static_cast<T>(rz / st->rz[(k - 1) & 1]);
+  return !stop;
+}
+
 /// Entries per LDS chunk of the stream SpMV (16 KB of products).
 template <typename T>
 constexpr int stream_chunk()
@@ -283,10 +376,6 @@ __global__ void __launch_bounds__(kBlock)
       c16[j] = static_cast<std::uint16_t>(ci[j] - first);
 }
 
-/// Two consecutive values, aligned to their size.
-template <typename T>
-using Pair = T __attribute__((ext_vector_type(2)));
-
 /// Stream CSR SpMV, y (+)= A x. Each row block (consecutive rows whose
 /// entries fit one chunk) is processed by one workgroup: the products
 /// v_j x[c_j] of the block's contiguous entry range are formed with fully
@@ -303,17 +392,18 @@ using Pair = T __attribute__((ext_vector_type(2)));
 /// entries, 47 per row: 43 rows in a chunk) 36 us; with one thread per row
 /// the sums, 47 LDS reads one after the other in 43 of the 256 threads, took
 /// longer than the loads and the product 72 us.
-template <typename T>
+template <typename T, bool DIR>
 __global__ void __launch_bounds__(kBlock)
     spmv_stream_k(std::int32_t nblk, const int2* __restrict__ rbj,
                   const std::int32_t* __restrict__ rbase, const std::int32_t* __restrict__ rp,
                   const std::int32_t* __restrict__ ci, const std::uint16_t* __restrict__ c16,
                   std::int32_t ncols, const T* __restrict__ v, const T* __restrict__ x,
                   T* __restrict__ y, int accumulate, const T* __restrict__ dotv,
-                  double* partials, const int* stop)
+                  double* partials, const int* stop, DirArgs<T> dir)
 {
-  if (stop && block_flag(stop))
+  if (!DIR && stop && block_flag(stop))
     return;
+  T beta = T(0);
   constexpr int NC = stream_chunk<T>();
   constexpr int U = NC / (2 * kBlock); // pairs per thread
   __shared__ Pair<T> prod2[NC / 2];
@@ -331,6 +421,7 @@ __global__ void __launch_bounds__(kBlock)
     std::int32_t r, kb, ke;
     int lg;
     T yold, dv;
+    Pair<T> own; // DIR: the row's (z, previous p)
   };
   auto bounds = [&](int b) -> Bounds
   {
@@ -342,16 +433,21 @@ __global__ void __launch_bounds__(kBlock)
     int lg = 0;
     while (lg < 6 && (static_cast<std::uint32_t>(B.r1 - B.r0) << (lg + 1)) <= kBlock)
       ++lg;
-    Row w{B.r0 + static_cast<std::int32_t>(threadIdx.x >> lg), 0, 0, lg, T(0), T(0)};
+    Row w{B.r0 + static_cast<std::int32_t>(threadIdx.x >> lg), 0, 0, lg, T(0), T(0), Pair<T>(T(0))};
     if (w.r < B.r1)
     {
       const std::int32_t j00 = B.j0 & ~1;
       w.kb = rp[w.r] - j00;
       w.ke = rp[w.r + 1] - j00;
-      if (accumulate)
-        w.yold = y[w.r];
-      if (dotv)
-        w.dv = dotv[w.r];
+      if constexpr (DIR)
+        w.own = dir.zp[w.r];
+      else
+      {
+        if (accumulate)
+          w.yold = y[w.r];
+        if (dotv)
+          w.dv = dotv[w.r];
+      }
     }
     return w;
   };
@@ -396,37 +492,79 @@ __global__ void __launch_bounds__(kBlock)
       }
     }
   };
+  // x at a column; DIR: the pair, reduced to p when used
+  using X = std::conditional_t<DIR, Pair<T>, T>;
+  auto gather = [&](std::int32_t c) -> X
+  {
+    if constexpr (DIR)
+      return dir.zp[c];
+    else
+      return x[c];
+  };
+  auto value = [&](X g) -> T
+  {
+    if constexpr (DIR)
+      return dir_of<T>(g, beta);
+    else
+      return g;
+  };
+  // result of a row
+  auto finish = [&](const Row& w, T sum)
+  {
+    if constexpr (DIR)
+    {
+      const T pi = dir_of<T>(w.own, beta);
+      y[w.r] = sum;
+      dir.p[w.r] = pi;
+      d[0] += double(sum) * double(pi);
+    }
+    else
+    {
+      const T yr = accumulate ? w.yold + sum : sum;
+      y[w.r] = yr;
+      if (dotv)
+        d[0] += double(yr) * double(w.dv);
+    }
+  };
   const XcdRange xr = xcd_range(nblk);
   int bi = xr.first;
+  Bounds cur{0, 0, 0, 0, 0};
+  Row row{0, 0, 0, 0, T(0), T(0), Pair<T>(T(0))};
+  auto is_short = [](const Bounds& B) { return B.j1 - B.j0 <= stream_entries<T>(); };
   if (bi < xr.end)
   {
-    Bounds cur = bounds(bi);
-    auto is_short = [](const Bounds& B) { return B.j1 - B.j0 <= stream_entries<T>(); };
+    cur = bounds(bi);
     if (is_short(cur) && cur.j1 > cur.j0)
       stage(cur);
-    Row row = row_of(cur);
+    row = row_of(cur);
+  }
+  if constexpr (DIR)
+    if (!cg_begin<T>(dir, beta))
+      return;
+  if (bi < xr.end)
+  {
     int nbi = bi + xr.step;
     Bounds nxt = nbi < xr.end ? bounds(nbi) : Bounds{0, 0, 0, 0, 0};
     for (;;)
     {
       const bool more = nbi < xr.end;
       const int nnbi = nbi + xr.step;
-      Row nrow{0, 0, 0, 0, T(0), T(0)};
+      Row nrow{0, 0, 0, 0, T(0), T(0), Pair<T>(T(0))};
       Bounds nnxt{0, 0, 0, 0, 0};
       if (is_short(cur))
       {
         if (cur.j1 > cur.j0)
         {
-          T xv[U][2];
+          X xv[U][2];
 #pragma unroll
           for (int u = 0; u < U; ++u)
           {
-            xv[u][0] = x[cc[u][0]];
-            xv[u][1] = x[cc[u][1]];
+            xv[u][0] = gather(cc[u][0]);
+            xv[u][1] = gather(cc[u][1]);
           }
 #pragma unroll
           for (int u = 0; u < U; ++u)
-            prod2[threadIdx.x + u * kBlock] = Pair<T>{vv[u].x * xv[u][0], vv[u].y * xv[u][1]};
+            prod2[threadIdx.x + u * kBlock] = Pair<T>{vv[u].x * value(xv[u][0]), vv[u].y * value(xv[u][1])};
         }
         lds_barrier();
         // the next block's loads go out before the sums
@@ -455,27 +593,17 @@ __global__ void __launch_bounds__(kBlock)
         for (int off = step >> 1; off > 0; off >>= 1)
           sum += __shfl_xor(sum, off, 64);
         if (lane == 0 && row.r < cur.r1)
-        {
-          const T yr = accumulate ? row.yold + sum : sum;
-          y[row.r] = yr;
-          if (dotv)
-            d[0] += double(yr) * double(row.dv);
-        }
+          finish(row, sum);
         lds_barrier();
       }
       else
       {
         double sum = 0;
         for (std::int32_t j = cur.j0 + threadIdx.x; j < cur.j1; j += kBlock)
-          sum += double(v[j] * x[ci[j]]);
+          sum += double(v[j] * value(gather(ci[j])));
         const double t = block_sum_256(sum, red);
         if (threadIdx.x == 0)
-        {
-          const T yr = accumulate ? row.yold + static_cast<T>(t) : static_cast<T>(t);
-          y[cur.r0] = yr;
-          if (dotv)
-            d[0] += double(yr) * double(row.dv);
-        }
+          finish(row, static_cast<T>(t));
         if (more)
         {
           if (is_short(nxt) && nxt.j1 > nxt.j0)
@@ -671,10 +799,8 @@ __global__ void __launch_bounds__(2 * kRowGroup)
   }
   if (partials)
   {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1)
-      d += __shfl_down(d, off, 64);
-    if (lane == 0)
+    d = wave_sum(d);
+    if (lane == 63)
       red[wave] = d;
     __syncthreads();
     if (threadIdx.x == 0)
@@ -778,15 +904,22 @@ __global__ void __launch_bounds__(kBlock)
 /// reference's row loop; padding is skipped. Workgroups take groups of 4
 /// slices, each XCD a contiguous range. With dotv, partial sums of y.dotv
 /// go to partials.
-template <typename T, int G>
+template <typename T, int G, bool DIR>
 __global__ void __launch_bounds__(kBlock)
     sell_spmv_k(std::int32_t nrows, std::int32_t nslices, const std::int64_t* __restrict__ off,
                 const std::int32_t* __restrict__ cbase, const std::int32_t* __restrict__ rp,
                 const unsigned char* __restrict__ cols, const T* __restrict__ sval,
                 const T* __restrict__ x, T* __restrict__ y, int accumulate,
-                const T* __restrict__ dotv, double* partials, const int* stop)
+                const T* __restrict__ dotv, double* partials, const int* stop,
+                DirArgs<T> dir)
 {
-  if (stop && block_flag(stop))
+  T beta = T(0);
+  if constexpr (DIR)
+  {
+    if (!cg_begin<T>(dir, beta))
+      return;
+  }
+  else if (stop && block_flag(stop))
     return;
   double d[1] = {0.0};
   const int lane = threadIdx.x % kSlice, wave = threadIdx.x / kSlice;
@@ -806,7 +939,8 @@ __global__ void __launch_bounds__(kBlock)
     T sum = T(0);
     for (std::int32_t k = 0; k < w; k += G)
     {
-      T vv[G], xv[G];
+      T vv[G];
+      std::conditional_t<DIR, Pair<T>, T> xv[G];
       std::int32_t cc[G];
       if (b >= 0)
       {
@@ -832,17 +966,37 @@ __global__ void __launch_bounds__(kBlock)
       }
 #pragma unroll
       for (int u = 0; u < G; ++u)
-        xv[u] = x[cc[u]];
+      {
+        if constexpr (DIR)
+          xv[u] = dir.zp[cc[u]];
+        else
+          xv[u] = x[cc[u]];
+      }
       {
         // product then sum, not a fused multiply-add
 #pragma clang fp contract(off)
 #pragma unroll
         for (int u = 0; u < G; ++u)
           if (k + u < len)
-            sum = sum + vv[u] * xv[u];
+          {
+            if constexpr (DIR)
+              sum = sum + vv[u] * dir_of<T>(xv[u], beta);
+            else
+              sum = sum + vv[u] * xv[u];
+          }
       }
     }
-    if (r < nrows)
+    if constexpr (DIR)
+    {
+      if (r < nrows)
+      {
+        const T pi = dir_of<T>(dir.zp[r], beta);
+        y[r] = sum;
+        dir.p[r] = pi;
+        d[0] += double(sum) * double(pi);
+      }
+    }
+    else if (r < nrows)
     {
       const T yr = accumulate ? y[r] + sum : sum;
       y[r] = yr;
@@ -854,25 +1008,38 @@ __global__ void __launch_bounds__(kBlock)
     block_partials<1>(d, partials);
 }
 
+/// Tasks (block, block-row component) of a row block of the block stream
+/// SpMV for matrices of rows up to max_row blocks: 1024, so that four tasks
+/// per thread and their loads leave room for more wavefronts; the 16 KB of
+/// products that a longer row needs otherwise.
+template <typename T>
+inline int bsr_chunk(std::int32_t max_row, int bs)
+{
+  return std::int64_t(max_row) * bs <= 1024 ? 1024 : stream_chunk<T>();
+}
+
 /// Stream SpMV of a block-CSR matrix with BS x BS blocks (row-major inside
 /// a block), y (+)= A x. Row blocks hold at most kBlock / BS block rows and
-/// stream_chunk / BS blocks. Phase 1: task t = (block b, block-row component
-/// a) loads the BS contiguous values of that block row (consecutive tasks
-/// read consecutive addresses) and the BS entries of x, and stores their
-/// product sum in LDS; phase 2: one thread per (block row, component) sums
-/// its row's block products left to right. The next row block's entries
-/// are loaded while the current rows are summed.
-template <typename T, int BS>
+/// NC / BS blocks (bsr_chunk). Phase 1: task t = (block b, block-row
+/// component a) loads the BS contiguous values of that block row
+/// (consecutive tasks read consecutive addresses) and the BS entries of x,
+/// and stores their product sum in LDS; phase 2: 2^lg threads per (block
+/// row, component), as many as the workgroup has, sum its products. The next
+/// row block's entries are loaded while the current rows are summed. P2
+/// elasticity on 24 x 19 x 17 cubes (1.84 M blocks, 140 MB) 24.9 us = 5.6
+/// TB/s; with eight tasks per thread (4 wavefronts per SIMD) and one thread
+/// per row and component 30.1 us.
+template <typename T, int BS, int NC, bool DIR>
 __global__ void __launch_bounds__(kBlock)
     bsr_stream_k(std::int32_t nblk, const int2* __restrict__ rbj,
                  const std::int32_t* __restrict__ rp, const std::int32_t* __restrict__ ci,
                  const T* __restrict__ v, const T* __restrict__ x, T* __restrict__ y,
                  int accumulate, const T* __restrict__ dotv, double* partials,
-                 const int* stop)
+                 const int* stop, DirArgs<T> dir)
 {
-  if (stop && block_flag(stop))
+  if (!DIR && stop && block_flag(stop))
     return;
-  constexpr int NC = stream_chunk<T>();        // products per chunk
+  T beta = T(0);
   constexpr int U = NC / kBlock;               // tasks per thread
   __shared__ T prod[NC];
   double d[1] = {0.0};
@@ -920,35 +1087,54 @@ __global__ void __launch_bounds__(kBlock)
     if (j1 > j0)
       stage();
   }
+  if constexpr (DIR)
+    if (!cg_begin<T>(dir, beta))
+      return;
   while (bi < xr.end)
   {
     const int nbi = bi + xr.step;
     const std::int32_t ntask = (j1 - j0) * BS;
-    T xv[U][BS];
+    std::conditional_t<DIR, Pair<T>, T> xv[U][BS];
 #pragma unroll
     for (int u = 0; u < U; ++u)
     {
-      const T* xx = x + std::int64_t(cc[u]) * BS;
+      const std::int64_t at = std::int64_t(cc[u]) * BS;
 #pragma unroll
       for (int k = 0; k < BS; ++k)
-        xv[u][k] = xx[k];
+      {
+        if constexpr (DIR)
+          xv[u][k] = dir.zp[at + k];
+        else
+          xv[u][k] = x[at + k];
+      }
     }
+    auto value = [&](auto g) -> T
+    {
+      if constexpr (DIR)
+        return dir_of<T>(g, beta);
+      else
+        return g;
+    };
 #pragma unroll
     for (int u = 0; u < U; ++u)
     {
       const std::int32_t t = threadIdx.x + u * kBlock;
       if (t < ntask)
       {
-        T s = vv[u][0] * xv[u][0];
+        T s = vv[u][0] * value(xv[u][0]);
 #pragma unroll
         for (int k = 1; k < BS; ++k)
-          s += vv[u][k] * xv[u][k];
+          s += vv[u][k] * value(xv[u][k]);
         prod[t] = s;
       }
     }
     lds_barrier();
-    const std::int32_t br = r0 + static_cast<std::int32_t>(threadIdx.x) / BS;
-    const int comp = static_cast<int>(threadIdx.x) % BS;
+    int lg = 0;
+    while (lg < 6 && ((r1 - r0) * BS << (lg + 1)) <= kBlock)
+      ++lg;
+    const int step = 1 << lg, lane = threadIdx.x & (step - 1), item = threadIdx.x >> lg;
+    const std::int32_t br = r0 + item / BS;
+    const int comp = item % BS;
     const bool has = br < r1;
     std::int32_t kb = 0, ke = 0;
     const std::int64_t yi = std::int64_t(br) * BS + comp;
@@ -957,10 +1143,15 @@ __global__ void __launch_bounds__(kBlock)
     {
       kb = rp[br] - j0;
       ke = rp[br + 1] - j0;
-      if (accumulate)
-        yold = y[yi];
-      if (dotv)
-        dv = dotv[yi];
+      if constexpr (DIR)
+        dv = dir_of<T>(dir.zp[yi], beta);
+      else
+      {
+        if (accumulate)
+          yold = y[yi];
+        if (dotv)
+          dv = dotv[yi];
+      }
     }
     if (nbi < xr.end)
     {
@@ -968,15 +1159,38 @@ __global__ void __launch_bounds__(kBlock)
       if (j1 > j0)
         stage();
     }
-    if (has)
+    T s = 0;
     {
-      T s = 0;
-      for (std::int32_t k = kb; k < ke; ++k)
+      std::int32_t k = kb + lane;
+      for (; k + 3 * step < ke; k += 4 * step)
+      {
+        const T p0 = prod[k * BS + comp], p1 = prod[(k + step) * BS + comp],
+                p2 = prod[(k + 2 * step) * BS + comp], p3 = prod[(k + 3 * step) * BS + comp];
+        s += p0;
+        s += p1;
+        s += p2;
+        s += p3;
+      }
+      for (; k < ke; k += step)
         s += prod[k * BS + comp];
-      const T yr = accumulate ? yold + s : s;
-      y[yi] = yr;
-      if (dotv)
-        d[0] += double(yr) * double(dv);
+    }
+    for (int off = step >> 1; off > 0; off >>= 1)
+      s += __shfl_xor(s, off, 64);
+    if (has && lane == 0)
+    {
+      if constexpr (DIR)
+      {
+        y[yi] = s;
+        dir.p[yi] = dv;
+        d[0] += double(s) * double(dv);
+      }
+      else
+      {
+        const T yr = accumulate ? yold + s : s;
+        y[yi] = yr;
+        if (dotv)
+          d[0] += double(yr) * double(dv);
+      }
     }
     lds_barrier();
     bi = nbi;
@@ -1082,27 +1296,32 @@ void prime_stream_grids()
   std::call_once(once,
                  []
                  {
-                   const void* k[] = {reinterpret_cast<const void*>(spmv_stream_k<double>),
-                                      reinterpret_cast<const void*>(spmv_stream_k<float>),
-                                      reinterpret_cast<const void*>(bsr_stream_k<double, 3>),
-                                      reinterpret_cast<const void*>(bsr_stream_k<float, 3>),
-                                      reinterpret_cast<const void*>(bsr_stream_k<double, 2>),
-                                      reinterpret_cast<const void*>(bsr_stream_k<float, 2>)};
+                   const void* k[] = {reinterpret_cast<const void*>(spmv_stream_k<double, false>),
+                                      reinterpret_cast<const void*>(bsr_stream_k<double, 3, 1024, false>),
+                                      reinterpret_cast<const void*>(bsr_stream_k<double, 2, 1024, false>),
+                                      reinterpret_cast<const void*>(spmv_stream_k<float, false>),
+                                      reinterpret_cast<const void*>(bsr_stream_k<float, 3, 1024, false>),
+                                      reinterpret_cast<const void*>(bsr_stream_k<float, 2, 1024, false>),
+                                      reinterpret_cast<const void*>(spmv_stream_k<double, true>),
+                                      reinterpret_cast<const void*>(bsr_stream_k<double, 3, 1024, true>),
+                                      reinterpret_cast<const void*>(bsr_stream_k<double, 2, 1024, true>),
+                                      reinterpret_cast<const void*>(spmv_stream_k<float, true>),
+                                      reinterpret_cast<const void*>(bsr_stream_k<float, 3, 1024, true>),
+                                      reinterpret_cast<const void*>(bsr_stream_k<float, 2, 1024, true>)};
                    for (const void* f : k)
                      resident_blocks(f, kBlock, 0);
                  });
 }
 
-constexpr int kMaxPartials = 2048;
 /// Bytes after the last value: the stream SpMV loads values in pairs.
 constexpr std::size_t kValuePad = 16;
 
 /// y (+)= A x through the sliced-ELL copy of A (its values as last
-/// copied), with the partial sums of y . dotv into partials when given.
-/// Returns the number of workgroups.
-template <typename T>
+/// copied), with the partial sums of y . dotv into partials when given; DIR:
+/// q = A p of the two-kernel CG. Returns the number of workgroups.
+template <typename T, bool DIR = false>
 int launch_sell(const dfx_csr& A, const T* x, T* y, int accumulate, const T* dotv,
-                double* partials, const int* stop)
+                double* partials, const int* stop, DirArgs<T> dir = {})
 {
   // 1024 workgroups (16 wavefronts per CU) keep the stream fed and halve
   // the partials a reduction sums
@@ -1119,17 +1338,54 @@ int launch_sell(const dfx_csr& A, const T* x, T* y, int accumulate, const T* dot
     kern<<<nb, kBlock, 0, stream()>>>(A.nrows, A.nslices, A.sell_off, A.sell_base, A.row_ptr,
                                       static_cast<const unsigned char*>(A.sell_cols),
                                       static_cast<const T*>(A.sell_vals), x, y, accumulate, dotv,
-                                      partials, stop);
+                                      partials, stop, dir);
   };
   if (G == 9)
-    go(sell_spmv_k<T, 9>);
+    go(sell_spmv_k<T, 9, DIR>);
   else if (G == 12)
-    go(sell_spmv_k<T, 12>);
+    go(sell_spmv_k<T, 12, DIR>);
   else if (G == 8)
-    go(sell_spmv_k<T, 8>);
+    go(sell_spmv_k<T, 8, DIR>);
   else
-    go(sell_spmv_k<T, 16>);
+    go(sell_spmv_k<T, 16, DIR>);
   return nb;
+}
+
+/// The same through the stream kernels (scalar, and block sizes 2 and 3).
+template <typename T, bool DIR = false>
+int launch_stream(const dfx_csr& A, const T* x, T* y, int accumulate, const T* dotv,
+                  double* partials, const int* stop, DirArgs<T> dir = {})
+{
+  const T* v = static_cast<const T*>(A.values);
+  auto grid = [&](const void* kern)
+  {
+    const int nb = std::min(A.nblk, resident_blocks(kern, kBlock, 0));
+    return std::max(1, partials ? std::min(nb, kMaxPartials) : nb);
+  };
+  auto block = [&](auto kern)
+  {
+    const int nb = grid(reinterpret_cast<const void*>(kern));
+    kern<<<nb, kBlock, 0, stream()>>>(A.nblk, row_blocks(A), A.row_ptr, A.cols, v, x, y,
+                                      accumulate, dotv, partials, stop, dir);
+    return nb;
+  };
+  constexpr int NC = stream_chunk<T>();
+  const bool small = bsr_chunk<T>(A.max_row, A.bs) == 1024;
+  if (A.bs == 3)
+    return small ? block(bsr_stream_k<T, 3, 1024, DIR>) : block(bsr_stream_k<T, 3, NC, DIR>);
+  if (A.bs == 2)
+    return small ? block(bsr_stream_k<T, 2, 1024, DIR>) : block(bsr_stream_k<T, 2, NC, DIR>);
+  const int nb = grid(reinterpret_cast<const void*>(spmv_stream_k<T, DIR>));
+  spmv_stream_k<T, DIR><<<nb, kBlock, 0, stream()>>>(A.nblk, row_blocks(A), A.rbase, A.row_ptr,
+                                                     A.cols, A.cols16, A.ncols, v, x, y,
+                                                     accumulate, dotv, partials, stop, dir);
+  return nb;
+}
+
+/// Whether the stream kernel serves the block matrix A.
+inline bool block_stream(const dfx_csr& A)
+{
+  return A.nblk > 0 && A.lanes <= 1 && (A.bs == 2 || A.bs == 3);
 }
 
 /// Whether the row-lane SpMV serves A (rows of at most kRowLaneMax entries
@@ -1172,14 +1428,7 @@ void launch_spmv(const dfx_csr& A, const T* x, T* y, bool accumulate)
   if (use_rows(A))
     launch_rows<T>(A, x, y, accumulate ? 1 : 0, nullptr, nullptr, nullptr);
   else if (A.bs == 1 && lanes_per_row(A) == 1)
-  {
-    const int nb = std::max(
-        1, std::min(A.nblk, resident_blocks(reinterpret_cast<const void*>(spmv_stream_k<T>),
-                                            kBlock, 0)));
-    spmv_stream_k<T><<<nb, kBlock, 0, s>>>(A.nblk, row_blocks(A), A.rbase, A.row_ptr, A.cols,
-                                           A.cols16, A.ncols, static_cast<const T*>(A.values), x,
-                                           y, accumulate, nullptr, nullptr, nullptr);
-  }
+    launch_stream<T>(A, x, y, accumulate ? 1 : 0, nullptr, nullptr, nullptr);
   else if (A.bs == 1)
   {
     const int G = lanes_per_row(A);
@@ -1206,17 +1455,9 @@ void launch_spmv(const dfx_csr& A, const T* x, T* y, bool accumulate)
   else
   {
     const T* v = static_cast<const T*>(A.values);
-    if (A.nblk > 0 && A.lanes <= 1 && (A.bs == 2 || A.bs == 3))
+    if (block_stream(A))
     {
-      const void* kern = A.bs == 3 ? reinterpret_cast<const void*>(bsr_stream_k<T, 3>)
-                                   : reinterpret_cast<const void*>(bsr_stream_k<T, 2>);
-      const int nb = std::max(1, std::min(A.nblk, resident_blocks(kern, kBlock, 0)));
-      if (A.bs == 3)
-        bsr_stream_k<T, 3><<<nb, kBlock, 0, s>>>(A.nblk, row_blocks(A), A.row_ptr, A.cols, v, x, y,
-                                                 accumulate, nullptr, nullptr, nullptr);
-      else
-        bsr_stream_k<T, 2><<<nb, kBlock, 0, s>>>(A.nblk, row_blocks(A), A.row_ptr, A.cols, v, x, y,
-                                                 accumulate, nullptr, nullptr, nullptr);
+      launch_stream<T>(A, x, y, accumulate ? 1 : 0, nullptr, nullptr, nullptr);
       check_launch("spmv");
       return;
     }
@@ -1233,8 +1474,11 @@ void launch_spmv(const dfx_csr& A, const T* x, T* y, bool accumulate)
 }
 
 // ---------------------------------------------------------------------
-// Conjugate gradients, device resident. Three kernels per iteration k,
-// no atomics and no host round trip:
+// Conjugate gradients, device resident, no atomics and no host round trip.
+// With a sliced-ELL or stream SpMV an iteration is two kernels: the SpMV
+// forms p = z + beta p where it gathers it (cg_begin, DirArgs) and
+// cg_pair_update_k does the rest. Otherwise (and where the work vectors are
+// fixed, as without allocation) three kernels per iteration k:
 //   cg_spmv_k      q = A p, partial sums of p.q
 //   cg_update_k    alpha = rz_k / p.q (each block sums the partials);
 //                  x += alpha p, r -= alpha q; partials of r.z and r.r
@@ -1246,14 +1490,6 @@ void launch_spmv(const dfx_csr& A, const T* x, T* y, bool accumulate)
 // ---------------------------------------------------------------------
 
 
-struct CGState
-{
-  double rz[2];
-  double rr0, rr, tol2;
-  std::int32_t iter, done, max_it;
-  std::int32_t kd; // iteration the direction kernel completes (set by the update kernel)
-  double partials[3 * kMaxPartials];
-};
 
 /// Jacobi inverse diagonal of a (block) CSR matrix: 1 / A[i,i].
 template <typename T>
@@ -1270,10 +1506,12 @@ __global__ void __launch_bounds__(kBlock)
   dinv[t] = d != T(0) ? T(1) / d : T(1);
 }
 
-/// r = b - y; p = z = dinv r; partial sums of (r.z, r.r)
+/// r = b - y; p = z = dinv r, or with zp the pairs (z, 0) of the two-kernel
+/// iteration; partial sums of (r.z, r.r)
 template <typename T>
 __global__ void __launch_bounds__(kBlock)
-    cg_start_k(std::int64_t n, const T* b, const T* y, const T* dinv, T* r, T* p, CGState* st)
+    cg_start_k(std::int64_t n, const T* b, const T* y, const T* dinv, T* r, T* p, Pair<T>* zp,
+               CGState* st)
 {
   double s[2] = {0.0, 0.0};
   for (std::int64_t i = blockIdx.x * std::int64_t(kBlock) + threadIdx.x; i < n;
@@ -1282,7 +1520,10 @@ __global__ void __launch_bounds__(kBlock)
     const T ri = b[i] - y[i];
     const T zi = dinv ? dinv[i] * ri : ri;
     r[i] = ri;
-    p[i] = zi;
+    if (zp)
+      zp[i] = Pair<T>{zi, T(0)};
+    else
+      p[i] = zi;
     s[0] += double(ri) * double(zi);
     s[1] += double(ri) * double(ri);
   }
@@ -1300,6 +1541,8 @@ __global__ void __launch_bounds__(kBlock) cg_start_finish_k(int nb, CGState* st)
     st->rr0 = rr;
     st->rr = rr;
     st->iter = 0;
+    st->kd = 0;
+    st->tested = 0;
     st->done = (rr == 0.0 || st->max_it <= 0) ? 1 : 0;
   }
 }
@@ -1428,6 +1671,120 @@ __global__ void __launch_bounds__(kBlock)
     p[i] = (dinv ? dinv[i] * r[i] : r[i]) + beta * p[i];
 }
 
+/// Second kernel of the two-kernel iteration: alpha = rz_k / p.q; x +=
+/// alpha p, r -= alpha q, the pairs (dinv r, p) that the next SpMV gathers,
+/// partials of r.z and r.r. Two elements per 16-byte load, the first four of
+/// a thread in flight while the partials of p.q are summed.
+template <typename T>
+__global__ void __launch_bounds__(kBlock)
+    cg_pair_update_k(std::int64_t n, int nb_spmv, T* __restrict__ x, T* __restrict__ r,
+                     const T* __restrict__ p, const T* __restrict__ q,
+                     const T* __restrict__ dinv, Pair<T>* __restrict__ zp, CGState* st)
+{
+  __shared__ double lds[4];
+  __shared__ int done;
+  constexpr int E = 2; // pairs of elements per thread and step
+  const std::int64_t np = n / 2, step = std::int64_t(gridDim.x) * kBlock;
+  std::int64_t i = blockIdx.x * std::int64_t(kBlock) + threadIdx.x;
+  Pair<T> vx[E], vr[E], vp[E], vq[E], vd[E];
+  auto load = [&]()
+  {
+#pragma unroll
+    for (int u = 0; u < E; ++u)
+    {
+      const std::int64_t j = i + u * step;
+      if (j < np)
+      {
+        vx[u] = reinterpret_cast<const Pair<T>*>(x)[j];
+        vr[u] = reinterpret_cast<const Pair<T>*>(r)[j];
+        vp[u] = reinterpret_cast<const Pair<T>*>(p)[j];
+        vq[u] = reinterpret_cast<const Pair<T>*>(q)[j];
+        vd[u] = dinv ? reinterpret_cast<const Pair<T>*>(dinv)[j] : Pair<T>(T(1));
+      }
+    }
+  };
+  load();
+  if (threadIdx.x == 0)
+    done = __hip_atomic_load(&st->done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  double a = 0.0;
+  for (int k = threadIdx.x; k < nb_spmv; k += kBlock)
+    a += st->partials[k];
+  a = wave_sum(a);
+  if ((threadIdx.x & 63) == 63)
+    lds[threadIdx.x >> 6] = a;
+  __syncthreads();
+  if (done)
+    return;
+  const int k = st->iter;
+  const T alpha
+      = static_cast<T>(st->rz[k & 1] / ((lds[0] + lds[1]) + (lds[2] + lds[3])));
+  if (blockIdx.x == 0 && threadIdx.x == 0)
+    st->kd = k + 1;
+  double s[2] = {0.0, 0.0};
+  auto one = [&](T& xi, T& ri, T pi, T qi, T di) -> T
+  {
+    xi += alpha * pi;
+    ri -= alpha * qi;
+    const T zi = di * ri;
+    s[0] += double(ri) * double(zi);
+    s[1] += double(ri) * double(ri);
+    return zi;
+  };
+  while (i < np)
+  {
+#pragma unroll
+    for (int u = 0; u < E; ++u)
+    {
+      const std::int64_t j = i + u * step;
+      if (j < np)
+      {
+        T x0 = vx[u].x, x1 = vx[u].y, r0 = vr[u].x, r1 = vr[u].y;
+        const T z0 = one(x0, r0, vp[u].x, vq[u].x, vd[u].x);
+        const T z1 = one(x1, r1, vp[u].y, vq[u].y, vd[u].y);
+        reinterpret_cast<Pair<T>*>(x)[j] = Pair<T>{x0, x1};
+        reinterpret_cast<Pair<T>*>(r)[j] = Pair<T>{r0, r1};
+        zp[2 * j] = Pair<T>{z0, vp[u].x};
+        zp[2 * j + 1] = Pair<T>{z1, vp[u].y};
+      }
+    }
+    i += E * step;
+    load();
+  }
+  if ((n & 1) && blockIdx.x == 0 && threadIdx.x == 0)
+  {
+    const std::int64_t j = n - 1;
+    T xi = x[j], ri = r[j];
+    const T pi = p[j], zi = one(xi, ri, pi, q[j], dinv ? dinv[j] : T(1));
+    x[j] = xi;
+    r[j] = ri;
+    zp[j] = Pair<T>{zi, pi};
+  }
+  store_block_sums<2>(s, {st->partials + kMaxPartials, st->partials + kMaxPartials + gridDim.x},
+                      blockIdx.x);
+}
+
+/// After the last iteration of a batch: the stop test that the next SpMV
+/// would make (one block), so that the host reads the state of every
+/// iteration done.
+__global__ void __launch_bounds__(kBlock) cg_finish_k(int nb_upd, CGState* st)
+{
+  if (block_flag(&st->done) || st->tested == st->kd)
+    return;
+  double sums[2];
+  const double* pr = st->partials + kMaxPartials;
+  sum_ranges<2>({pr, pr + nb_upd}, 0, nb_upd, sums); // ends with a barrier
+  if (threadIdx.x == 0)
+  {
+    const int k = st->kd;
+    st->rz[k & 1] = sums[0];
+    st->rr = sums[1];
+    st->iter = k;
+    st->tested = k;
+    if (sums[1] / st->rr0 < st->tol2 || k >= st->max_it)
+      st->done = 1;
+  }
+}
+
 /// Partial sums of (r.z, r.r) with z = dinv r, into the update partials
 /// (used after the residual has been replaced).
 template <typename T>
@@ -1466,6 +1823,12 @@ int partial_blocks(std::int64_t n)
 {
   std::int64_t b = (n + kBlock - 1) / kBlock;
   return static_cast<int>(std::clamp<std::int64_t>(b, 1, 1024));
+}
+
+/// Workgroups of cg_pair_update_k: two elements per thread up to 1024.
+int pair_blocks(std::int64_t n)
+{
+  return static_cast<int>(std::clamp<std::int64_t>((n + 2 * kBlock - 1) / (2 * kBlock), 1, 1024));
 }
 
 // ---------------------------------------------------------------------
@@ -1787,8 +2150,9 @@ struct CGWork
 {
   std::int64_t n = 0;
   T *r = nullptr, *p = nullptr, *q = nullptr, *dinv = nullptr;
+  Pair<T>* zp = nullptr; // pairs of the two-kernel iteration (null: three kernels)
   bool own = true; // false: the vectors live in caller-provided scratch
-  void alloc(std::int64_t nn, bool jacobi)
+  void alloc(std::int64_t nn, bool jacobi, bool pairs = false)
   {
     n = nn;
     r = static_cast<T*>(dmalloc(sizeof(T) * n));
@@ -1796,6 +2160,8 @@ struct CGWork
     q = static_cast<T*>(dmalloc(sizeof(T) * n));
     if (jacobi)
       dinv = static_cast<T*>(dmalloc(sizeof(T) * n));
+    if (pairs)
+      zp = static_cast<Pair<T>*>(dmalloc(sizeof(Pair<T>) * n));
   }
   ~CGWork()
   {
@@ -1805,6 +2171,7 @@ struct CGWork
     dfree(p);
     dfree(q);
     dfree(dinv);
+    dfree(zp);
   }
 };
 
@@ -1913,16 +2280,7 @@ int launch_cg_spmv(const dfx_csr& A, const T* p, T* q, CGState* st, bool sell)
   if (use_rows(A))
     return launch_rows<T>(A, p, q, 0, p, st->partials, &st->done);
   if (A.bs == 1 && lanes_per_row(A) == 1)
-  {
-    const int nb = std::max(
-        1, std::min({A.nblk,
-                     resident_blocks(reinterpret_cast<const void*>(spmv_stream_k<T>), kBlock, 0),
-                     kMaxPartials}));
-    spmv_stream_k<T><<<nb, kBlock, 0, s>>>(A.nblk, row_blocks(A), A.rbase, A.row_ptr, A.cols,
-                                           A.cols16, A.ncols, v, p, q, 0, p, st->partials,
-                                           &st->done);
-    return nb;
-  }
+    return launch_stream<T>(A, p, q, 0, p, st->partials, &st->done);
   if (A.bs == 1)
   {
     const int G = lanes_per_row(A);
@@ -1945,19 +2303,8 @@ int launch_cg_spmv(const dfx_csr& A, const T* p, T* q, CGState* st, bool sell)
     }
     return nb;
   }
-  if (A.nblk > 0 && A.lanes <= 1 && (A.bs == 2 || A.bs == 3))
-  {
-    const void* kern = A.bs == 3 ? reinterpret_cast<const void*>(bsr_stream_k<T, 3>)
-                                 : reinterpret_cast<const void*>(bsr_stream_k<T, 2>);
-    const int nb = std::max(1, std::min({A.nblk, resident_blocks(kern, kBlock, 0), kMaxPartials}));
-    if (A.bs == 3)
-      bsr_stream_k<T, 3><<<nb, kBlock, 0, s>>>(A.nblk, row_blocks(A), A.row_ptr, A.cols, v, p, q, 0, p,
-                                               st->partials, &st->done);
-    else
-      bsr_stream_k<T, 2><<<nb, kBlock, 0, s>>>(A.nblk, row_blocks(A), A.row_ptr, A.cols, v, p, q, 0, p,
-                                               st->partials, &st->done);
-    return nb;
-  }
+  if (block_stream(A))
+    return launch_stream<T>(A, p, q, 0, p, st->partials, &st->done);
   const int nb = partial_blocks(std::int64_t(A.nrows) * A.bs);
   if (A.bs == 3)
     cg_bsr_spmv_k<T, 3><<<nb, kBlock, 0, s>>>(A.nrows, A.row_ptr, A.cols, v, p, q, st);
@@ -1966,6 +2313,35 @@ int launch_cg_spmv(const dfx_csr& A, const T* p, T* q, CGState* st, bool sell)
   else
     throw Error(DFX_ERR_ARG, "block size must be 1..3");
   return nb;
+}
+
+/// Whether the two-kernel iteration serves A: its SpMV is the sliced-ELL copy
+/// (sell) or a stream kernel, and the vectors stay in the on-package cache
+/// (at most 2^20 rows). It moves the same bytes as the three kernels, saves a
+/// launch and the chain of latencies of a kernel, and gathers twice the bytes.
+/// Per iteration, SpMV + the rest: FP32 Q1 of 880,000 rows 30.1 + 7.9 us
+/// against 26.5 + 16.1; P3 of 389,000 rows 38.7 + 8.9 against 36.2 + 15.6;
+/// 3 x 3 blocks of 67,000 rows 28.7 + 6.5 against 24.9 + 13.1; but FP64 Q1 of
+/// 2.1 M rows 155 + 28.7 against 142 + 39.1 (its vectors come from HBM).
+inline bool pair_cg(const dfx_csr& A, bool sell)
+{
+  if (std::int64_t(A.nrows) * A.bs > (1 << 20))
+    return false;
+  return sell || block_stream(A)
+         || (A.bs == 1 && A.nblk > 0 && lanes_per_row(A) == 1 && !use_rows(A));
+}
+
+/// One iteration of the two-kernel CG; w.zp set.
+template <typename T>
+void pair_iteration(const dfx_csr& A, CGWork<T>& w, T* x, bool jacobi, CGState* st, bool sell)
+{
+  const int nbu = pair_blocks(w.n);
+  const DirArgs<T> dir{w.zp, w.p, nbu, st};
+  const int nbs = sell ? launch_sell<T, true>(A, nullptr, w.q, 0, nullptr, st->partials, nullptr, dir)
+                       : launch_stream<T, true>(A, nullptr, w.q, 0, nullptr, st->partials, nullptr,
+                                                dir);
+  cg_pair_update_k<T><<<nbu, kBlock, 0, stream()>>>(w.n, nbs, x, w.r, w.p, w.q,
+                                                    jacobi ? w.dinv : nullptr, w.zp, st);
 }
 
 /// A captured sequence of launches on a stream, replayed with
@@ -2033,7 +2409,7 @@ int cg_run(const dfx_csr& A, const T* b, T* x, int max_it, double rtol, bool jac
   init.tol2 = rtol * rtol;
   init.max_it = max_it;
   DFX_HIP(hipMemcpyAsync(st, &init, offsetof(CGState, partials), hipMemcpyHostToDevice, s));
-  cg_start_k<T><<<nbv, kBlock, 0, s>>>(n, b, w.q, jacobi ? w.dinv : nullptr, w.r, w.p, st);
+  cg_start_k<T><<<nbv, kBlock, 0, s>>>(n, b, w.q, jacobi ? w.dinv : nullptr, w.r, w.p, w.zp, st);
   cg_start_finish_k<<<1, kBlock, 0, s>>>(nbv, st);
   check_launch("cg_start");
   struct
@@ -2043,6 +2419,11 @@ int cg_run(const dfx_csr& A, const T* b, T* x, int max_it, double rtol, bool jac
   const int batch = std::max(1, check_every);
   auto iteration = [&]()
   {
+    if (w.zp)
+    {
+      pair_iteration<T>(A, w, x, jacobi, st, sell);
+      return;
+    }
     const int nbs = launch_cg_spmv<T>(A, w.p, w.q, st, sell);
     cg_update_k<T><<<nbv, kBlock, 0, s>>>(n, nbs, x, w.r, w.p, w.q, jacobi ? w.dinv : nullptr,
                                           st);
@@ -2050,9 +2431,20 @@ int cg_run(const dfx_csr& A, const T* b, T* x, int max_it, double rtol, bool jac
   };
   // a batch of iterations captured once and replayed (the kernels read
   // the iteration index from the state and do nothing once it stopped)
+  auto finish = [&]()
+  {
+    if (w.zp)
+      cg_finish_k<<<1, kBlock, 0, s>>>(pair_blocks(n), st);
+  };
   BatchGraph graph;
   if (use_graph)
-    graph.capture(s, [&]() { for (int j = 0; j < batch; ++j) iteration(); });
+    graph.capture(s,
+                  [&]()
+                  {
+                    for (int j = 0; j < batch; ++j)
+                      iteration();
+                    finish();
+                  });
   int k = 0;
   while (true)
   {
@@ -2062,8 +2454,11 @@ int cg_run(const dfx_csr& A, const T* b, T* x, int max_it, double rtol, bool jac
       k += batch;
     }
     else
+    {
       for (int j = 0; j < batch && k < max_it; ++j, ++k)
         iteration();
+      finish();
+    }
     check_launch("cg iteration");
     DFX_HIP(hipMemcpyAsync(&h, &st->iter, sizeof(h), hipMemcpyDeviceToHost, s));
     DFX_HIP(hipStreamSynchronize(s));
@@ -2139,16 +2534,16 @@ void cg_solve_t(const dfx_csr& A, const dfx_vec& b, dfx_vec& x,
                        const dfx_cg_opts& o, dfx_cg_result& res)
 {
   const std::int64_t n = std::int64_t(A.nrows) * A.bs;
-  CGWork<T> w;
-  w.alloc(n, o.jacobi != 0);
-  StateHolder sh;
   Reducer& red = reducer();
-  DFX_HIP(hipMemsetAsync(sh.st, 0, sizeof(CGState), stream()));
   // pattern work of the sliced-ELL copy (as the sparsity pattern, outside
   // the timed window); its values are copied inside
-  sell_layout<T>(A);
-  DFX_HIP(hipStreamSynchronize(stream()));
+  const bool sell = sell_layout<T>(A);
   const auto [rpt, nbc] = o.classic ? std::pair<int, int>{0, 0} : coop_shape<T>(A, o.max_it);
+  CGWork<T> w;
+  w.alloc(n, o.jacobi != 0, !rpt && pair_cg(A, sell));
+  StateHolder sh;
+  DFX_HIP(hipMemsetAsync(sh.st, 0, sizeof(CGState), stream()));
+  DFX_HIP(hipStreamSynchronize(stream()));
   T* p1 = nullptr;
   CoopSync* cs = nullptr;
   if (rpt)
@@ -2457,7 +2852,7 @@ dfx_status dfx_csr_create(const int64_t* row_ptr, const int32_t* cols, int32_t n
         h2d(A->row_ptr, rp32.data(), sizeof(std::int32_t) * (nrows + 1));
         const std::int32_t chunk
             = bs == 1 ? (dtype == DFX_F64 ? stream_entries<double>() : stream_entries<float>())
-                      : (dtype == DFX_F64 ? stream_chunk<double>() : stream_chunk<float>()) / bs;
+                      : (dtype == DFX_F64 ? bsr_chunk<double>(maxrow, bs) : bsr_chunk<float>(maxrow, bs)) / bs;
         if (bs == 1 || (bs <= 3 && maxrow <= chunk))
         {
           // row blocks of the stream SpMV: greedy, at most kBlock / bs rows
@@ -3125,14 +3520,17 @@ dfx_status dfx_mixed_solve(const dfx_csr* A64, const dfx_csr* A32, const dfx_vec
         materialize_zero(*A32);
         // pattern work of the FP32 sliced-ELL copy outside the timed window
         // (as for the FP64 solve); its values are copied inside
-        sell_layout<float>(*A32);
+        const bool layout = sell_layout<float>(*A32);
+        const bool restart = o->restart != 0;
         *res = dfx_mixed_result{};
         hipStream_t s = stream();
         const std::int64_t n = b->n;
         const double* bd = static_cast<const double*>(b->data);
         double* xd = static_cast<double*>(x->data);
+        // a restarted inner CG runs the two-kernel iteration; keeping the
+        // direction across refinements needs the separate direction kernel
         CGWork<float> w;
-        w.alloc(n, true);
+        w.alloc(n, true, restart && pair_cg(*A32, layout));
         StateHolder sh;
         CGState* st = sh.st;
         float* d32 = static_cast<float*>(dmalloc(sizeof(float) * n));
@@ -3171,7 +3569,6 @@ dfx_status dfx_mixed_solve(const dfx_csr* A64, const dfx_csr* A32, const dfx_vec
           return std::max(o->inner_rtol * o->inner_rtol, fin);
         };
         bool ok = rr <= tol2;
-        const bool restart = o->restart != 0;
         if (!ok)
         {
           inv_diag_k<float><<<static_cast<int>((n + kBlock - 1) / kBlock), kBlock, 0, s>>>(
@@ -3183,7 +3580,7 @@ dfx_status dfx_mixed_solve(const dfx_csr* A64, const dfx_csr* A32, const dfx_vec
           init.max_it = o->max_inner;
           DFX_HIP(hipMemcpyAsync(st, &init, offsetof(CGState, partials), hipMemcpyHostToDevice, s));
           // r = r32 - A32 * 0, p = z: reuse cg_start with y = 0
-          cg_start_k<float><<<nbv, kBlock, 0, s>>>(n, w.r, w.q, w.dinv, w.r, w.p, st);
+          cg_start_k<float><<<nbv, kBlock, 0, s>>>(n, w.r, w.q, w.dinv, w.r, w.p, w.zp, st);
           cg_start_finish_k<<<1, kBlock, 0, s>>>(nbv, st);
           cg_resume_k<<<1, 1, 0, s>>>(st, rr, inner_tol2(rr), -1);
           check_launch("mixed start");
@@ -3196,15 +3593,31 @@ dfx_status dfx_mixed_solve(const dfx_csr* A64, const dfx_csr* A32, const dfx_vec
         const int batch = std::max(1, o->check_every);
         auto iteration = [&]()
         {
+          if (w.zp)
+          {
+            pair_iteration<float>(*A32, w, d32, true, st, sell);
+            return;
+          }
           const int nbs = launch_cg_spmv<float>(*A32, w.p, w.q, st, sell);
           cg_update_k<float><<<nbv, kBlock, 0, s>>>(n, nbs, d32, w.r, w.p, w.q, w.dinv, st);
           cg_direction_k<float><<<nbv, kBlock, 0, s>>>(n, nbv, w.r, w.dinv, w.p, st);
         };
         // inner iterations replayed from a captured batch (the kernels read
         // the iteration index from the state)
+        auto finish = [&]()
+        {
+          if (w.zp)
+            cg_finish_k<<<1, kBlock, 0, s>>>(pair_blocks(n), st);
+        };
         BatchGraph graph;
         if (o->graph && !ok)
-          graph.capture(s, [&]() { for (int j = 0; j < batch; ++j) iteration(); });
+          graph.capture(s,
+                        [&]()
+                        {
+                          for (int j = 0; j < batch; ++j)
+                            iteration();
+                          finish();
+                        });
         while (!ok && k < o->max_inner)
         {
           if (graph.exec)
@@ -3213,8 +3626,11 @@ dfx_status dfx_mixed_solve(const dfx_csr* A64, const dfx_csr* A32, const dfx_vec
             k += batch;
           }
           else
+          {
             for (int j = 0; j < batch && k < o->max_inner; ++j, ++k)
               iteration();
+            finish();
+          }
           check_launch("mixed iteration");
           DFX_HIP(hipMemcpyAsync(&h, &st->iter, sizeof(h), hipMemcpyDeviceToHost, s));
           DFX_HIP(hipStreamSynchronize(s));
@@ -3242,7 +3658,7 @@ dfx_status dfx_mixed_solve(const dfx_csr* A64, const dfx_csr* A32, const dfx_vec
             // classic refinement: a new inner CG from d = 0 on the new r
             inner_base += h.iter;
             fill_k<float><<<nb, kBlock, 0, s>>>(w.q, n, 0.0f);
-            cg_start_k<float><<<nbv, kBlock, 0, s>>>(n, w.r, w.q, w.dinv, w.r, w.p, st);
+            cg_start_k<float><<<nbv, kBlock, 0, s>>>(n, w.r, w.q, w.dinv, w.r, w.p, w.zp, st);
             cg_start_finish_k<<<1, kBlock, 0, s>>>(nbv, st);
             cg_resume_k<<<1, 1, 0, s>>>(st, rr, inner_tol2(rr), -1);
             k = 0;
@@ -3265,7 +3681,7 @@ dfx_status dfx_mixed_solve(const dfx_csr* A64, const dfx_csr* A32, const dfx_vec
         if (!ok && o->fallback && o->max_inner > 0)
         {
           CGWork<double> w64;
-          w64.alloc(n, true);
+          w64.alloc(n, true, pair_cg(*A64, sell_layout<double>(*A64)));
           bool conv = false;
           double rr0f = 0, rrf = 0;
           const double rt = std::sqrt(tol2 / std::max(rr, 1e-300));
