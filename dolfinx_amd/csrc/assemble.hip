@@ -22,8 +22,9 @@ namespace
 {
 
 constexpr int kBlock = 256;
-// LDS slice of one elasticity row group (6 rows at most)
-constexpr std::size_t kTeamSlice = 16 * 1024;
+// LDS slices that end a group of elasticity rows: on the box meshes four edge
+// rows of 27 blocks of 72 bytes, four vertex rows of 65
+constexpr std::size_t kTeamEdge = 8 * 1024, kTeamVertex = 20 * 1024;
 
 /// Two values of T as one aligned vector access (double2 or float2).
 template <typename T>
@@ -3354,12 +3355,26 @@ std::vector<double> gradient_tensors(const TetBasis& B)
   return t;
 }
 
+/// The two barycentric gradients that the gradient of P2 node i combines,
+/// two bits per node: d phi_v = (4 l_v - 1) g_v at vertex v (twice v, the
+/// second unused), d phi_(kl) = 4 l_l g_k + 4 l_k g_l on edge (k, l).
+constexpr std::uint32_t p2_nodes(const int (&v)[10])
+{
+  std::uint32_t b = 0;
+  for (int i = 0; i < 10; ++i)
+    b |= static_cast<std::uint32_t>(v[i]) << (2 * i);
+  return b;
+}
+constexpr std::uint32_t kP2First = p2_nodes({0, 1, 2, 3, 2, 1, 1, 0, 0, 0});
+constexpr std::uint32_t kP2Second = p2_nodes({0, 1, 2, 3, 3, 3, 2, 3, 2, 1});
+
 // ---------------------------------------------------------------------
 // P2 vector elasticity, a = sigma(u):eps(v) with DG0 lambda, mu. Per cell
-// a record of 16 values: J^{-1} (9), 0, |det J| lambda, |det J| mu, 0...
+// a record of 16 values: the barycentric gradients g_0 .. g_3 (12; g_1 .. g_3
+// are the rows of J^{-1}), |det J| lambda, |det J| mu, their sum, and the BC
+// column mask (bit 3 j + component) in the low bits of the last.
 // Entry block (i, j) (3 x 3, row component c, column component d) with
-// P = J^{-T}-transformed reference gradient products,
-// P_cd = sum_ab Kinv[a][c] S_ab(i,j) Kinv[b][d]:
+// P_cd = int d_c phi_i d_d phi_j / |det J|:
 //   A_(i,c)(j,d) = |det J| mu (delta_cd tr P + P_dc) + |det J| lambda P_cd.
 // ---------------------------------------------------------------------
 
@@ -3393,20 +3408,16 @@ __global__ void __launch_bounds__(kBlock)
   T o[16];
 #pragma unroll
   for (int q = 0; q < 9; ++q)
-    o[q] = adj[q] / det;
-  o[9] = T(0);
-  o[10] = adet * coeffs[c * cstride];     // |det J| lambda
-  o[11] = adet * coeffs[c * cstride + 1]; // |det J| mu
+    o[3 + q] = adj[q] / det;
 #pragma unroll
-  for (int q = 12; q < 16; ++q)
-    o[q] = T(0);
-  T2* out = reinterpret_cast<T2*>(cd + 16 * c);
-#pragma unroll
-  for (int h = 0; h < 8; ++h)
-    out[h] = T2{o[2 * h], o[2 * h + 1]};
+  for (int q = 0; q < 3; ++q)
+    o[q] = -(o[3 + q] + o[6 + q] + o[9 + q]);
+  o[12] = adet * coeffs[c * cstride];     // |det J| lambda
+  o[13] = adet * coeffs[c * cstride + 1]; // |det J| mu
+  o[14] = o[12] + o[13];
+  std::uint32_t m = 0;
   if (mask)
   {
-    std::uint32_t m = 0;
     for (int j = 0; j < 10; ++j)
     {
       const std::int32_t node = dm[c * 10 + j];
@@ -3416,180 +3427,207 @@ __global__ void __launch_bounds__(kBlock)
     }
     mask[c] = m;
   }
+  if constexpr (sizeof(T) == 8)
+    o[15] = __longlong_as_double(static_cast<long long>(m));
+  else
+    o[15] = __uint_as_float(m);
+  T2* out = reinterpret_cast<T2*>(cd + 16 * c);
+#pragma unroll
+  for (int h = 0; h < 8; ++h)
+    out[h] = T2{o[2 * h], o[2 * h + 1]};
 }
 
-/// Row teams for the elasticity rows: a wavefront holds 6 teams of 10
-/// lanes; team t takes one block row, lane j the column node j of every
+/// The value of lane L of each row of 16 lanes, in every lane of the row
+/// (all of which are active).
+template <int L>
+__device__ inline std::uint32_t row_bcast(std::uint32_t v)
+{
+  return static_cast<std::uint32_t>(
+      __builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x150 + L, 0xf, 0xf, true));
+}
+template <int L>
+__device__ inline double row_bcast(double v)
+{
+  return __longlong_as_double(
+      __builtin_amdgcn_update_dpp(0ll, __double_as_longlong(v), 0x150 + L, 0xf, 0xf, true));
+}
+template <int L>
+__device__ inline float row_bcast(float v)
+{
+  return __uint_as_float(row_bcast<L>(__float_as_uint(v)));
+}
+
+/// Row teams for the elasticity rows: a wavefront holds 4 teams of 16
+/// lanes; team t takes one block row, lane j < 10 the column node j of every
 /// incidence of that row. The team walks the row's incidences in cell
 /// order, lane j adding the 3 x 3 block (i, j) into the row's LDS slice at
 /// the block of column slot j (the 10 slots of one incidence are distinct,
 /// so the additions need no atomics and every entry is summed in cell
-/// order). Rows come in groups of up to 6 with similar incidence counts
-/// (egrp: per group its first position in erow and its LDS slice length,
-/// then a terminating entry; erow: per row (row, slice offset, first
-/// incidence, incidences)); blocks are stored in LDS padded to 10 values.
-template <typename T, typename O>
+/// order). Rows come in groups of 4 with similar incidence counts, two int4
+/// per row: (row or -1, first incidence, incidences, CSR position) and
+/// (slice offset, row length, 0, 0).
+/// A P2 gradient combines two barycentric gradients, so the block's P is
+/// u_0 w_0^T + u_1 w_1^T with w_s = C_s0 v_0 + C_s1 v_1: 30 operations for
+/// J^{-T} S(i, j) J^{-1}. C_st = int a_is a_jt (a_i0 = 4 l_v - 1 at vertex v;
+/// a_is = 4 l_o, o the edge's other vertex) takes two values, so it is
+/// selected, not loaded. KIND 0: edge rows, the local node of every incidence
+/// is an edge's; 1: vertex rows (u_1 and half of P fall away); 2: rows of a
+/// dofmap that has a dof at vertices and edges. Lane j's v are at fixed places
+/// of the cell record; what the whole team needs (u, the Lame factors, the
+/// mask) is one value per lane, handed on by row broadcasts.
+/// Teams of 10 lanes that each loaded the whole record and S (176 bytes per
+/// lane and step) kept the data return of the vector memory path busy 97 % of
+/// the time; now the vector ALU is busy half of the time and the LDS adds 44 %,
+/// with 20 wavefronts per CU by LDS and registers. 48^3 cubes (25.8 M blocks,
+/// 1.85 GB): 0.90 ms for both kinds of rows against 1.27 ms. Resident
+/// wavefronts that prefetch the next group were slower (1.24 ms), so were
+/// plain stores (1.02 ms; non-temporal ones keep the records in the L2).
+template <typename T, typename O, int KIND>
 __global__ void __launch_bounds__(64)
-    elast_team_k(const int2* __restrict__ egrp, const int4* __restrict__ erow, const std::int32_t* __restrict__ inc,
+    elast_team_k(const int4* __restrict__ erow, const std::int32_t* __restrict__ inc,
                  const O* __restrict__ islots, const T* __restrict__ cd,
-                 const std::uint32_t* __restrict__ mask, const std::int8_t* __restrict__ bc,
-                 const std::int32_t* __restrict__ rp, const T* __restrict__ ref,
-                 T* __restrict__ vals, int accumulate)
+                 const std::int8_t* __restrict__ bc, T* __restrict__ vals, int accumulate)
 {
-  using T2 = vec2_t<T>;
   constexpr int K = 10;
   extern __shared__ unsigned char smem_raw[];
   T* acc = reinterpret_cast<T*>(smem_raw);
-  const int lane = threadIdx.x, team = lane / K, j = lane - K * team;
-  // A group's description as seen by this lane's team: the group's rows
-  // [q0, q1) and slice length, the team's (row, slice offset, first
-  // incidence, incidences), the row's CSR position and length, its
-  // Dirichlet components and its first 30 incidences (3 per lane).
-  struct Meta
+  const int lane = threadIdx.x, team = lane >> 4, j = lane & 15, jc = min(j, K - 1);
+  const std::int64_t at = 4 * std::int64_t(xcd_contiguous(blockIdx.x, gridDim.x)) + team;
+  const int4 ro = erow[2 * at];
+  const int2 rs = *reinterpret_cast<const int2*>(erow + 2 * at + 1);
+  const std::int32_t r = ro.x, p0 = ro.y, n = ro.z;
+  T* a = acc + rs.x;
+  std::int32_t c0 = 0, c1 = 0, c2 = 0, c3 = 0;
+  std::uint32_t rowbc = 0;
+  if (r >= 0)
   {
-    std::int32_t q0, q1, total;
-    bool has;
-    int4 ro;
-    std::int32_t rbase, rlen;
-    std::uint32_t rowbc;
-    std::int32_t pre0, pre1, pre2;
-  };
-  // first stage: the group's bounds and the team's row entry
-  auto meta_rows = [&](Meta& m, int g)
-  {
-    const int2 gb = egrp[g];
-    m.q0 = gb.x;
-    m.total = gb.y;
-    m.q1 = egrp[g + 1].x;
-    m.has = lane < 6 * K && m.q0 + team < m.q1;
-    m.ro = m.has ? erow[m.q0 + team] : make_int4(0, 0, 0, 0);
-  };
-  // second stage: the loads that need the row entry
-  auto meta_data = [&](Meta& m)
-  {
-    m.rbase = m.rlen = 0;
-    m.rowbc = 0;
-    m.pre0 = m.pre1 = m.pre2 = 0;
-    if (m.has)
+    if (n > 0)
     {
-      const std::int32_t r = m.ro.x, p0 = m.ro.z, n = m.ro.w;
-      m.rbase = rp[r];
-      m.rlen = rp[r + 1] - m.rbase;
-      if (bc)
-        for (int cc = 0; cc < 3; ++cc)
-          if (bc[3 * std::int64_t(r) + cc])
-            m.rowbc |= 1u << cc;
-      if (n > 0)
-      {
-        m.pre0 = inc[p0 + min(j, n - 1)];
-        m.pre1 = inc[p0 + min(K + j, n - 1)];
-        m.pre2 = inc[p0 + min(2 * K + j, n - 1)];
-      }
+      c0 = inc[p0];
+      c1 = inc[p0 + min(1, n - 1)];
+      c2 = inc[p0 + min(2, n - 1)];
+      c3 = inc[p0 + min(3, n - 1)];
     }
-  };
-  // the team adds its row's incidences into the row's slice
-  auto rows = [&](const Meta m)
+    if (bc)
+      for (int cc = 0; cc < 3; ++cc)
+        if (bc[3 * std::int64_t(r) + cc])
+          rowbc |= 1u << cc;
+  }
+  // the rows' slices follow one another
+  using T2 = vec2_t<T>;
+  std::int32_t total = 0;
+#pragma unroll
+  for (int t = 0; t < 4; ++t)
+    total = max(total, __builtin_amdgcn_readlane(rs.x + 9 * rs.y, 16 * t));
+  for (int t = 2 * lane; t < total; t += 128)
+    *reinterpret_cast<T2*>(acc + t) = T2{T(0), T(0)};
+  wave_sync();
+  if (r >= 0 && n > 0 && rowbc != 7u)
   {
-    const std::uint32_t rowbc = m.rowbc;
-    const std::int32_t p0 = m.ro.z, n = m.ro.w;
-    if (!m.has || rowbc == 7u || n == 0)
-      return;
-    T* a = acc + m.ro.y;
-    // the first 30 incidences are handed out by shuffles within the team
-    // (the team's lanes run the same steps)
-    const std::int32_t pre0 = m.pre0, pre1 = m.pre1, pre2 = m.pre2;
-    auto cik_at = [pre0, pre1, pre2, p0, inc, team](int st) -> std::int32_t
-    {
-      if (st < 3 * K)
-      {
-        const int h = st >= 2 * K ? 2 : (st >= K ? 1 : 0);
-        // (masks rather than a select chain, which the compiler turns into
-        // a table in scratch memory)
-        const std::int32_t m1 = -static_cast<std::int32_t>(h == 1);
-        const std::int32_t m2 = -static_cast<std::int32_t>(h == 2);
-        const std::int32_t v = (pre0 & ~(m1 | m2)) | (pre1 & m1) | (pre2 & m2);
-        return __shfl(v, team * K + (st - K * h), 64);
-      }
-      return inc[p0 + st];
-    };
-    // each step's cell record, mask, slot and reference block are loaded
-    // two steps ahead
+    // each step's values and slot are loaded two steps ahead, its cell two
+    // steps before that
     struct Stage
     {
-      T2 rec[6];
-      T2 tm[5];
-      std::uint32_t m;
+      T v0[3], v1[3], b;
+      std::uint32_t i;
       std::int32_t sl;
     };
     // 32-bit byte offsets from the (uniform) array bases; the launcher
     // checks that every offset fits
     const char* cdb = reinterpret_cast<const char*>(cd);
-    const char* refb = reinterpret_cast<const char*>(ref);
-    const char* maskb = reinterpret_cast<const char*>(mask);
     const char* slb = reinterpret_cast<const char*>(islots);
-    auto fetch = [&](Stage& sg, int st)
+    constexpr std::uint32_t B = sizeof(T), G = 3 * B; // bytes of a value, a gradient
+    const std::uint32_t ov0 = ((kP2First >> (2 * jc)) & 3u) * G,
+                        ov1 = ((kP2Second >> (2 * jc)) & 3u) * G;
+    // this lane's value for the team: lanes 0-2 u_0, 3-5 u_1, 6-8 lambda, mu
+    // and their sum, 9 the mask
+    const std::uint32_t bnodes = j < 3 ? kP2First : kP2Second, bstep = j < 6 ? G : 0u,
+                        bbase = (j < 6 ? j % 3 : j < 9 ? 6 + j : 15) * B;
+    auto fetch = [&](Stage& sg, std::int32_t cik, int st)
     {
-      const std::int32_t cik = cik_at(st);
-      const std::int32_t c = cik / K;
-      const int i = cik - c * K;
-      const T2* src = reinterpret_cast<const T2*>(
-          cdb + static_cast<std::uint32_t>(c) * std::uint32_t(16 * sizeof(T)));
-#pragma unroll
-      for (int h = 0; h < 6; ++h)
-        sg.rec[h] = src[h];
-      const T2* s2 = reinterpret_cast<const T2*>(
-          refb + static_cast<std::uint32_t>(i * K + j) * std::uint32_t(10 * sizeof(T)));
-#pragma unroll
-      for (int h = 0; h < 5; ++h)
-        sg.tm[h] = s2[h];
-      sg.m = mask ? *reinterpret_cast<const std::uint32_t*>(
-                 maskb + static_cast<std::uint32_t>(c) * std::uint32_t(sizeof(std::uint32_t)))
-                  : 0u;
+      const std::uint32_t c = static_cast<std::uint32_t>(cik) / K;
+      sg.i = static_cast<std::uint32_t>(cik) - c * K;
+      const std::uint32_t oc = c * (16 * B);
+      auto grad = [&](T (&g)[3], std::uint32_t o)
+      {
+        const T* q = reinterpret_cast<const T*>(cdb + (oc + o));
+        g[0] = q[0];
+        g[1] = q[1];
+        g[2] = q[2];
+      };
+      grad(sg.v0, ov0);
+      grad(sg.v1, ov1);
+      sg.b = *reinterpret_cast<const T*>(
+          cdb + (oc + bbase + ((bnodes >> (2 * sg.i)) & 3u) * bstep));
       sg.sl = *reinterpret_cast<const O*>(
-          slb + static_cast<std::uint32_t>((p0 + st) * K + j) * std::uint32_t(sizeof(O)));
+          slb + static_cast<std::uint32_t>((p0 + min(st, n - 1)) * K + jc)
+                    * std::uint32_t(sizeof(O)));
     };
+    // C of column j: c_eq where the two linear factors have the same
+    // coordinate, c_ne otherwise; none for the second of a vertex column
+    const std::uint32_t q0 = (kP2Second >> (2 * jc)) & 3u, q1 = (kP2First >> (2 * jc)) & 3u;
+    const bool mixed = KIND == 1 || j < 4;
+    const T ne0 = mixed ? T(-1) / T(30) : T(16) / T(120),
+            eq0 = mixed ? T(1) / T(10) : T(32) / T(120), ne1 = j < 4 ? T(0) : ne0,
+            eq1 = j < 4 ? T(0) : eq0;
     auto add = [&](const Stage& sg)
     {
-      T Ki[9], Tm[10];
-#pragma unroll
-      for (int h = 0; h < 4; ++h)
+      const T u0[3] = {row_bcast<0>(sg.b), row_bcast<1>(sg.b), row_bcast<2>(sg.b)};
+      const T lam = row_bcast<6>(sg.b), mu = row_bcast<7>(sg.b), sum = row_bcast<8>(sg.b);
+      std::uint32_t m;
+      if constexpr (sizeof(T) == 8)
+        m = row_bcast<9>(static_cast<std::uint32_t>(__double_as_longlong(sg.b)));
+      else
+        m = row_bcast<9>(__float_as_uint(sg.b));
+      const std::uint32_t o0 = (kP2Second >> (2 * sg.i)) & 3u;
+      T w0[3], P[9];
       {
-        Ki[2 * h] = sg.rec[h].x;
-        Ki[2 * h + 1] = sg.rec[h].y;
-      }
-      Ki[8] = sg.rec[4].x;
-      const T lam = sg.rec[5].x, mu = sg.rec[5].y;
-#pragma unroll
-      for (int h = 0; h < 5; ++h)
-      {
-        Tm[2 * h] = sg.tm[h].x;
-        Tm[2 * h + 1] = sg.tm[h].y;
-      }
-      // W = S Kinv, P = Kinv^T W
-      T W[9], P[9];
-#pragma unroll
-      for (int aa = 0; aa < 3; ++aa)
+        T C00 = o0 == q0 ? eq0 : ne0, C01 = o0 == q1 ? eq1 : ne1;
+        if (KIND == 2 && sg.i < 4)
+        {
+          C00 = o0 == q0 ? T(1) / T(10) : T(-1) / T(30);
+          C01 = j < 4 ? T(0) : o0 == q1 ? T(1) / T(10) : T(-1) / T(30);
+        }
 #pragma unroll
         for (int d = 0; d < 3; ++d)
-          W[aa * 3 + d] = Tm[aa * 3 + 0] * Ki[0 * 3 + d] + Tm[aa * 3 + 1] * Ki[1 * 3 + d]
-                          + Tm[aa * 3 + 2] * Ki[2 * 3 + d];
+          w0[d] = C00 * sg.v0[d] + C01 * sg.v1[d];
+      }
+      if constexpr (KIND == 1)
+      {
 #pragma unroll
-      for (int cc = 0; cc < 3; ++cc)
+        for (int cc = 0; cc < 3; ++cc)
+#pragma unroll
+          for (int d = 0; d < 3; ++d)
+            P[cc * 3 + d] = u0[cc] * w0[d];
+      }
+      else
+      {
+        const T u1[3] = {row_bcast<3>(sg.b), row_bcast<4>(sg.b), row_bcast<5>(sg.b)};
+        const std::uint32_t o1 = (kP2First >> (2 * sg.i)) & 3u;
+        T C10 = o1 == q0 ? eq0 : ne0, C11 = o1 == q1 ? eq1 : ne1;
+        if (KIND == 2 && sg.i < 4)
+          C10 = C11 = T(0);
+        T w1[3];
 #pragma unroll
         for (int d = 0; d < 3; ++d)
-          P[cc * 3 + d] = Ki[0 * 3 + cc] * W[0 * 3 + d] + Ki[1 * 3 + cc] * W[1 * 3 + d]
-                          + Ki[2 * 3 + cc] * W[2 * 3 + d];
-      const T tr = P[0] + P[4] + P[8];
+          w1[d] = C10 * sg.v0[d] + C11 * sg.v1[d];
+#pragma unroll
+        for (int cc = 0; cc < 3; ++cc)
+#pragma unroll
+          for (int d = 0; d < 3; ++d)
+            P[cc * 3 + d] = u0[cc] * w0[d] + u1[cc] * w1[d];
+      }
+      const T mt = mu * (P[0] + P[4] + P[8]);
       T out[9];
 #pragma unroll
       for (int cc = 0; cc < 3; ++cc)
 #pragma unroll
         for (int d = 0; d < 3; ++d)
-          out[cc * 3 + d] = cc == d ? mu * (tr + P[cc * 4]) + lam * P[cc * 4]
+          out[cc * 3 + d] = cc == d ? sum * P[cc * 4] + mt
                                     : mu * P[d * 3 + cc] + lam * P[cc * 3 + d];
       // Dirichlet components of the row and of column node j add nothing
       // (rare: branched around)
-      const std::uint32_t colb = (sg.m >> (3 * j)) & 7u;
+      const std::uint32_t colb = (m >> (3 * jc)) & 7u;
       if (rowbc | colb)
       {
 #pragma unroll
@@ -3599,64 +3637,60 @@ __global__ void __launch_bounds__(64)
             if (((rowbc >> cc) | (colb >> d)) & 1u)
               out[cc * 3 + d] = T(0);
       }
-      T2* blk = reinterpret_cast<T2*>(a + K * sg.sl);
-#pragma unroll
-      for (int h = 0; h < 4; ++h)
+      if (j < K)
       {
-        T2 w = blk[h];
-        w.x += out[2 * h];
-        w.y += out[2 * h + 1];
-        blk[h] = w;
+        T* blk = a + 9 * sg.sl;
+        T o[9];
+#pragma unroll
+        for (int h = 0; h < 9; ++h)
+          o[h] = blk[h];
+#pragma unroll
+        for (int h = 0; h < 9; ++h)
+          blk[h] = o[h] + out[h];
       }
-      a[K * sg.sl + 8] += out[8];
     };
-    Stage s0, s1, s2;
-    fetch(s0, 0);
-    fetch(s1, min(1, n - 1));
-    for (int st = 0; st < n; st += 3)
+    Stage s0, s1;
+    fetch(s0, c0, 0);
+    fetch(s1, c1, 1);
+    for (int st = 0; st < n; st += 2)
     {
-      fetch(s2, min(st + 2, n - 1));
       add(s0);
+      fetch(s0, c2, st + 2);
+      c2 = inc[p0 + min(st + 4, n - 1)];
       if (st + 1 >= n)
         break;
-      fetch(s0, min(st + 3, n - 1));
       add(s1);
-      if (st + 2 >= n)
-        break;
-      fetch(s1, min(st + 4, n - 1));
-      add(s2);
+      fetch(s1, c3, st + 3);
+      c3 = inc[p0 + min(st + 5, n - 1)];
     }
-  };
+  }
+  wave_sync();
   // the group's rows are stored one at a time by the whole wavefront (row
-  // t's position, length and slice offset come from lane K t)
-  auto store = [&](const Meta m)
+  // t's position, length and slice offset come from lane 16 t)
+  for (int t = 0; t < 4; ++t)
   {
-    for (std::int32_t t = 0; t < m.q1 - m.q0; ++t)
+    if (__builtin_amdgcn_readlane(r, 16 * t) < 0)
+      continue;
+    const std::int32_t n9 = 9 * __builtin_amdgcn_readlane(rs.y, 16 * t);
+    const T* src = acc + __builtin_amdgcn_readlane(rs.x, 16 * t);
+    T* dst = vals + std::int64_t(__builtin_amdgcn_readlane(ro.w, 16 * t)) * 9;
+    for (std::int32_t e = lane; e < n9; e += 256)
     {
-      const std::int32_t base = __builtin_amdgcn_readlane(m.rbase, K * t);
-      const std::int32_t n9 = 9 * __builtin_amdgcn_readlane(m.rlen, K * t);
-      const T* src = acc + __builtin_amdgcn_readlane(m.ro.y, K * t);
-      T* dst = vals + std::int64_t(base) * 9;
-      for (int e = lane; e < n9; e += 64)
-      {
-        const int blk = e / 9;
-        const T v = src[blk * K + (e - 9 * blk)];
-        if (accumulate)
-          dst[e] += v;
-        else
-          dst[e] = v;
-      }
+      T v[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        v[u] = src[min(e + 64 * u, n9 - 1)];
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (e + 64 * u < n9)
+        {
+          if (accumulate)
+            dst[e + 64 * u] += v[u];
+          else
+            __builtin_nontemporal_store(v[u], dst + e + 64 * u);
+        }
     }
-  };
-  Meta cur;
-  meta_rows(cur, xcd_contiguous(blockIdx.x, gridDim.x));
-  for (int t = lane; t < cur.total; t += 64)
-    acc[t] = T(0);
-  meta_data(cur);
-  __syncthreads();
-  rows(cur);
-  __syncthreads();
-  store(cur);
+  }
 }
 
 /// Lifting of the P2 elasticity form, b[(r, c)] -= alpha sum over the
@@ -3705,8 +3739,8 @@ __global__ void __launch_bounds__(kBlock)
       T Ki[9];
 #pragma unroll
       for (int q = 0; q < 9; ++q)
-        Ki[q] = rec[q];
-      const T lam = rec[10], mu = rec[11];
+        Ki[q] = rec[3 + q];
+      const T lam = rec[12], mu = rec[13];
       for (int j = 0; j < K; ++j)
       {
         const std::uint32_t colb = (m >> (3 * j)) & 7u;
@@ -3747,14 +3781,11 @@ __global__ void __launch_bounds__(kBlock)
     b[t] = static_cast<T>(double(b[t]) - alpha * s);
 }
 
-/// Element vectors of the tetrahedral source forms with constant data,
-/// one thread per cell, stored corner-major (be[(i BS + comp) nc + c]):
-/// P2 body force b_(i,c) = |det J| w_i f_c; P3 source b_i = |det J| w_i f
-/// (w_i = int phi_i over the reference cell).
-template <typename T, int K, int BS>
+/// |det J| of every cell (tetrahedral source forms with constant data).
+template <typename T>
 __global__ void __launch_bounds__(kBlock)
-    cell_const_source_k(std::int32_t nc, const T* __restrict__ x, const std::int32_t* __restrict__ xdm,
-                        const T* __restrict__ w, T f0, T f1, T f2, T* __restrict__ be)
+    cell_measure_k(std::int32_t nc, const T* __restrict__ x, const std::int32_t* __restrict__ xdm,
+                   T* __restrict__ out)
 {
   const std::int64_t c = blockIdx.x * std::int64_t(kBlock) + threadIdx.x;
   if (c >= nc)
@@ -3774,13 +3805,50 @@ __global__ void __launch_bounds__(kBlock)
   }
   const T det = adjugate(J, adj);
   const T adet = det < T(0) ? -det : det;
-  const T f[3] = {f0, f1, f2};
-  for (int i = 0; i < K; ++i)
+  out[c] = adet;
+}
+
+/// Tetrahedral source forms with constant data, P2 body force
+/// b_(i,c) = |det J| w_i f_c and P3 source b_i = |det J| w_i f (w_i = int
+/// phi_i over the reference cell): the row adds f_c times the sum over its
+/// incidences, in cell order, of |det J| w_i. One thread per row reads its
+/// incidences and the cells' measures (they stay in the L2); element vectors
+/// stored by a cell pass and gathered per row and component took 142 us for
+/// P2 on 48^3 cubes (660,000 cells, 2.7 M dofs), this 40 us.
+template <typename T, int K, int BS>
+__global__ void __launch_bounds__(kBlock)
+    row_const_source_k(std::int32_t nplan, const std::int32_t* __restrict__ inc_off,
+                       const std::int32_t* __restrict__ inc, const T* __restrict__ measure,
+                       const T* __restrict__ w, T f0, T f1, T f2, T* __restrict__ b)
+{
+  __shared__ T sw[K];
+  if (threadIdx.x < K)
+    sw[threadIdx.x] = w[threadIdx.x];
+  __syncthreads();
+  const std::int32_t r = xcd_contiguous(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
+  if (r >= nplan)
+    return;
+  const std::int32_t p0 = inc_off[r], p1 = inc_off[r + 1];
+  T s = 0;
+  for (std::int32_t pb = p0; pb < p1; pb += 8)
   {
+    std::int32_t q[8];
+    T m[8];
 #pragma unroll
-    for (int b = 0; b < BS; ++b)
-      be[std::int64_t(i * BS + b) * nc + c] = adet * w[i] * f[b];
+    for (int u = 0; u < 8; ++u)
+      q[u] = inc[min(pb + u, p1 - 1)];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      m[u] = measure[q[u] / K];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (pb + u < p1)
+        s += m[u] * sw[q[u] % K];
   }
+  const T f[3] = {f0, f1, f2};
+#pragma unroll
+  for (int c = 0; c < BS; ++c)
+    b[std::int64_t(r) * BS + c] += f[c] * s;
 }
 
 
@@ -3962,77 +4030,85 @@ void launch_lanes(dfx_form& f, dfx_csr& A, const dfx_bc* bc)
         A.zeroed ? 0 : 1);
 }
 
-/// Row groups of the elasticity team kernel. Rows are ordered by their
-/// incidence count (longest first) inside chunks of 4096 consecutive rows,
-/// so the 6 rows of a wavefront take similar numbers of steps while a
-/// chunk's cells stay together in the L2; a group is cut at 6 rows or when
-/// its padded LDS slice would exceed kTeamSlice. Groups are stored as
-/// (first position, slice length) pairs ended by (number of rows, 0), rows
-/// as (row, slice offset, first incidence, incidences).
+/// Row groups of the elasticity team kernel: the edge rows', the vertex rows'
+/// and those of rows that are both (none on a Lagrange dofmap), ending at
+/// team_end. Rows are ordered by their incidence count
+/// (longest first) inside chunks of 4096 consecutive rows, so the 4 rows of
+/// a wavefront take similar numbers of steps while a chunk's cells stay
+/// together in the L2; a group is cut at 4 rows or when its LDS slice would
+/// exceed kTeamEdge or kTeamVertex, and filled with rows -1. team_lds: the
+/// values of LDS that the kinds' longest slices need.
 void ensure_teams(dfx_form& f, const dfx_csr& A, std::size_t tsize)
 {
-  const std::int64_t cap = static_cast<std::int64_t>(kTeamSlice / tsize);
-  if (f.team_grp && f.team_pattern == A.pattern_id && f.team_cap == cap)
+  const std::int64_t most = static_cast<std::int64_t>(16 * 1024 / tsize);
+  if (f.team_rows && f.team_pattern == A.pattern_id && f.team_cap == most)
     return;
-  dfree(f.team_grp);
-  f.team_grp = nullptr;
-  f.nteam = 0;
+  dfree(f.team_rows);
+  f.team_rows = nullptr;
+  for (std::int32_t& e : f.team_end)
+    e = 0;
   if (A.nrows == 0)
     return;
-  require(10 * std::int64_t(A.max_row) <= cap, "row too long for the LDS slice");
+  require(10 * std::int64_t(A.max_row) <= most, "row too long for the LDS slice");
   const std::int32_t nplan = f.max_dof + 1;
   std::vector<std::int32_t> off(nplan + 1), rp(A.nrows + 1);
+  std::vector<std::int32_t> inc(std::size_t(f.d.num_cells) * 10);
   d2h(off.data(), f.inc_off, sizeof(std::int32_t) * off.size());
   d2h(rp.data(), A.row_ptr, sizeof(std::int32_t) * rp.size());
+  d2h(inc.data(), f.inc, sizeof(std::int32_t) * inc.size());
   auto count = [&](std::int32_t r) { return r < nplan ? off[r + 1] - off[r] : 0; };
-  std::vector<std::int32_t> order(A.nrows);
+  std::vector<std::int32_t> order[3];
   for (std::int32_t r = 0; r < A.nrows; ++r)
-    order[r] = r;
-  std::sort(order.begin(), order.end(),
-            [&](std::int32_t x, std::int32_t y)
-            {
-              if ((x >> 12) != (y >> 12))
-                return x < y;
-              const std::int32_t cx = count(x), cy = count(y);
-              return cx != cy ? cx > cy : x < y;
-            });
-  std::vector<std::int32_t> grp{0, 0}, rows;
-  rows.reserve(4 * std::size_t(A.nrows));
-  std::int64_t slice = 0;
-  int members = 0;
-  for (std::int32_t q = 0; q < A.nrows; ++q)
   {
-    const std::int32_t r = order[q];
-    const std::int64_t len = 10 * std::int64_t(rp[r + 1] - rp[r]);
-    if (members == 6 || slice + len > cap)
-    {
-      grp.back() = static_cast<std::int32_t>(slice);
-      grp.push_back(q);
-      grp.push_back(0);
-      slice = 0;
-      members = 0;
-    }
-    rows.push_back(r);
-    rows.push_back(static_cast<std::int32_t>(slice));
-    rows.push_back(r < nplan ? off[r] : 0);
-    rows.push_back(count(r));
-    slice += len;
-    ++members;
+    int vertices = 0;
+    for (std::int32_t p = 0; p < count(r); ++p)
+      vertices += inc[off[r] + p] % 10 < 4;
+    order[vertices == 0 ? 0 : vertices == count(r) ? 1 : 2].push_back(r);
   }
-  grp.back() = static_cast<std::int32_t>(slice);
-  grp.push_back(A.nrows);
-  grp.push_back(0);
-  f.nteam = static_cast<std::int32_t>(grp.size() / 2) - 1;
-  // the row quads start at a multiple of 4 (16-byte aligned)
-  const std::size_t at = (grp.size() + 3) & ~std::size_t(3);
-  std::vector<std::int32_t> buf(at + rows.size(), 0);
-  std::copy(grp.begin(), grp.end(), buf.begin());
-  std::copy(rows.begin(), rows.end(), buf.begin() + at);
-  f.team_grp = static_cast<std::int32_t*>(dmalloc(sizeof(std::int32_t) * buf.size()));
-  h2d(f.team_grp, buf.data(), sizeof(std::int32_t) * buf.size());
-  f.team_rows_at = static_cast<std::int32_t>(at);
+  std::vector<std::int32_t> rows, group;
+  rows.reserve(9 * std::size_t(A.nrows));
+  for (int kind = 0; kind < 3; ++kind)
+  {
+    const std::int64_t cap
+        = static_cast<std::int64_t>((kind ? kTeamVertex : kTeamEdge) / tsize);
+    std::sort(order[kind].begin(), order[kind].end(),
+              [&](std::int32_t x, std::int32_t y)
+              {
+                if ((x >> 12) != (y >> 12))
+                  return x < y;
+                const std::int32_t cx = count(x), cy = count(y);
+                return cx != cy ? cx > cy : x < y;
+              });
+    std::int64_t slice = 0, longest = 0;
+    auto flush = [&]()
+    {
+      if (group.empty())
+        return;
+      while (group.size() < 32)
+        group.insert(group.end(), {-1, 0, 0, 0, 0, 0, 0, 0});
+      rows.insert(rows.end(), group.begin(), group.end());
+      longest = std::max(longest, slice);
+      group.clear();
+      slice = 0;
+    };
+    for (const std::int32_t r : order[kind])
+    {
+      const std::int32_t len = rp[r + 1] - rp[r];
+      if (group.size() == 32 || slice + 9 * std::int64_t(len) > cap)
+        flush();
+      group.insert(group.end(), {r, r < nplan ? off[r] : 0, count(r), rp[r],
+                                 static_cast<std::int32_t>(slice), len, 0, 0});
+      slice += 9 * std::int64_t(len);
+    }
+    flush();
+    // slices are cleared two values at a time
+    f.team_lds[kind] = static_cast<std::int32_t>((longest + 1) / 2 * 2);
+    f.team_end[kind] = static_cast<std::int32_t>(rows.size() / 32);
+  }
+  f.team_rows = static_cast<std::int32_t*>(dmalloc(sizeof(std::int32_t) * rows.size()));
+  h2d(f.team_rows, rows.data(), sizeof(std::int32_t) * rows.size());
   f.team_pattern = A.pattern_id;
-  f.team_cap = cap;
+  f.team_cap = most;
 }
 
 /// Row order of variant 16 (built once per pattern): rows sorted by their
@@ -4091,14 +4167,18 @@ void launch_elast(dfx_form& f, dfx_csr& A, const dfx_bc* bc)
               && std::int64_t(nc) * 100 * std::int64_t(sizeof(O)) <= 0xffffffffLL,
           "mesh too large for the elasticity row kernel (cell records above 4 GiB)");
   ensure_teams(f, A, sizeof(T));
-  if (f.nteam > 0)
-    elast_team_k<T, O><<<f.nteam, 64, kTeamSlice, stream()>>>(
-        reinterpret_cast<const int2*>(f.team_grp),
-        reinterpret_cast<const int4*>(f.team_grp + f.team_rows_at), f.inc,
-        static_cast<const O*>(f.islots),
-        static_cast<const T*>(f.cell_data), bc ? f.cell_mask : nullptr, bc ? bc->marker : nullptr,
-        A.row_ptr, static_cast<const T*>(f.ref_tensors), static_cast<T*>(A.values),
-        A.zeroed ? 0 : 1);
+  auto go = [&](auto kern, int kind)
+  {
+    const std::int32_t first = kind ? f.team_end[kind - 1] : 0, count = f.team_end[kind] - first;
+    if (count > 0)
+      kern<<<count, 64, sizeof(T) * f.team_lds[kind], stream()>>>(
+          reinterpret_cast<const int4*>(f.team_rows) + 8 * std::int64_t(first), f.inc,
+          static_cast<const O*>(f.islots), static_cast<const T*>(f.cell_data),
+          bc ? bc->marker : nullptr, static_cast<T*>(A.values), A.zeroed ? 0 : 1);
+  };
+  go(elast_team_k<T, O, 1>, 1);
+  go(elast_team_k<T, O, 0>, 0);
+  go(elast_team_k<T, O, 2>, 2);
   check_launch("elasticity assembly");
 }
 
@@ -4784,23 +4864,20 @@ void vector_rows(const dfx_form& f, T* b)
   const int nv = f.d.nodes_per_cell;
   T* be = static_cast<T*>(f.cell_vec);
   const std::int32_t np = f.max_dof + 1;
-  if (f.d.kernel == DFX_K_P2TET_ELAST_L)
+  if (f.d.kernel == DFX_K_P2TET_ELAST_L || f.d.kernel == DFX_K_P3TET_L)
   {
-    cell_const_source_k<T, 10, 3><<<blocks_for(nc), kBlock, 0, stream()>>>(
-        nc, static_cast<const T*>(f.x), f.x_dofmap, static_cast<const T*>(f.ref_tensors),
-        static_cast<T>(f.constants[0]), static_cast<T>(f.constants[1]),
-        static_cast<T>(f.constants[2]), be);
-    row_vector_k<T, 10, 3><<<blocks_for(std::int64_t(np) * 3), kBlock, 0, stream()>>>(
-        np, nc, f.inc_off, f.inc, be, b);
-    check_launch("assemble_vector");
-    return;
-  }
-  if (f.d.kernel == DFX_K_P3TET_L)
-  {
-    cell_const_source_k<T, 20, 1><<<blocks_for(nc), kBlock, 0, stream()>>>(
-        nc, static_cast<const T*>(f.x), f.x_dofmap, static_cast<const T*>(f.ref_tensors),
-        static_cast<T>(f.constants[0]), T(0), T(0), be);
-    row_vector_k<T, 20, 1><<<blocks_for(np), kBlock, 0, stream()>>>(np, nc, f.inc_off, f.inc, be, b);
+    cell_measure_k<T><<<blocks_for(nc), kBlock, 0, stream()>>>(nc, static_cast<const T*>(f.x),
+                                                               f.x_dofmap, be);
+    auto rows = [&](auto kern, double f1, double f2)
+    {
+      kern<<<blocks_for(np), kBlock, 0, stream()>>>(
+          np, f.inc_off, f.inc, be, static_cast<const T*>(f.ref_tensors),
+          static_cast<T>(f.constants[0]), static_cast<T>(f1), static_cast<T>(f2), b);
+    };
+    if (f.d.kernel == DFX_K_P2TET_ELAST_L)
+      rows(row_const_source_k<T, 10, 3>, f.constants[1], f.constants[2]);
+    else
+      rows(row_const_source_k<T, 20, 1>, 0.0, 0.0);
     check_launch("assemble_vector");
     return;
   }
@@ -5504,7 +5581,10 @@ dfx_status dfx_form_create(const dfx_form_desc* desc, dfx_form** out)
           }
           else
           {
-            f->cell_vec = dmalloc(ts * std::max<std::int64_t>(nc * k * d.bs, 1));
+            // element vectors, or the cells' measures (constant sources)
+            const bool measures
+                = d.kernel == DFX_K_P2TET_ELAST_L || d.kernel == DFX_K_P3TET_L;
+            f->cell_vec = dmalloc(ts * std::max<std::int64_t>(measures ? nc : nc * k * d.bs, 1));
             const std::vector<double> w = reference_tensors(d.kernel);
             if (!w.empty())
               f->ref_tensors = upload_as(w.data(), static_cast<std::int64_t>(w.size()), d.dtype);
@@ -5759,7 +5839,7 @@ dfx_status dfx_form_destroy(dfx_form* f)
     dfree(f->cell_vec);
     dfree(f->inc_row);
     dfree(f->gblk);
-    dfree(f->team_grp);
+    dfree(f->team_rows);
     dfree(f->trow);
     dfree(f->facets);
     dfree(f->finc_off);

@@ -405,13 +405,14 @@ struct dfx_form
   std::int32_t* trow = nullptr;
   std::int32_t ntrow = 0;
   std::uint64_t trow_pattern = 0;
-  // Elasticity row groups: nteam + 1 (first row position, slice length)
-  // pairs, then from team_rows_at the (row, LDS slice offset, first
-  // incidence, incidences) of all rows in group order; built for
-  // team_pattern with team_cap values of slice per group.
-  std::int32_t* team_grp = nullptr;
-  std::int32_t nteam = 0;
-  std::int32_t team_rows_at = 0;
+  // Elasticity row groups: 4 rows each of 8 values (row or -1, first
+  // incidence, incidences, CSR position, LDS slice offset, row length, 0,
+  // 0); groups of edge rows, vertex rows and rows that are both end at
+  // team_end and take team_lds values of LDS; built for team_pattern with
+  // slices of team_cap values at most.
+  std::int32_t* team_rows = nullptr;
+  std::int32_t team_end[3] = {0, 0, 0};
+  std::int32_t team_lds[3] = {0, 0, 0};
   std::int64_t team_cap = 0;
   std::uint64_t team_pattern = 0;
   // Facet integrals. Exterior: (cell, local facet) pairs, per row the

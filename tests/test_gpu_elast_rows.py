@@ -1,0 +1,74 @@
+"""P2 elasticity rows at the edges of their groups: vertex and edge rows, row
+counts that do not fill a group, long rows, single Dirichlet components, adding
+into a matrix; and the constant sources, against the oracle."""
+
+import numpy as np
+import pytest
+
+import oracle as O
+from dolfinx_amd import fem, la, mesh, problems
+
+from conftest import rel_err
+from test_mesh_create import bicone, box_input
+
+pytestmark = pytest.mark.gpu
+
+MESHES = {
+    "one": (np.array([[0, 1, 2, 3]]), np.array([[0, 0, 0], [1, 0, 0], [0.2, 1, 0], [0.1, 0.3, 1.]])),
+    "fan": bicone(24),                                  # 48 cells at a vertex
+    "box": box_input((3, 2, 1), O.TET, 4),
+    "slab": box_input((17, 9, 2), O.TET, 5),            # more rows than one sorting chunk
+}
+
+
+@pytest.mark.parametrize("dtype,tol", [(np.float64, 1e-12), (np.float32, 5e-6)])
+@pytest.mark.parametrize("name", list(MESHES))
+def test_rows(name, dtype, tol):
+    cells, x = MESHES[name]
+    om = O.Mesh.from_cells(O.TET, cells, x)
+    pm = mesh.create_mesh(mesh.CellType.tetrahedron, cells, x)
+    V = fem.functionspace(pm, ("Lagrange", 2, (3,)))
+    dm, nn = om.dofmap(2)
+    rng = np.random.default_rng(3)
+    co = np.stack(problems.lame_from_E(rng.uniform(0.5, 2.0, om.num_cells)), 1)
+    a = fem.form("p2_elasticity", V, co, None, dtype)
+    rp, cols = O.sparsity(dm, dm, nn)
+    # a fifth of the dofs, components of a node independently
+    bdofs = np.nonzero(rng.random(3 * nn) < 0.2)[0].astype(np.int32)
+    mark = np.zeros(3 * nn, np.int8)
+    mark[bdofs] = 1
+    for m, bcs in ((None, []), (mark, [fem.dirichletbc(V, bdofs)])):
+        ref = O.assemble_matrix(O.K_P2TET_ELAST_A, om.x, om.cells, dm, 3, co, None, m, m, rp, cols)
+        if m is not None:
+            O.set_diagonal(ref, bdofs, 3, 1.0, rp, cols)
+        A = fem.assemble_matrix(a, bcs)
+        assert rel_err(A.data, ref) <= tol
+        if m is None:
+            fem.assemble_matrix(a, [], 1.0, A)  # added to what is there
+            assert rel_err(A.data, 2 * ref) <= tol
+    f = [0.3, -0.7, 1.1]
+    b = fem.assemble_vector(fem.form("p2_body_force", V, None, f, dtype))
+    br = O.assemble_vector(O.K_P2TET_ELAST_L, om.x, om.cells, dm, 3, None, np.array(f), 3 * nn)
+    assert rel_err(b.array, br) <= tol
+    V3 = fem.functionspace(pm, ("Lagrange", 3))
+    dm3, nn3 = om.dofmap(3)
+    b3 = fem.assemble_vector(fem.form("p3_source", V3, None, [1.7], dtype))
+    br3 = O.assemble_vector(O.K_P3TET_L, om.x, om.cells, dm3, 1, None, np.array([1.7]), nn3)
+    assert rel_err(b3.array, br3) <= tol
+
+
+def test_rows_of_both_kinds():
+    """A dofmap that has one dof at a vertex of one cell and on an edge of
+    another (no Lagrange space gives it; the form takes any dofmap)."""
+    cells, x = MESHES["box"]
+    pm = mesh.create_mesh(mesh.CellType.tetrahedron, cells, x)
+    V = fem.functionspace(pm, ("Lagrange", 2, (3,)))
+    nn, dm = V.dofmap.index_map_size, V.dofmap.list
+    dm[1::2] = dm[1::2, ::-1]  # every other cell's nodes in reverse order
+    co = np.stack(problems.lame_from_E(np.ones(len(dm))), 1)
+    a = fem.form("p2_elasticity", V, co, None)
+    rp, cols = O.sparsity(dm, dm, nn)
+    A = fem.assemble_matrix(a, [], 1.0, la.MatrixCSR(rp, cols, bs=3))
+    ref = O.assemble_matrix(O.K_P2TET_ELAST_A, pm.geometry.x, pm.geometry.dofmap, dm, 3, co, None,
+                            None, None, rp, cols)
+    assert rel_err(A.data, ref) <= 1e-12
