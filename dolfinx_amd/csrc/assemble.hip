@@ -584,6 +584,22 @@ __global__ void __launch_bounds__(kBlock)
   b[d] = static_cast<T>(alpha * (gv - xv));
 }
 
+/// set_diagonal_k and bc_set_k (alpha = 1, no x0) of a system in one launch;
+/// every dof's diagonal entry is in the pattern.
+template <typename T>
+__global__ void __launch_bounds__(kBlock)
+    system_bc_k(std::int32_t n, const std::int32_t* dofs, int bs, const std::int32_t* diag,
+                T* vals, T value, const double* g, T* b)
+{
+  const std::int32_t t = blockIdx.x * kBlock + threadIdx.x;
+  if (t >= n)
+    return;
+  const std::int32_t d = dofs[t];
+  const int k = d % bs;
+  vals[(std::int64_t(diag[d / bs]) * bs + k) * bs + k] = value;
+  b[d] = static_cast<T>(g ? g[d] : 0.0);
+}
+
 template <typename T>
 __global__ void __launch_bounds__(kBlock) to_dtype_k(T* dst, const double* src, std::int64_t n)
 {
@@ -1569,6 +1585,19 @@ __global__ void __launch_bounds__(kBlock)
       vals[base + t] = acc[t];
 }
 
+/// Lanes per row (dof) of the lifting kernels: a lane takes every eighth
+/// incidence. With a thread per row a row beside the boundary walked up to 24
+/// cells one after another, each a chain of dependent loads, and the whole
+/// pass took that long (61 x 47 x 53 P1 FP32: 58 us for 160,000 rows).
+constexpr int kLiftLanes = 8;
+__device__ inline double lift_sum(double s)
+{
+#pragma unroll
+  for (int o = 1; o < kLiftLanes; o <<= 1)
+    s += __shfl_xor(s, o, 64);
+  return s;
+}
+
 /// Lifting b[r] -= alpha sum_{(c,i) at r} sum_{j in BC} A_ij (g_j - x0_j),
 /// one thread per row, over cells whose mask marks a BC column.
 template <typename T, int K, bool COMPACT = false>
@@ -1579,61 +1608,64 @@ __global__ void __launch_bounds__(kBlock)
                const T* __restrict__ ref, const double* __restrict__ g,
                const T* __restrict__ x0, double alpha, T* __restrict__ b)
 {
-  const std::int32_t r = blockIdx.x * kBlock + threadIdx.x;
-  if (r >= nplan)
-    return;
+  const std::int64_t t = blockIdx.x * std::int64_t(kBlock) + threadIdx.x;
+  const std::int32_t r = static_cast<std::int32_t>(t / kLiftLanes);
+  const int lane = static_cast<int>(t % kLiftLanes);
   double s = 0.0;
-  const std::int32_t p0 = inc_off[r], p1 = inc_off[r + 1];
-  // eight incidences at a time: their cells and masks loaded together
-  // (clamped positions), then the cells with a Dirichlet column in order
-  for (std::int32_t pb = p0; pb < p1; pb += 8)
+  const std::int32_t p0 = r < nplan ? inc_off[r] : 0, p1 = r < nplan ? inc_off[r + 1] : 0;
+  for (std::int32_t p = p0 + lane; p < p1; p += kLiftLanes)
   {
-    std::int32_t cq[8];
-    std::uint32_t mq[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u)
-      cq[u] = inc[min(pb + u, p1 - 1)];
-#pragma unroll
-    for (int u = 0; u < 8; ++u)
-      mq[u] = mask[cq[u] / K];
-    for (int u = 0; u < 8 && pb + u < p1; ++u)
+    const std::int32_t cik = inc[p];
+    const std::int32_t c = cik / K;
+    const std::uint32_t m = mask[c];
+    if (!m)
+      continue;
+    const int i = cik - c * K;
+    T G[7];
+    if constexpr (COMPACT)
     {
-      const std::uint32_t m = mq[u];
-      if (!m)
-        continue;
-      const std::int32_t cik = cq[u];
-      const std::int32_t c = cik / K;
-      const int i = cik - c * K;
-      T G[7];
-      if constexpr (COMPACT)
-      {
-        const T* rc = cd + 4 * std::int64_t(c);
-        G[0] = rc[0]; G[1] = rc[1]; G[2] = rc[2]; G[6] = rc[3];
-        G[3] = G[4] = G[5] = T(0);
-      }
-      else
-      {
-        const T* rc = cd + 8 * std::int64_t(c);
+      const T* rc = cd + 4 * std::int64_t(c);
+      G[0] = rc[0]; G[1] = rc[1]; G[2] = rc[2]; G[6] = rc[3];
+      G[3] = G[4] = G[5] = T(0);
+    }
+    else
+    {
+      const T* rc = cd + 8 * std::int64_t(c);
 #pragma unroll
-        for (int q = 0; q < 7; ++q)
-          G[q] = rc[q];
-      }
-      const T* Si = ref + i * K;
-      for (int j = 0; j < K; ++j)
+      for (int q = 0; q < 7; ++q)
+        G[q] = rc[q];
+    }
+    const T* Si = ref + i * K;
+    // four columns at a time: their dofs, then their data, together
+    for (int j0 = 0; j0 < K; j0 += 4)
+    {
+      const std::uint32_t mj = (m >> j0) & 15u;
+      if (!mj)
+        continue;
+      const int4 col = *reinterpret_cast<const int4*>(dm + std::int64_t(c) * K + j0);
+      const std::int32_t cj[4] = {col.x, col.y, col.z, col.w};
+      double d[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        d[q] = ((mj >> q) & 1u) && g ? g[cj[q]] : 0.0;
+      if (x0)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+          if ((mj >> q) & 1u)
+            d[q] -= double(x0[cj[q]]);
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
       {
-        if (!((m >> j) & 1u))
-          continue;
-        const T v = G[0] * Si[j] + G[1] * Si[K * K + j] + G[2] * Si[2 * K * K + j]
-                    + G[3] * Si[3 * K * K + j] + G[4] * Si[4 * K * K + j]
-                    + G[5] * Si[5 * K * K + j] + G[6] * Si[6 * K * K + j];
-        const std::int32_t col = dm[std::int64_t(c) * K + j];
-        const double gv = g ? g[col] : 0.0;
-        const double xv = x0 ? double(x0[col]) : 0.0;
-        s += double(v) * (gv - xv);
+        const T* Sj = Si + j0 + q;
+        const T v = G[0] * Sj[0] + G[1] * Sj[K * K] + G[2] * Sj[2 * K * K] + G[3] * Sj[3 * K * K]
+                    + G[4] * Sj[4 * K * K] + G[5] * Sj[5 * K * K] + G[6] * Sj[6 * K * K];
+        if ((mj >> q) & 1u)
+          s += double(v) * d[q];
       }
     }
   }
-  if (s != 0.0)
+  s = lift_sum(s);
+  if (lane == 0 && s != 0.0)
     b[r] = static_cast<T>(double(b[r]) - alpha * s);
 }
 
@@ -1813,6 +1845,173 @@ __global__ void __launch_bounds__(kBlock)
   else
     for (int t = threadIdx.x; t < len; t += kBlock)
       vals[base + t] = acc[t];
+}
+
+/// Plan of variant 18, one thread per row: the contributions to the row (four
+/// per incidence) sorted by slot and, inside a slot, by incidence. ipos gives
+/// each contribution its place, soff (row length + 1 values at rp[r] + r) the
+/// first place of each slot.
+template <typename O, typename P>
+__global__ void __launch_bounds__(kBlock)
+    p1_places_k(std::int32_t nrows, std::int32_t nplan, const std::int32_t* __restrict__ inc_off,
+                const O* __restrict__ islots, const std::int32_t* __restrict__ rp,
+                P* __restrict__ ipos, P* __restrict__ soff)
+{
+  const std::int32_t r = blockIdx.x * kBlock + threadIdx.x;
+  if (r >= nrows)
+    return;
+  const std::int32_t len = rp[r + 1] - rp[r];
+  P* start = soff + (std::int64_t(rp[r]) + r);
+  for (std::int32_t t = 0; t <= len; ++t)
+    start[t] = 0;
+  if (r >= nplan)
+    return;
+  const std::int64_t b = 4 * std::int64_t(inc_off[r]), e = 4 * std::int64_t(inc_off[r + 1]);
+  for (std::int64_t q = b; q < e; ++q)
+    ++start[islots[q] + 1];
+  for (std::int32_t t = 0; t < len; ++t)
+    start[t + 1] += start[t];
+  for (std::int64_t q = b; q < e; ++q)
+    ipos[q] = start[islots[q]]++;
+  for (std::int32_t t = len; t > 0; --t)
+    start[t] = start[t - 1];
+  start[0] = 0;
+}
+
+/// The P1 element matrix row i from the cell factors: the terms of
+/// element_entry that are not zero, in its order and (as the compiler fuses
+/// its first sum into the first product) with its rounding.
+template <typename T>
+__device__ inline void p1_row(const T (&g)[7], int i, T (&e)[4])
+{
+  const T s = T(1.0 / 6.0), d = T(1.0 / 3.0), m0 = T(1.0 / 60.0), m1 = T(1.0 / 120.0);
+  auto mass = [&](T k, T m) { return fma_t(g[6], m, k); };
+  const T k00 = mass(fma_t(
+                         g[5], d,
+                         fma_t(g[4], d,
+                                       fma_t(g[3], d,
+                                                     fma_t(g[2], s,
+                                                                   fma_t(g[0], s, g[1] * s))))),
+                     m0);
+  const T k01 = mass(fma_t(g[4], -s, fma_t(g[3], -s, g[0] * -s)), m1);
+  const T k02 = mass(fma_t(g[5], -s, fma_t(g[3], -s, g[1] * -s)), m1);
+  const T k03 = mass(fma_t(g[5], -s, fma_t(g[4], -s, g[2] * -s)), m1);
+  const T k11 = mass(g[0] * s, m0), k22 = mass(g[1] * s, m0), k33 = mass(g[2] * s, m0);
+  const T k12 = mass(g[3] * s, m1), k13 = mass(g[4] * s, m1), k23 = mass(g[5] * s, m1);
+  e[0] = i == 0 ? k00 : i == 1 ? k01 : i == 2 ? k02 : k03;
+  e[1] = i == 0 ? k01 : i == 1 ? k11 : i == 2 ? k12 : k13;
+  e[2] = i == 0 ? k02 : i == 1 ? k12 : i == 2 ? k22 : k23;
+  e[3] = i == 0 ? k03 : i == 1 ? k13 : i == 2 ? k23 : k33;
+}
+
+/// Variant 18 (P1): 16 lanes per row. First a lane per incidence: the four
+/// entries of its element row go to their places (p1_places_k) in the row's
+/// LDS buffer; then a lane per CSR entry sums its contributions, in cell
+/// order as the other variants do. A thread per row (variants 0-2, 4-6) walks
+/// up to 24 incidences one group after another, each a chain of dependent
+/// loads and LDS read-modify-writes: that chain was the whole time of a small
+/// mesh (9 x 8 x 7 cubes FP64: 18.7 us on six workgroups; here 8.9, cell pass
+/// and two launches included) and left 61 x 47 x 53 at 90 us (here 59; FP32 58
+/// and 38) for 120 MB.
+template <typename T, typename P>
+__global__ void __launch_bounds__(kBlock)
+    row_p1_k(std::int32_t nrows, std::int32_t nplan, const std::int32_t* __restrict__ inc_off,
+             const std::int32_t* __restrict__ inc, const P* __restrict__ ipos,
+             const P* __restrict__ soff, const T* __restrict__ cd,
+             const std::int8_t* __restrict__ bc, const std::int32_t* __restrict__ rp,
+             T* __restrict__ vals, int accumulate, std::int32_t places)
+{
+  extern __shared__ unsigned char smem_raw[];
+  const int team = threadIdx.x >> 4, lane = threadIdx.x & 15;
+  T* buf = reinterpret_cast<T*>(smem_raw) + team * places;
+  const std::int32_t r
+      = xcd_contiguous(blockIdx.x, gridDim.x) * (kBlock / 16) + team;
+  const bool live = r < nrows;
+  const std::int32_t rbase = live ? rp[r] : 0, rlen = live ? rp[r + 1] - rbase : 0;
+  const bool dirichlet = live && bc && bc[r];
+  std::int32_t p0 = 0, n = 0;
+  if (live && r < nplan && !dirichlet)
+  {
+    p0 = inc_off[r];
+    n = inc_off[r + 1] - p0;
+  }
+  // first place of this lane's slots (two rounds are loaded early)
+  const P* start = soff + (std::int64_t(rbase) + r);
+  std::int32_t a0 = 0, a1 = 0, b0 = 0, b1 = 0;
+  if (n > 0)
+  {
+    const std::int32_t s0 = min(lane, rlen - 1), s1 = min(lane + 16, rlen - 1);
+    a0 = start[s0];
+    a1 = start[s0 + 1];
+    b0 = start[s1];
+    b1 = start[s1 + 1];
+  }
+  struct alignas(4 * sizeof(P)) Places
+  {
+    P p[4];
+  };
+  const Places* ip = reinterpret_cast<const Places*>(ipos) + p0;
+  for (std::int32_t q = lane; q < n; q += 32)
+  {
+    // two incidences together: indices, then records
+    std::int32_t cik[2];
+    Places pl[2];
+    T g[2][7];
+    std::uint32_t m[2];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+    {
+      const std::int32_t qq = min(q + 16 * u, n - 1);
+      cik[u] = inc[p0 + qq];
+      pl[u] = ip[qq];
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+      load_factors<T>(cd, cik[u] >> 2, g[u], m[u]);
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+      if (q + 16 * u < n)
+      {
+        T e[4];
+        p1_row<T>(g[u], cik[u] & 3, e);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          buf[pl[u].p[j]] = (m[u] >> j) & 1u ? T(0) : e[j];
+      }
+  }
+  wave_sync();
+  for (std::int32_t sl = lane; sl < rlen; sl += 16)
+  {
+    T sum = T(0);
+    if (n > 0)
+    {
+      std::int32_t k, e;
+      if (sl < 32)
+      {
+        k = sl < 16 ? a0 : b0;
+        e = sl < 16 ? a1 : b1;
+      }
+      else
+      {
+        k = start[sl];
+        e = start[sl + 1];
+      }
+      for (; k + 3 < e; k += 4)
+      {
+        const T v0 = buf[k], v1 = buf[k + 1], v2 = buf[k + 2], v3 = buf[k + 3];
+        sum += v0;
+        sum += v1;
+        sum += v2;
+        sum += v3;
+      }
+      for (; k < e; ++k)
+        sum += buf[k];
+    }
+    if (accumulate)
+      vals[rbase + sl] += sum;
+    else
+      vals[rbase + sl] = sum;
+  }
 }
 
 /// Variant 16 (forms with reference tensors, K <= 32 nodes per cell): a
@@ -3145,7 +3344,7 @@ template <typename T, int K, int BS>
 __global__ void __launch_bounds__(kBlock)
     row_vector_k(std::int32_t nplan, std::int32_t nc, const std::int32_t* __restrict__ inc_off,
                  const std::int32_t* __restrict__ inc, const T* __restrict__ be,
-                 T* __restrict__ b)
+                 T* __restrict__ b, int store)
 {
   const std::int64_t t = blockIdx.x * std::int64_t(kBlock) + threadIdx.x;
   if (t >= std::int64_t(nplan) * BS)
@@ -3169,7 +3368,7 @@ __global__ void __launch_bounds__(kBlock)
       if (pb + u < p1)
         s += v[u];
   }
-  b[t] += s;
+  b[t] = store ? s : b[t] + s;
 }
 
 // ---------------------------------------------------------------------
@@ -3708,76 +3907,64 @@ __global__ void __launch_bounds__(kBlock)
                  const T* __restrict__ x0, double alpha, T* __restrict__ b)
 {
   constexpr int K = 10;
-  const std::int64_t t = blockIdx.x * std::int64_t(kBlock) + threadIdx.x;
-  if (t >= std::int64_t(nplan) * 3)
-    return;
+  const std::int64_t q = blockIdx.x * std::int64_t(kBlock) + threadIdx.x;
+  const std::int64_t t = q / kLiftLanes;
+  const int lane = static_cast<int>(q % kLiftLanes);
   const std::int32_t r = static_cast<std::int32_t>(t / 3);
   const int comp = static_cast<int>(t - 3 * std::int64_t(r));
   double s = 0.0;
-  const std::int32_t p0 = inc_off[r], p1 = inc_off[r + 1];
-  // eight incidences at a time: their cells and masks loaded together
-  // (clamped positions), then the cells with a Dirichlet column in order
-  for (std::int32_t pb = p0; pb < p1; pb += 8)
+  const std::int32_t p0 = r < nplan ? inc_off[r] : 0, p1 = r < nplan ? inc_off[r + 1] : 0;
+  for (std::int32_t p = p0 + lane; p < p1; p += kLiftLanes)
   {
-    std::int32_t cq[8];
-    std::uint32_t mq[8];
+    const std::int32_t cik = inc[p];
+    const std::int32_t c = cik / K;
+    const std::uint32_t m = mask[c];
+    if (!m)
+      continue;
+    const int i = cik - c * K;
+    const T* rec = cd + 16 * std::int64_t(c);
+    T Ki[9];
 #pragma unroll
-    for (int u = 0; u < 8; ++u)
-      cq[u] = inc[min(pb + u, p1 - 1)];
-#pragma unroll
-    for (int u = 0; u < 8; ++u)
-      mq[u] = mask[cq[u] / K];
-    for (int u = 0; u < 8 && pb + u < p1; ++u)
+    for (int q = 0; q < 9; ++q)
+      Ki[q] = rec[3 + q];
+    const T lam = rec[12], mu = rec[13];
+    for (int j = 0; j < K; ++j)
     {
-      const std::int32_t cik = cq[u];
-      const std::int32_t c = cik / K;
-      const std::uint32_t m = mq[u];
-      if (!m)
+      const std::uint32_t colb = (m >> (3 * j)) & 7u;
+      if (!colb)
         continue;
-      const int i = cik - c * K;
-      const T* rec = cd + 16 * std::int64_t(c);
-      T Ki[9];
+      const T* Tm = ref + (i * K + j) * 10;
+      T W[9], P[9];
 #pragma unroll
-      for (int q = 0; q < 9; ++q)
-        Ki[q] = rec[3 + q];
-      const T lam = rec[12], mu = rec[13];
-      for (int j = 0; j < K; ++j)
-      {
-        const std::uint32_t colb = (m >> (3 * j)) & 7u;
-        if (!colb)
-          continue;
-        const T* Tm = ref + (i * K + j) * 10;
-        T W[9], P[9];
-#pragma unroll
-        for (int aa = 0; aa < 3; ++aa)
-#pragma unroll
-          for (int d = 0; d < 3; ++d)
-            W[aa * 3 + d] = Tm[aa * 3 + 0] * Ki[0 * 3 + d] + Tm[aa * 3 + 1] * Ki[1 * 3 + d]
-                            + Tm[aa * 3 + 2] * Ki[2 * 3 + d];
-#pragma unroll
-        for (int cc = 0; cc < 3; ++cc)
-#pragma unroll
-          for (int d = 0; d < 3; ++d)
-            P[cc * 3 + d] = Ki[0 * 3 + cc] * W[0 * 3 + d] + Ki[1 * 3 + cc] * W[1 * 3 + d]
-                            + Ki[2 * 3 + cc] * W[2 * 3 + d];
-        const T tr = P[0] + P[4] + P[8];
-        const std::int64_t node = dm[std::int64_t(c) * K + j];
+      for (int aa = 0; aa < 3; ++aa)
 #pragma unroll
         for (int d = 0; d < 3; ++d)
-        {
-          if (!((colb >> d) & 1u))
-            continue;
-          const T v = comp == d ? mu * (tr + P[comp * 4]) + lam * P[comp * 4]
-                                : mu * P[d * 3 + comp] + lam * P[comp * 3 + d];
-          const std::int64_t col = 3 * node + d;
-          const double gv = g ? g[col] : 0.0;
-          const double xv = x0 ? double(x0[col]) : 0.0;
-          s += double(v) * (gv - xv);
-        }
+          W[aa * 3 + d] = Tm[aa * 3 + 0] * Ki[0 * 3 + d] + Tm[aa * 3 + 1] * Ki[1 * 3 + d]
+                          + Tm[aa * 3 + 2] * Ki[2 * 3 + d];
+#pragma unroll
+      for (int cc = 0; cc < 3; ++cc)
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+          P[cc * 3 + d] = Ki[0 * 3 + cc] * W[0 * 3 + d] + Ki[1 * 3 + cc] * W[1 * 3 + d]
+                          + Ki[2 * 3 + cc] * W[2 * 3 + d];
+      const T tr = P[0] + P[4] + P[8];
+      const std::int64_t node = dm[std::int64_t(c) * K + j];
+#pragma unroll
+      for (int d = 0; d < 3; ++d)
+      {
+        if (!((colb >> d) & 1u))
+          continue;
+        const T v = comp == d ? mu * (tr + P[comp * 4]) + lam * P[comp * 4]
+                              : mu * P[d * 3 + comp] + lam * P[comp * 3 + d];
+        const std::int64_t col = 3 * node + d;
+        const double gv = g ? g[col] : 0.0;
+        const double xv = x0 ? double(x0[col]) : 0.0;
+        s += double(v) * (gv - xv);
       }
     }
   }
-  if (s != 0.0)
+  s = lift_sum(s);
+  if (lane == 0 && s != 0.0)
     b[t] = static_cast<T>(double(b[t]) - alpha * s);
 }
 
@@ -3819,7 +4006,8 @@ template <typename T, int K, int BS>
 __global__ void __launch_bounds__(kBlock)
     row_const_source_k(std::int32_t nplan, const std::int32_t* __restrict__ inc_off,
                        const std::int32_t* __restrict__ inc, const T* __restrict__ measure,
-                       const T* __restrict__ w, T f0, T f1, T f2, T* __restrict__ b)
+                       const T* __restrict__ w, T f0, T f1, T f2, T* __restrict__ b,
+                       int store)
 {
   __shared__ T sw[K];
   if (threadIdx.x < K)
@@ -3848,7 +4036,10 @@ __global__ void __launch_bounds__(kBlock)
   const T f[3] = {f0, f1, f2};
 #pragma unroll
   for (int c = 0; c < BS; ++c)
-    b[std::int64_t(r) * BS + c] += f[c] * s;
+  {
+    T* o = b + std::int64_t(r) * BS + c;
+    *o = store ? f[c] * s : *o + f[c] * s;
+  }
 }
 
 
@@ -3964,6 +4155,7 @@ void ensure_plan(dfx_form& f, const dfx_csr& A)
 template <typename T>
 void launch_cell_factors(const dfx_form& f, const dfx_bc* bc, bool compact = false)
 {
+  f.cell_records = compact ? 2 : 1;
   // done by the system cell pass of this assembly
   if (f.cell_data_ready)
   {
@@ -4013,7 +4205,7 @@ int incidence_lanes(const dfx_form& f)
 /// 11 as 1 with eight incidences in flight; 12..14 fixed-width Q1 rows;
 /// 15 structured Q1 rows in registers stored through an LDS slice; 16 row
 /// teams forming the entries; 17 row teams gathering the element matrices.
-constexpr int kRowVariants = 18;
+constexpr int kRowVariants = 19;
 
 template <typename T, typename O, int K, int L>
 void launch_lanes(dfx_form& f, dfx_csr& A, const dfx_bc* bc)
@@ -4152,10 +4344,20 @@ void ensure_trow(dfx_form& f, const dfx_csr& A)
   f.trow_pattern = A.pattern_id;
 }
 
+/// LDS of a workgroup of nw wavefronts of variant 16 at K = 20 (the reference
+/// tensors, the slices, the teams' slots), and whether four fit in 64 KB.
+template <typename T>
+bool team_fits(const dfx_csr& A)
+{
+  const std::size_t slices = (std::size_t(4) * 3 * A.max_row + 3) & ~std::size_t(3);
+  return (7 * 400 + slices + 4 * 3 * 8) * sizeof(T) <= 64 * 1024;
+}
+
 template <typename T, typename O>
 void launch_elast(dfx_form& f, dfx_csr& A, const dfx_bc* bc)
 {
   const std::int32_t nc = f.d.num_cells;
+  f.cell_records = 1;
   if (nc > 0)
     elast_factors_k<T><<<blocks_for(nc), kBlock, 0, stream()>>>(
         nc, static_cast<const T*>(f.x), f.x_dofmap, f.dofmap, static_cast<const T*>(f.coeffs),
@@ -4180,6 +4382,61 @@ void launch_elast(dfx_form& f, dfx_csr& A, const dfx_bc* bc)
   go(elast_team_k<T, O, 0>, 0);
   go(elast_team_k<T, O, 2>, 2);
   check_launch("elasticity assembly");
+}
+
+/// Plan of variant 18 for A's pattern (built once); false when a row's buffer
+/// would not fit: 16 rows of 4 max_inc values in 64 KB of LDS.
+template <typename T>
+bool ensure_p1(dfx_form& f, const dfx_csr& A)
+{
+  if (f.d.kernel != DFX_K_P1TET_A || 16 * 4 * std::int64_t(f.max_inc) * sizeof(T) > 64 * 1024)
+    return false;
+  if (f.p1_places && f.p1_pattern == A.pattern_id)
+    return true;
+  dfree(f.p1_places);
+  f.p1_places = nullptr;
+  const std::int64_t ncon = 16 * std::int64_t(f.d.num_cells),
+                     noff = A.nnz + std::int64_t(A.nrows);
+  const int pb = 4 * f.max_inc <= 255 ? 1 : 2;
+  unsigned char* buf = static_cast<unsigned char*>(dmalloc(pb * (ncon + noff)));
+  auto go = [&](auto o, auto p)
+  {
+    using O = decltype(o);
+    using P = decltype(p);
+    if (A.nrows > 0)
+      p1_places_k<O, P><<<blocks_for(A.nrows), kBlock, 0, stream()>>>(
+          A.nrows, f.max_dof + 1, f.inc_off, static_cast<const O*>(f.islots), A.row_ptr,
+          reinterpret_cast<P*>(buf), reinterpret_cast<P*>(buf) + ncon);
+  };
+  if (f.islot_bytes == 1)
+    pb == 1 ? go(std::uint8_t{}, std::uint8_t{}) : go(std::uint8_t{}, std::uint16_t{});
+  else
+    pb == 1 ? go(std::uint16_t{}, std::uint8_t{}) : go(std::uint16_t{}, std::uint16_t{});
+  check_launch("P1 row places");
+  f.p1_places = buf;
+  f.p1_place_bytes = pb;
+  f.p1_pattern = A.pattern_id;
+  return true;
+}
+
+template <typename T>
+void launch_p1(dfx_form& f, dfx_csr& A, const dfx_bc* bc)
+{
+  require(ensure_p1<T>(f, A), "variant not available for this element");
+  launch_cell_factors<T>(f, bc);
+  const std::int64_t ncon = 16 * std::int64_t(f.d.num_cells);
+  auto go = [&](auto p)
+  {
+    using P = decltype(p);
+    const P* pos = static_cast<const P*>(f.p1_places);
+    if (A.nrows > 0)
+      row_p1_k<T, P><<<(A.nrows + 15) / 16, kBlock, sizeof(T) * 64 * f.max_inc, stream()>>>(
+          A.nrows, f.max_dof + 1, f.inc_off, f.inc, pos, pos + ncon,
+          static_cast<const T*>(f.cell_data), bc ? bc->marker : nullptr, A.row_ptr,
+          static_cast<T*>(A.values), A.zeroed ? 0 : 1, 4 * f.max_inc);
+  };
+  f.p1_place_bytes == 1 ? go(std::uint8_t{}) : go(std::uint16_t{});
+  check_launch("row_assemble");
 }
 
 /// Structured-box plan of a Q1 form (corner cells and slot positions);
@@ -4399,6 +4656,14 @@ template <typename T, typename O, int K>
 void launch_row_assemble(dfx_form& f, dfx_csr& A, const dfx_bc* bc)
 {
   const int variant = f.row_variant;
+  if (variant == 18)
+  {
+    if constexpr (K == 4)
+      launch_p1<T>(f, A, bc);
+    else
+      throw Error(DFX_ERR_ARG, "variant not available for this element");
+    return;
+  }
   if (variant == 15)
   {
     if constexpr (K == 8)
@@ -4615,10 +4880,32 @@ void launch_row_assemble(dfx_form& f, dfx_csr& A, const dfx_bc* bc)
   check_launch("row_assemble");
 }
 
+/// Variant of a form that neither set nor autotuned it, for A's pattern.
+/// Measured (us per matrix, FP64 unless noted): P1, 18 against 1: 8.9 and 18.7
+/// at 720 rows, 18.9 and 28.9 at 36,000, 59 and 90 at 160,000 (FP32 38 and
+/// 58). Q1 on a structured box, 15 against 1: 8.8 and 13.3 at 8^3 cells, 12.6
+/// and 21.8 at 40 x 41 x 42, 174 and 375 at 128^3. P3, 16 against 3: 20.5 and
+/// 12.0 at 4^3 cubes (2,200 rows), 39.0 and 44.4 at 12^3 (51,000), 196 and 288
+/// at 24^3 (FP32 122 and 310).
+template <typename T>
+void choose_variant(dfx_form& f, const dfx_csr& A)
+{
+  if (!f.default_variant || !row_path(f))
+    return;
+  ensure_plan(f, A);
+  if (f.d.kernel == DFX_K_P1TET_A)
+    f.row_variant = ensure_p1<T>(f, A) ? 18 : 1;
+  else if (f.d.kernel == DFX_K_Q1HEX_A)
+    f.row_variant = ensure_struct(f, A) ? 15 : 1;
+  else if (f.d.kernel == DFX_K_P3TET_A)
+    f.row_variant = A.nrows >= 20000 && team_fits<T>(A) ? 16 : 3;
+}
+
 template <typename T>
 void assemble_rows(dfx_form& f, dfx_csr& A, const dfx_bc* bc)
 {
   ensure_plan(f, A);
+  choose_variant<T>(f, A);
   const int K = f.d.dofs_per_cell;
   if (f.d.kernel == DFX_K_P2TET_ELAST_A)
   {
@@ -4655,22 +4942,27 @@ void lift_rows(dfx_form& f, const dfx_bc& bc, const T* x0, double alpha, T* b)
 {
   // axis-aligned Q1 boxes: the 4-value records (the masks are always
   // written here, a BC being given)
-  const bool compact = f.compact_records && f.d.dofs_per_cell == 8;
-  launch_cell_factors<T>(f, &bc, compact);
+  bool compact = f.compact_records && f.d.dofs_per_cell == 8;
+  // inside a system call the matrix assembly's records (same form data, same
+  // BC) are still there
+  if (f.keep_records && f.cell_records)
+    compact = f.cell_records == 2;
+  else
+    launch_cell_factors<T>(f, &bc, compact);
   const std::int32_t nplan = f.max_dof + 1;
   const T* cd = static_cast<const T*>(f.cell_data);
   const T* ref = static_cast<const T*>(f.ref_tensors);
   if (f.d.dofs_per_cell == 4)
-    row_lift_k<T, 4><<<blocks_for(nplan), kBlock, 0, stream()>>>(
+    row_lift_k<T, 4><<<blocks_for(std::int64_t(nplan) * kLiftLanes), kBlock, 0, stream()>>>(
         nplan, f.inc_off, f.inc, f.dofmap, cd, f.cell_mask, ref, bc.g, x0, alpha, b);
   else if (compact)
-    row_lift_k<T, 8, true><<<blocks_for(nplan), kBlock, 0, stream()>>>(
+    row_lift_k<T, 8, true><<<blocks_for(std::int64_t(nplan) * kLiftLanes), kBlock, 0, stream()>>>(
         nplan, f.inc_off, f.inc, f.dofmap, cd, f.cell_mask, ref, bc.g, x0, alpha, b);
   else if (f.d.dofs_per_cell == 8)
-    row_lift_k<T, 8><<<blocks_for(nplan), kBlock, 0, stream()>>>(
+    row_lift_k<T, 8><<<blocks_for(std::int64_t(nplan) * kLiftLanes), kBlock, 0, stream()>>>(
         nplan, f.inc_off, f.inc, f.dofmap, cd, f.cell_mask, ref, bc.g, x0, alpha, b);
   else
-    row_lift_k<T, 20><<<blocks_for(nplan), kBlock, 0, stream()>>>(
+    row_lift_k<T, 20><<<blocks_for(std::int64_t(nplan) * kLiftLanes), kBlock, 0, stream()>>>(
         nplan, f.inc_off, f.inc, f.dofmap, cd, f.cell_mask, ref, bc.g, x0, alpha, b);
   check_launch("row_lift");
 }
@@ -4681,13 +4973,13 @@ template <typename T>
 void elast_lift_rows(dfx_form& f, const dfx_bc& bc, const T* x0, double alpha, T* b)
 {
   const std::int32_t nc = f.d.num_cells;
-  if (nc > 0)
+  if (nc > 0 && !(f.keep_records && f.cell_records))
     elast_factors_k<T><<<blocks_for(nc), kBlock, 0, stream()>>>(
         nc, static_cast<const T*>(f.x), f.x_dofmap, f.dofmap, static_cast<const T*>(f.coeffs),
         f.d.cstride, bc.marker, static_cast<T*>(f.cell_data), f.cell_mask);
   const std::int32_t nplan = f.max_dof + 1;
   if (nplan > 0)
-    elast_lift_k<T><<<blocks_for(std::int64_t(nplan) * 3), kBlock, 0, stream()>>>(
+    elast_lift_k<T><<<blocks_for(std::int64_t(nplan) * 3 * kLiftLanes), kBlock, 0, stream()>>>(
         nplan, f.inc_off, f.inc, f.dofmap, static_cast<const T*>(f.cell_data), f.cell_mask,
         static_cast<const T*>(f.ref_tensors), bc.g, x0, alpha, b);
   check_launch("elasticity lifting");
@@ -4862,6 +5154,9 @@ void vector_rows(const dfx_form& f, T* b)
 {
   const std::int32_t nc = f.d.num_cells;
   const int nv = f.d.nodes_per_cell;
+  // b = instead of b += (a system call that starts from zero)
+  const int store = f.store_vec ? 1 : 0;
+  f.store_vec = false;
   T* be = static_cast<T*>(f.cell_vec);
   const std::int32_t np = f.max_dof + 1;
   if (f.d.kernel == DFX_K_P2TET_ELAST_L || f.d.kernel == DFX_K_P3TET_L)
@@ -4872,7 +5167,7 @@ void vector_rows(const dfx_form& f, T* b)
     {
       kern<<<blocks_for(np), kBlock, 0, stream()>>>(
           np, f.inc_off, f.inc, be, static_cast<const T*>(f.ref_tensors),
-          static_cast<T>(f.constants[0]), static_cast<T>(f1), static_cast<T>(f2), b);
+          static_cast<T>(f.constants[0]), static_cast<T>(f1), static_cast<T>(f2), b, store);
     };
     if (f.d.kernel == DFX_K_P2TET_ELAST_L)
       rows(row_const_source_k<T, 10, 3>, f.constants[1], f.constants[2]);
@@ -4894,10 +5189,10 @@ void vector_rows(const dfx_form& f, T* b)
   const std::int32_t nplan = f.max_dof + 1;
   if (nv == 4)
     row_vector_k<T, 4, 1><<<blocks_for(nplan), kBlock, 0, stream()>>>(nplan, nc, f.inc_off, f.inc,
-                                                                       be, b);
+                                                                       be, b, store);
   else
     row_vector_k<T, 8, 1><<<blocks_for(nplan), kBlock, 0, stream()>>>(nplan, nc, f.inc_off, f.inc,
-                                                                       be, b);
+                                                                       be, b, store);
   check_launch("assemble_vector");
 }
 
@@ -5565,6 +5860,7 @@ dfx_status dfx_form_create(const dfx_form_desc* desc, dfx_form** out)
           build_incidences(*f, d.dofmap);
           // thread-per-row slices do not fit LDS for wide elements
           f->row_variant = k > 8 ? 3 : 1;
+          f->default_variant = true;
           const std::size_t ts = dtype_size(d.dtype);
           if (is_facet_kernel(d.kernel) || is_interior_kernel(d.kernel))
           {
@@ -5840,6 +6136,7 @@ dfx_status dfx_form_destroy(dfx_form* f)
     dfree(f->inc_row);
     dfree(f->gblk);
     dfree(f->team_rows);
+    dfree(f->p1_places);
     dfree(f->trow);
     dfree(f->facets);
     dfree(f->finc_off);
@@ -6128,6 +6425,7 @@ dfx_status dfx_form_autotune(dfx_form* a, dfx_csr* A, const dfx_bc* bc, int32_t*
         require(!is_facet_matrix_kernel(a->d.kernel) && !is_interior_kernel(a->d.kernel),
                 "facet forms have no kernel variants");
         dfx_form& f = *a;
+        f.default_variant = false;
         int best = f.row_variant;
         float bms = -1;
         // the elasticity form has one row kernel
@@ -6209,6 +6507,12 @@ dfx_status dfx_form_autotune(dfx_form* a, dfx_csr* A, const dfx_bc* bc, int32_t*
           f.struct_pattern = 0;
           f.struct_ok = -1;
         }
+        if (best != 18)
+        {
+          dfree(f.p1_places);
+          f.p1_places = nullptr;
+          f.p1_pattern = 0;
+        }
         if (best != 16 && best != 17)
         {
           dfree(f.trow);
@@ -6234,6 +6538,7 @@ dfx_status dfx_form_set_variant(dfx_form* a, int32_t variant)
         require(a, "null form");
         require(variant >= 0 && variant < kRowVariants, "variant out of range");
         a->row_variant = variant;
+        a->default_variant = false;
       });
 }
 
@@ -6640,12 +6945,22 @@ dfx_status dfx_assemble_system(dfx_csr* A, const dfx_form* a, const dfx_bc* bc, 
         {
           dfx_form& a;
           dfx_form& L;
+          ReadyGuard(dfx_form& a_, dfx_form& L_) : a(a_), L(L_)
+          {
+            a.keep_records = true;
+            a.cell_records = 0;
+          }
           ~ReadyGuard()
           {
             a.cell_data_ready = false;
+            a.keep_records = false;
             L.cell_vec_ready = false;
+            L.store_vec = false;
           }
         } rg{af, Lf};
+        if (A->dtype == a->d.dtype && A->bs == a->d.bs && a->max_dof < A->nrows
+            && a->max_dof < A->ncols)
+          a->d.dtype == DFX_F64 ? choose_variant<double>(af, *A) : choose_variant<float>(af, *A);
         const bool shared = system_cell_pass(af, Lf, bc);
         // the vector assembly reads only L's data and writes only b: on
         // large meshes it runs on the second stream while the matrix is
@@ -6683,22 +6998,48 @@ dfx_status dfx_assemble_system(dfx_csr* A, const dfx_form* a, const dfx_bc* bc, 
         }
         {
           StreamScope on(fork ? c.aux : c.stream);
-          if (zero_b)
+          // a source form that reaches every entry stores them; others add
+          // to zeros
+          const int k = L->d.kernel;
+          if (zero_b && b->dtype == L->d.dtype && !L->host_kernel && !L->host_facets
+              && (k == DFX_K_P1TET_L || k == DFX_K_Q1HEX_L || k == DFX_K_P2TET_ELAST_L
+                  || k == DFX_K_P3TET_L)
+              && std::int64_t(L->max_dof + 1) * L->d.bs == b->n)
+            Lf.store_vec = true;
+          else if (zero_b)
             ok(dfx_vec_set(b, 0.0));
           ok(dfx_assemble_vector(b, L));
         }
         if (fork)
           DFX_HIP(hipEventRecord(c.join, c.aux));
         ok(dfx_assemble_matrix(A, a, bc));
-        if (bc)
+        // the diagonal and the entries of b in one launch once the pattern is
+        // known to hold the diagonal
+        const bool both = bc && bc->diag_checked == A->pattern_id && bc->ndofs > 0
+                          && bc->n_total == A->nrows * A->bs && bc->n_total == b->n
+                          && b->dtype == A->dtype;
+        if (bc && !both)
           ok(dfx_set_diagonal(A, bc, diag));
         if (fork)
           jg.join();
         if (bc)
-        {
           ok(dfx_apply_lifting(b, a, bc, nullptr, 1.0));
-          ok(dfx_bc_set(b, bc, nullptr, 1.0));
+        if (both)
+        {
+          materialize_zero(*A);
+          if (A->dtype == DFX_F64)
+            system_bc_k<double><<<blocks_for(bc->ndofs), kBlock, 0, stream()>>>(
+                bc->ndofs, bc->dofs, A->bs, A->diag, static_cast<double*>(A->values), diag, bc->g,
+                static_cast<double*>(b->data));
+          else
+            system_bc_k<float><<<blocks_for(bc->ndofs), kBlock, 0, stream()>>>(
+                bc->ndofs, bc->dofs, A->bs, A->diag, static_cast<float*>(A->values),
+                static_cast<float>(diag), bc->g, static_cast<float*>(b->data));
+          check_launch("system bc");
+          A->zeroed = false;
         }
+        else if (bc)
+          ok(dfx_bc_set(b, bc, nullptr, 1.0));
       });
 }
 

@@ -101,6 +101,10 @@ __device__ inline XcdRange xcd_range(int n)
   return {lo + (b >> 3), hi, (nb - x + 7) >> 3};
 }
 
+/// Fused multiply-add in T (__builtin_fma alone works in double).
+__device__ inline double fma_t(double a, double b, double c) { return __builtin_fma(a, b, c); }
+__device__ inline float fma_t(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+
 /// One step of wave_sum: the value of the lane that DPP control C names
 /// (zero where there is none), added.
 template <int C, int ROWS>
@@ -317,6 +321,12 @@ struct dfx_form
   std::uint64_t same_geometry_as = 0;
   mutable bool cell_data_ready = false;
   mutable bool cell_vec_ready = false;
+  // Inside a system call (keep_records): the layout of the cell records that
+  // its matrix assembly left (1 full, 2 compact, 0 none), which the lifting
+  // then reads; and whether the vector assembly stores instead of adds.
+  mutable bool keep_records = false;
+  mutable int cell_records = 0;
+  mutable bool store_vec = false;
   // Facet integrals whose kernel has the reference's ABI (run on the
   // host): 1 exterior, given as (cell, local facet) pairs; 2 interior,
   // given as (cell0, local facet0, cell1, local facet1) quads; 0 none. The
@@ -405,6 +415,12 @@ struct dfx_form
   std::int32_t* trow = nullptr;
   std::int32_t ntrow = 0;
   std::uint64_t trow_pattern = 0;
+  // Variant 18 (P1): the place of every contribution in its row's buffer
+  // (16 per cell), then the first places of the slots, of p1_place_bytes
+  // each; built for p1_pattern.
+  void* p1_places = nullptr;
+  int p1_place_bytes = 0;
+  std::uint64_t p1_pattern = 0;
   // Elasticity row groups: 4 rows each of 8 values (row or -1, first
   // incidence, incidences, CSR position, LDS slice offset, row length, 0,
   // 0); groups of edge rows, vertex rows and rows that are both end at
@@ -436,6 +452,7 @@ struct dfx_form
   std::int32_t nfrows = 0;
   void* cell_elem = nullptr;
   int row_variant = 1;             // row-kernel variant (dfx_form_autotune)
+  bool default_variant = false;    // neither set nor autotuned: choose_variant
 };
 
 namespace dfx

@@ -263,7 +263,7 @@ struct DirArgs
 template <typename T>
 __device__ inline T dir_of(Pair<T> g, T beta)
 {
-  return __builtin_fma(beta, g.y, g.x);
+  return fma_t(beta, g.y, g.x);
 }
 
 /// Start of the SpMV of iteration k: the stop test ||r||^2/||r0||^2 < rtol^2
@@ -1922,7 +1922,7 @@ __device__ inline bool coop_barrier(CoopSync* g, unsigned int nb, unsigned int& 
 template <typename T>
 __device__ inline T coop_dir(T z, T pold, T beta, bool first)
 {
-  return first ? z : __builtin_fma(beta, pold, z);
+  return first ? z : fma_t(beta, pold, z);
 }
 
 template <typename T, int RPT>

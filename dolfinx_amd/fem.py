@@ -283,7 +283,9 @@ class Form:
         with their plan at fixed positions, 15 structured Q1 rows in
         registers stored through an LDS slice, 16 a team of lanes per row
         forming the entries, 17 such teams gathering the element matrices
-        of 7)."""
+        of 7, 18 P1 rows by 16 lanes, a lane per incidence and then per
+        entry). Without a call the library chooses one for the element, the
+        mesh and the number of rows."""
         _lib.call("dfx_form_set_variant", self._h, int(variant))
 
     @property

@@ -1,0 +1,96 @@
+"""P1 rows by 16 lanes (variant 18, the default on tetrahedra), the default
+variants, the lifting and the system call's stored vector, against the oracle."""
+
+import numpy as np
+import pytest
+
+import oracle as O
+from dolfinx_amd import fem, la, mesh
+
+from conftest import rel_err
+from test_mesh_create import bicone, box_input
+
+pytestmark = pytest.mark.gpu
+
+MESHES = {
+    "one": (np.array([[0, 1, 2, 3]]), np.array([[0, 0, 0], [1, 0, 0], [0.2, 1, 0], [0.1, 0.3, 1.]])),
+    "box": box_input((5, 3, 4), O.TET, 4),
+    "fan": bicone(24),      # 48 cells at a vertex, 27 entries in its row
+    "wide": bicone(40),     # 320 contributions to a row, 43 entries
+}
+
+
+@pytest.mark.parametrize("dtype,tol", [(np.float64, 1e-13), (np.float32, 2e-6)])
+@pytest.mark.parametrize("name", list(MESHES))
+def test_rows_and_lifting(name, dtype, tol):
+    cells, x = MESHES[name]
+    om = O.Mesh.from_cells(O.TET, cells, x)
+    pm = mesh.create_mesh(mesh.CellType.tetrahedron, cells, x)
+    V = fem.functionspace(pm, ("Lagrange", 1))
+    dm, nd = om.dofmap(1)
+    rng = np.random.default_rng(8)
+    kap = rng.uniform(0.5, 2.0, (om.num_cells, 1))
+    f = rng.standard_normal((om.num_cells, 4))
+    a = fem.form("p1_stiffness_reaction", V, kap, [0.7], dtype)
+    L = fem.form("p1_source", V, f, None, dtype)
+    rp, cols = O.sparsity(dm, dm, nd)
+    bdofs = np.nonzero(rng.random(nd) < 0.3)[0].astype(np.int32)
+    mark = np.zeros(nd, np.int8)
+    mark[bdofs] = 1
+    g = rng.standard_normal(nd)
+    bc = fem.dirichletbc(V, bdofs, g)
+    c = np.array([0.7])
+    plain = O.assemble_matrix(O.K_P1TET_A, om.x, om.cells, dm, 1, kap, c, None, None, rp, cols)
+    zeroed = O.assemble_matrix(O.K_P1TET_A, om.x, om.cells, dm, 1, kap, c, mark, mark, rp, cols)
+    O.set_diagonal(zeroed, bdofs, 1, 2.0, rp, cols)
+    for variant in (None, 18):
+        if variant is not None:
+            a.set_variant(variant)
+        A = fem.assemble_matrix(a)
+        assert rel_err(A.data, plain) <= tol
+        fem.assemble_matrix(a, [], 1.0, A)
+        assert rel_err(A.data, 2 * plain) <= tol
+        assert rel_err(fem.assemble_matrix(a, [bc], 2.0).data, zeroed) <= tol
+    br = O.assemble_vector(O.K_P1TET_L, om.x, om.cells, dm, 1, f, None, nd)
+    O.lift_bc(br, O.K_P1TET_A, om.x, om.cells, dm, 1, kap, c, g, mark)
+    O.bc_set(br, bdofs, g)
+    # a system call from scratch, again over its results, and its parts
+    A, b = fem.assemble_system(a, L, [bc], 2.0)
+    for _ in range(2):
+        assert rel_err(A.data, zeroed) <= tol and rel_err(b.array, br) <= 2 * tol
+        fem.assemble_system(a, L, [bc], 2.0, A, b)
+    parts = fem.assemble_vector(L)
+    fem.apply_lifting(parts, [a], [[bc]])
+    fem.set_bc(parts, [bc])
+    assert np.array_equal(parts.array, b.array)
+
+
+@pytest.mark.parametrize("cell,n,name", [
+    (O.HEX, (6, 5, 4), "q1"), (O.TET, (4, 3, 3), "p3"), (O.TET, (11, 9, 8), "p3")])
+def test_defaults_lift_from_the_assemblys_records(cell, n, name):
+    """Nonzero data through a system call (the lifting reads the records that
+    the matrix assembly left) equals the separate calls, for the variants that
+    the library chooses and some others."""
+    deg = 3 if name == "p3" else 1
+    pm = mesh.create_box([[0, 0, 0], [1, 1, 1]], n, mesh.CellType(cell))
+    V = fem.functionspace(pm, ("Lagrange", deg))
+    rng = np.random.default_rng(2)
+    nc = pm.topology.cells.shape[0]
+    a = fem.form(f"{name}_stiffness_reaction", V, rng.uniform(0.5, 2.0, (nc, 1)), [0.3])
+    L = (fem.form("q1_source", V, rng.standard_normal((nc, 8))) if name == "q1"
+         else fem.form("p3_source", V, None, [1.3]))
+    bc = fem.dirichletbc(V, fem.locate_boundary_dofs(V), rng.standard_normal(V.num_dofs))
+    ref = None
+    for variant in [None] + ([1, 10, 13, 15] if name == "q1" else [3, 7, 16]):
+        if variant is not None:
+            a.set_variant(variant)
+        A, b = fem.assemble_system(a, L, [bc])
+        A1 = fem.assemble_matrix(a, [bc])
+        b1 = fem.assemble_vector(L)
+        fem.apply_lifting(b1, [a], [[bc]])
+        fem.set_bc(b1, [bc])
+        if variant != 3:  # (LDS atomics: the order of the additions varies)
+            assert np.array_equal(A.data, A1.data)
+        assert rel_err(b.array, b1.array) <= 1e-14
+        ref = ref or (A.data, b.array)
+        assert rel_err(A.data, ref[0]) <= 1e-13 and rel_err(b.array, ref[1]) <= 1e-13
