@@ -1847,6 +1847,116 @@ __global__ void __launch_bounds__(kBlock)
       vals[base + t] = acc[t];
 }
 
+/// The P1 element matrix row i from the cell factors: the terms of
+/// element_entry that are not zero, in its order and (as the compiler fuses
+/// its first sum into the first product) with its rounding.
+template <typename T>
+__device__ inline void p1_row(const T (&g)[7], int i, T (&e)[4])
+{
+  const T s = T(1.0 / 6.0), d = T(1.0 / 3.0), m0 = T(1.0 / 60.0), m1 = T(1.0 / 120.0);
+  auto mass = [&](T k, T m) { return fma_t(g[6], m, k); };
+  const T k00 = mass(fma_t(
+                         g[5], d,
+                         fma_t(g[4], d,
+                                       fma_t(g[3], d,
+                                                     fma_t(g[2], s,
+                                                                   fma_t(g[0], s, g[1] * s))))),
+                     m0);
+  const T k01 = mass(fma_t(g[4], -s, fma_t(g[3], -s, g[0] * -s)), m1);
+  const T k02 = mass(fma_t(g[5], -s, fma_t(g[3], -s, g[1] * -s)), m1);
+  const T k03 = mass(fma_t(g[5], -s, fma_t(g[4], -s, g[2] * -s)), m1);
+  const T k11 = mass(g[0] * s, m0), k22 = mass(g[1] * s, m0), k33 = mass(g[2] * s, m0);
+  const T k12 = mass(g[3] * s, m1), k13 = mass(g[4] * s, m1), k23 = mass(g[5] * s, m1);
+  e[0] = i == 0 ? k00 : i == 1 ? k01 : i == 2 ? k02 : k03;
+  e[1] = i == 0 ? k01 : i == 1 ? k11 : i == 2 ? k12 : k13;
+  e[2] = i == 0 ? k02 : i == 1 ? k12 : i == 2 ? k22 : k23;
+  e[3] = i == 0 ? k03 : i == 1 ? k13 : i == 2 ? k23 : k33;
+}
+
+/// Lifting part of a P1 cell: le[i] = sum over its Dirichlet columns j (bits
+/// of m) of A_ij d_j, in FP64.
+template <typename T>
+__device__ inline void p1_lift(const T (&g)[7], std::uint32_t m, const double (&d)[4],
+                               double* __restrict__ lift)
+{
+  double le[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+  {
+    T e[4];
+    p1_row<T>(g, i, e);
+    le[i] = 0.0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      if ((m >> j) & 1u)
+        le[i] = __builtin_fma(double(e[j]), d[j], le[i]);
+  }
+  double2* o = reinterpret_cast<double2*>(lift);
+  o[0] = make_double2(le[0], le[1]);
+  o[1] = make_double2(le[2], le[3]);
+}
+
+/// P1 lifting, cells: the parts of the cells with a Dirichlet column, d = g -
+/// x0 (cell_system_k leaves the same parts in a system call).
+template <typename T>
+__global__ void __launch_bounds__(kBlock)
+    p1_cell_lift_k(std::int32_t nc, const std::int32_t* __restrict__ dm, const T* __restrict__ cd,
+                   const std::uint32_t* __restrict__ mask, const double* __restrict__ gd,
+                   const T* __restrict__ x0, double* __restrict__ lift)
+{
+  const std::int64_t c = blockIdx.x * std::int64_t(kBlock) + threadIdx.x;
+  if (c >= nc)
+    return;
+  const std::uint32_t m = mask[c];
+  if (!m)
+    return;
+  const int4 v4 = *reinterpret_cast<const int4*>(dm + 4 * c);
+  const std::int32_t v[4] = {v4.x, v4.y, v4.z, v4.w};
+  T g[7];
+  std::uint32_t bits;
+  load_factors<T>(cd, c, g, bits);
+  double d[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j)
+  {
+    const bool on = (m >> j) & 1u;
+    d[j] = (on && gd ? gd[v[j]] : 0.0) - (on && x0 ? double(x0[v[j]]) : 0.0);
+  }
+  p1_lift<T>(g, m, d, lift + 4 * c);
+}
+
+/// P1 lifting, rows: b[r] -= alpha times the parts of the row's incidences, in
+/// cell order (as row_vector_k with LIFT).
+template <typename T>
+__global__ void __launch_bounds__(kBlock)
+    p1_row_lift_k(std::int32_t nplan, const std::int32_t* __restrict__ inc_off,
+                  const std::int32_t* __restrict__ inc, const std::uint32_t* __restrict__ mask,
+                  const double* __restrict__ lift, double alpha, T* __restrict__ b)
+{
+  const std::int32_t r = blockIdx.x * kBlock + threadIdx.x;
+  if (r >= nplan)
+    return;
+  const std::int32_t p0 = inc_off[r], p1 = inc_off[r + 1];
+  double s = 0;
+  for (std::int32_t pb = p0; pb < p1; pb += 8)
+  {
+    std::int32_t q[8];
+    std::uint32_t m[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      q[u] = inc[min(pb + u, p1 - 1)];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      m[u] = mask[q[u] / 4];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (pb + u < p1 && m[u])
+        s += lift[q[u]];
+  }
+  if (s != 0.0)
+    b[r] = static_cast<T>(double(b[r]) - alpha * s);
+}
+
 /// Plan of variant 18, one thread per row: the contributions to the row (four
 /// per incidence) sorted by slot and, inside a slot, by incidence. ipos gives
 /// each contribution its place, soff (row length + 1 values at rp[r] + r) the
@@ -1876,32 +1986,6 @@ __global__ void __launch_bounds__(kBlock)
   for (std::int32_t t = len; t > 0; --t)
     start[t] = start[t - 1];
   start[0] = 0;
-}
-
-/// The P1 element matrix row i from the cell factors: the terms of
-/// element_entry that are not zero, in its order and (as the compiler fuses
-/// its first sum into the first product) with its rounding.
-template <typename T>
-__device__ inline void p1_row(const T (&g)[7], int i, T (&e)[4])
-{
-  const T s = T(1.0 / 6.0), d = T(1.0 / 3.0), m0 = T(1.0 / 60.0), m1 = T(1.0 / 120.0);
-  auto mass = [&](T k, T m) { return fma_t(g[6], m, k); };
-  const T k00 = mass(fma_t(
-                         g[5], d,
-                         fma_t(g[4], d,
-                                       fma_t(g[3], d,
-                                                     fma_t(g[2], s,
-                                                                   fma_t(g[0], s, g[1] * s))))),
-                     m0);
-  const T k01 = mass(fma_t(g[4], -s, fma_t(g[3], -s, g[0] * -s)), m1);
-  const T k02 = mass(fma_t(g[5], -s, fma_t(g[3], -s, g[1] * -s)), m1);
-  const T k03 = mass(fma_t(g[5], -s, fma_t(g[4], -s, g[2] * -s)), m1);
-  const T k11 = mass(g[0] * s, m0), k22 = mass(g[1] * s, m0), k33 = mass(g[2] * s, m0);
-  const T k12 = mass(g[3] * s, m1), k13 = mass(g[4] * s, m1), k23 = mass(g[5] * s, m1);
-  e[0] = i == 0 ? k00 : i == 1 ? k01 : i == 2 ? k02 : k03;
-  e[1] = i == 0 ? k01 : i == 1 ? k11 : i == 2 ? k12 : k13;
-  e[2] = i == 0 ? k02 : i == 1 ? k12 : i == 2 ? k22 : k23;
-  e[3] = i == 0 ? k03 : i == 1 ? k13 : i == 2 ? k23 : k33;
 }
 
 /// Variant 18 (P1): 16 lanes per row. First a lane per incidence: the four
@@ -3253,14 +3337,16 @@ __global__ void __launch_bounds__(kBlock)
 /// stiffness form and the P1/Q1 source form on the same mesh): the cell
 /// factor record and BC mask of the matrix, as cell_factors_k, and the
 /// element source vector, as cell_source_k, from one load of the cell's
-/// vertex row and coordinates.
+/// vertex row and coordinates. With lift (P1, nonzero Dirichlet data g), the
+/// cells with a Dirichlet column also leave their part of the lifting, lift[4 c
+/// + i] = sum over those columns j of A_ij g_j, for the row pass of the vector.
 template <typename T, int NV, bool COMPACT = false>
 __global__ void __launch_bounds__(kBlock)
     cell_system_k(std::int32_t nc, const T* __restrict__ x, const std::int32_t* __restrict__ xdm,
                   const T* __restrict__ coeffs, int cstride, T creac,
                   const std::int8_t* __restrict__ bc, T* __restrict__ cd,
                   std::uint32_t* __restrict__ mask, const T* __restrict__ src, int sstride,
-                  T* __restrict__ be)
+                  T* __restrict__ be, const double* __restrict__ gd, double* __restrict__ lift)
 {
   const std::int64_t c
       = xcd_contiguous(blockIdx.x, gridDim.x) * std::int64_t(kBlock) + threadIdx.x;
@@ -3296,6 +3382,17 @@ __global__ void __launch_bounds__(kBlock)
   affine_source<T, NV>(q0, q1, q2, q3, f, out);
   if (mask)
     mask[c] = m;
+  if constexpr (NV == 4)
+  {
+    if (lift && m)
+    {
+      double d[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        d[j] = (m >> j) & 1u ? gd[v[j]] : 0.0;
+      p1_lift<T>(g, m, d, lift + 4 * c);
+    }
+  }
   if constexpr (COMPACT)
     store_compact<T>(cd, c, g);
   else
@@ -3339,12 +3436,17 @@ __global__ void __launch_bounds__(kBlock)
 /// incidences, in cell order. inc holds c * K + i; the cell pass stored
 /// entry (i, comp) of cell c at be[(i BS + comp) nc + c] (corner-major).
 /// Eight incidences per group, loads at clamped positions so that all
-/// sixteen loads of a group are in flight together.
-template <typename T, int K, int BS>
+/// sixteen loads of a group are in flight together. LIFT: minus the lifting
+/// parts that cell_system_k left for the cells with a Dirichlet column, summed
+/// in FP64 and subtracted once. 61 x 47 x 53 P1 FP32: 30 us for both, against
+/// 16 us and a lifting pass of 37 us (nearly every wavefront of that pass had a
+/// row beside the boundary, and formed its entries for a few lanes).
+template <typename T, int K, int BS, bool LIFT = false>
 __global__ void __launch_bounds__(kBlock)
     row_vector_k(std::int32_t nplan, std::int32_t nc, const std::int32_t* __restrict__ inc_off,
                  const std::int32_t* __restrict__ inc, const T* __restrict__ be,
-                 T* __restrict__ b, int store)
+                 T* __restrict__ b, int store, const std::uint32_t* __restrict__ mask = nullptr,
+                 const double* __restrict__ lift = nullptr)
 {
   const std::int64_t t = blockIdx.x * std::int64_t(kBlock) + threadIdx.x;
   if (t >= std::int64_t(nplan) * BS)
@@ -3353,20 +3455,36 @@ __global__ void __launch_bounds__(kBlock)
   const int comp = static_cast<int>(t % BS);
   const std::int32_t p0 = inc_off[r], p1 = inc_off[r + 1];
   T s = 0;
+  double sl = 0;
   for (std::int32_t pb = p0; pb < p1; pb += 8)
   {
     std::int32_t q[8];
     T v[8];
+    std::uint32_t m[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u)
       q[u] = inc[min(pb + u, p1 - 1)];
 #pragma unroll
     for (int u = 0; u < 8; ++u)
+    {
       v[u] = be[std::int64_t((q[u] % K) * BS + comp) * nc + q[u] / K];
+      if constexpr (LIFT)
+        m[u] = mask[q[u] / K];
+    }
 #pragma unroll
     for (int u = 0; u < 8; ++u)
       if (pb + u < p1)
+      {
         s += v[u];
+        if constexpr (LIFT)
+          if (m[u])
+            sl += lift[q[u]];
+      }
+  }
+  if constexpr (LIFT)
+  {
+    b[t] = static_cast<T>(double(s) - sl);
+    return;
   }
   b[t] = store ? s : b[t] + s;
 }
@@ -4953,8 +5071,15 @@ void lift_rows(dfx_form& f, const dfx_bc& bc, const T* x0, double alpha, T* b)
   const T* cd = static_cast<const T*>(f.cell_data);
   const T* ref = static_cast<const T*>(f.ref_tensors);
   if (f.d.dofs_per_cell == 4)
-    row_lift_k<T, 4><<<blocks_for(std::int64_t(nplan) * kLiftLanes), kBlock, 0, stream()>>>(
-        nplan, f.inc_off, f.inc, f.dofmap, cd, f.cell_mask, ref, bc.g, x0, alpha, b);
+  {
+    if (!f.lift_vec)
+      f.lift_vec = static_cast<double*>(
+          dmalloc(sizeof(double) * 4 * std::max<std::int64_t>(f.d.num_cells, 1)));
+    p1_cell_lift_k<T><<<blocks_for(f.d.num_cells), kBlock, 0, stream()>>>(
+        f.d.num_cells, f.dofmap, cd, f.cell_mask, bc.g, x0, f.lift_vec);
+    p1_row_lift_k<T><<<blocks_for(nplan), kBlock, 0, stream()>>>(nplan, f.inc_off, f.inc,
+                                                                f.cell_mask, f.lift_vec, alpha, b);
+  }
   else if (compact)
     row_lift_k<T, 8, true><<<blocks_for(std::int64_t(nplan) * kLiftLanes), kBlock, 0, stream()>>>(
         nplan, f.inc_off, f.inc, f.dofmap, cd, f.cell_mask, ref, bc.g, x0, alpha, b);
@@ -5187,7 +5312,10 @@ void vector_rows(const dfx_form& f, T* b)
         nc, static_cast<const T*>(f.x), f.x_dofmap, static_cast<const T*>(f.coeffs),
         f.d.cstride, f.affine ? 1 : 0, be);
   const std::int32_t nplan = f.max_dof + 1;
-  if (nv == 4)
+  if (nv == 4 && f.use_lift)
+    row_vector_k<T, 4, 1, true><<<blocks_for(nplan), kBlock, 0, stream()>>>(
+        nplan, nc, f.inc_off, f.inc, be, b, store, f.use_lift_mask, f.use_lift);
+  else if (nv == 4)
     row_vector_k<T, 4, 1><<<blocks_for(nplan), kBlock, 0, stream()>>>(nplan, nc, f.inc_off, f.inc,
                                                                        be, b, store);
   else
@@ -6137,6 +6265,7 @@ dfx_status dfx_form_destroy(dfx_form* f)
     dfree(f->gblk);
     dfree(f->team_rows);
     dfree(f->p1_places);
+    dfree(f->lift_vec);
     dfree(f->trow);
     dfree(f->facets);
     dfree(f->finc_off);
@@ -6853,7 +6982,7 @@ namespace
 /// is the same is checked once per pair (one comparison pass and a host
 /// round trip), then remembered by form id.
 template <typename T>
-void launch_cell_system(const dfx_form& a, const dfx_form& L, const dfx_bc* bc)
+void launch_cell_system(const dfx_form& a, const dfx_form& L, const dfx_bc* bc, bool lift)
 {
   const std::int32_t nc = a.d.num_cells;
   auto go = [&](auto kern)
@@ -6862,7 +6991,8 @@ void launch_cell_system(const dfx_form& a, const dfx_form& L, const dfx_bc* bc)
         nc, static_cast<const T*>(a.x), a.x_dofmap, static_cast<const T*>(a.coeffs),
         a.d.cstride, static_cast<T>(a.constants[0]), bc ? bc->marker : nullptr,
         static_cast<T*>(a.cell_data), bc ? a.cell_mask : nullptr,
-        static_cast<const T*>(L.coeffs), L.d.cstride, static_cast<T*>(L.cell_vec));
+        static_cast<const T*>(L.coeffs), L.d.cstride, static_cast<T*>(L.cell_vec),
+        lift ? bc->g : nullptr, lift ? a.lift_vec : nullptr);
   };
   // the records variant 15 reads when the form keeps compact ones
   if (a.d.nodes_per_cell == 8 && a.row_variant == 15 && a.compact_records)
@@ -6874,7 +7004,9 @@ void launch_cell_system(const dfx_form& a, const dfx_form& L, const dfx_bc* bc)
   check_launch("cell_system");
 }
 
-bool system_cell_pass(dfx_form& a, dfx_form& L, const dfx_bc* bc)
+/// want_lift: the vector pass may take the lifting with it (b is stored from
+/// zero, every row of it); *lifted says whether it will.
+bool system_cell_pass(dfx_form& a, dfx_form& L, const dfx_bc* bc, bool want_lift, bool* lifted)
 {
   const int ka = a.d.kernel, kl = L.d.kernel;
   const bool pair = (ka == DFX_K_P1TET_A && kl == DFX_K_P1TET_L)
@@ -6908,12 +7040,22 @@ bool system_cell_pass(dfx_form& a, dfx_form& L, const dfx_bc* bc)
       return false;
     a.same_geometry_as = L.id;
   }
+  const bool lift = want_lift && ka == DFX_K_P1TET_A && bc && bc->g && bc->ndofs > 0
+                    && (a.lift_vec || !capturing());
+  if (lift && !a.lift_vec)
+    a.lift_vec = static_cast<double*>(dmalloc(sizeof(double) * 4 * a.d.num_cells));
   if (a.d.dtype == DFX_F64)
-    launch_cell_system<double>(a, L, bc);
+    launch_cell_system<double>(a, L, bc, lift);
   else
-    launch_cell_system<float>(a, L, bc);
+    launch_cell_system<float>(a, L, bc, lift);
   a.cell_data_ready = true;
   L.cell_vec_ready = true;
+  if (lift)
+  {
+    L.use_lift = a.lift_vec;
+    L.use_lift_mask = a.cell_mask;
+    *lifted = true;
+  }
   return true;
 }
 } // namespace
@@ -6956,12 +7098,23 @@ dfx_status dfx_assemble_system(dfx_csr* A, const dfx_form* a, const dfx_bc* bc, 
             a.keep_records = false;
             L.cell_vec_ready = false;
             L.store_vec = false;
+            L.use_lift = nullptr;
           }
         } rg{af, Lf};
         if (A->dtype == a->d.dtype && A->bs == a->d.bs && a->max_dof < A->nrows
             && a->max_dof < A->ncols)
           a->d.dtype == DFX_F64 ? choose_variant<double>(af, *A) : choose_variant<float>(af, *A);
-        const bool shared = system_cell_pass(af, Lf, bc);
+        // a source form that reaches every entry of b stores them (zero_b);
+        // others add to zeros
+        const int kl = L->d.kernel;
+        const bool store_b
+            = zero_b && b->dtype == L->d.dtype && !L->host_kernel && !L->host_facets
+              && (kl == DFX_K_P1TET_L || kl == DFX_K_Q1HEX_L || kl == DFX_K_P2TET_ELAST_L
+                  || kl == DFX_K_P3TET_L)
+              && std::int64_t(L->max_dof + 1) * L->d.bs == b->n;
+        bool lifted = false;
+        const bool shared
+            = system_cell_pass(af, Lf, bc, store_b && bc && bc->n_total == b->n, &lifted);
         // the vector assembly reads only L's data and writes only b: on
         // large meshes it runs on the second stream while the matrix is
         // assembled (below ~1M cells the fork and join cost more than the
@@ -6998,13 +7151,7 @@ dfx_status dfx_assemble_system(dfx_csr* A, const dfx_form* a, const dfx_bc* bc, 
         }
         {
           StreamScope on(fork ? c.aux : c.stream);
-          // a source form that reaches every entry stores them; others add
-          // to zeros
-          const int k = L->d.kernel;
-          if (zero_b && b->dtype == L->d.dtype && !L->host_kernel && !L->host_facets
-              && (k == DFX_K_P1TET_L || k == DFX_K_Q1HEX_L || k == DFX_K_P2TET_ELAST_L
-                  || k == DFX_K_P3TET_L)
-              && std::int64_t(L->max_dof + 1) * L->d.bs == b->n)
+          if (store_b)
             Lf.store_vec = true;
           else if (zero_b)
             ok(dfx_vec_set(b, 0.0));
@@ -7022,7 +7169,7 @@ dfx_status dfx_assemble_system(dfx_csr* A, const dfx_form* a, const dfx_bc* bc, 
           ok(dfx_set_diagonal(A, bc, diag));
         if (fork)
           jg.join();
-        if (bc)
+        if (bc && !lifted)
           ok(dfx_apply_lifting(b, a, bc, nullptr, 1.0));
         if (both)
         {

@@ -327,6 +327,13 @@ struct dfx_form
   mutable bool keep_records = false;
   mutable int cell_records = 0;
   mutable bool store_vec = false;
+  // Lifting parts of the cells with a Dirichlet column (4 per cell, FP64,
+  // written by the cell pass of a P1 system call with nonzero data), and in
+  // the linear form, during such a call, the parts and masks that its row
+  // pass subtracts.
+  double* lift_vec = nullptr;
+  mutable const double* use_lift = nullptr;
+  mutable const std::uint32_t* use_lift_mask = nullptr;
   // Facet integrals whose kernel has the reference's ABI (run on the
   // host): 1 exterior, given as (cell, local facet) pairs; 2 interior,
   // given as (cell0, local facet0, cell1, local facet1) quads; 0 none. The
