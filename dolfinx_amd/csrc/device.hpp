@@ -32,6 +32,7 @@ struct Context
   int device = 0;
   int num_cu = 256;
   bool cooperative = false; // cooperative launches (co-resident grids) supported
+  std::size_t lds_per_block = 64 * 1024; // LDS a workgroup may have
   hipStream_t stream = nullptr;
   hipStream_t aux = nullptr;
   hipEvent_t fork = nullptr, join = nullptr;
