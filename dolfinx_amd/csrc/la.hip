@@ -901,8 +901,8 @@ __global__ void __launch_bounds__(kBlock)
 /// consecutive rows (coalesced, no LDS), 16-bit column offsets where the
 /// slice allows. Entries are taken sixteen at a time (values and columns,
 /// then the x gathers) and each row is summed left to right with separate
-/// multiply and add, the order and rounding of the stream kernel and of the
-/// reference's row loop; padding is skipped. Workgroups take groups of 4
+/// multiply and add, the order and rounding of the reference's row loop;
+/// padding is skipped. Workgroups take groups of 4
 /// slices, each XCD a contiguous range. With dotv, partial sums of y.dotv
 /// go to partials.
 template <typename T, int G, bool DIR>
@@ -1835,7 +1835,7 @@ int pair_blocks(std::int64_t n)
 // ---------------------------------------------------------------------
 // CG of a small scalar system in one cooperative launch. A system of a few
 // ten thousand rows lives in the L2 caches, and each kernel of the
-// three-kernel iteration is a short chain of dependent round trips plus a
+// other paths is a short chain of dependent round trips plus a
 // launch; here every block stays resident for the whole solve and the
 // phases are separated by grid barriers, two per iteration:
 //   phase A  p = z + beta p_old on the block's rows (z = dinv r), written
@@ -1855,8 +1855,8 @@ int pair_blocks(std::int64_t n)
 // barrier only the gathers go out, all of a thread's together); a wait gives
 // up after a bounded
 // number of polls and raises a flag that every block sees, so the grid
-// always drains. Same stop test and FP64 reductions as the
-// three-kernel path; sums are grouped differently, so the last bits (and
+// always drains. Same stop test and FP64 reductions as the other
+// paths; sums are grouped differently, so the last bits (and
 // at most an iteration) may differ from it. P1 on 32^3 cubes (36,000 rows, 71
 // workgroups): 13.9 us per iteration, 18.2 us with the rows read again in
 // every iteration.
@@ -2222,7 +2222,7 @@ int cg_coop_run(const dfx_csr& A, const T* b, T* x, int max_it, double rtol, boo
   if (le != hipSuccess)
   {
     // refused (the process cannot launch co-resident grids): the caller
-    // runs the three-kernel iteration, here and for later solves
+    // runs the separate kernels, here and for later solves
     (void)hipGetLastError();
     ctx().cooperative = false;
     return -1;

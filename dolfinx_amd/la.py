@@ -132,7 +132,8 @@ class MatrixCSR:
                   _lib.ptr(cols), _lib.ptr(v))
 
     def set_lanes(self, lanes):
-        """SpMV kernel of mult: 0 default, 1 row-block stream, 2..64 lanes
+        """SpMV kernel of mult: 0 default, 1 row-block stream (or,
+        where the matrix is large enough, a lane per row), 2..64 lanes
         per row, -1 the solvers' sliced-ELL copy of the values as they are
         now (set again after the values change)."""
         _lib.call("dfx_csr_set_lanes", self._h, int(lanes))

@@ -188,8 +188,9 @@ dfx_status dfx_csr_get_pattern(const dfx_csr* A, int64_t* row_ptr,
 
 /* SpMV autotuner (no counterpart in the reference): times the SpMV
  * variants on this matrix and keeps the fastest for every later SpMV/CG on
- * it: 1 the row-block stream kernel, 2..64 lanes per row (scalar CSR), 2
- * one thread per (block row, component) (block CSR). Returns the choice
+ * it: 1 the row-block stream kernel (or the row-lane kernel, where a scalar
+ * matrix is large enough for it), 2..64 lanes per row (scalar CSR), 2 one
+ * thread per (block row, component) (block CSR). Returns the choice
  * and its time per SpMV. */
 dfx_status dfx_csr_autotune(dfx_csr* A, int32_t* lanes, float* ms);
 /* Fix the SpMV variant as above (0 restores the built-in heuristic). */
@@ -432,7 +433,7 @@ typedef struct
   int32_t classic;     /* 0: a scalar system of at most 65,536 rows is solved
                           in one cooperative launch (resident blocks, grid
                           barriers; check_every and graph do not apply);
-                          1: always the three-kernel iteration */
+                          1: always separate kernels per iteration */
 } dfx_cg_opts;
 
 typedef struct
