@@ -2994,12 +2994,14 @@ dfx_status dfx_csr_create(const int64_t* row_ptr, const int32_t* cols, int32_t n
               A->win = nullptr;
             }
           }
-          if (!A->win)
-          {
-            A->rbase = static_cast<std::int32_t*>(dmalloc(sizeof(std::int32_t) * A->nblk));
-            stream_cols_k<<<A->nblk, kBlock, 0, stream()>>>(row_blocks(*A), A->row_ptr, A->cols,
-                                                            A->rbase, A->cols16);
-          }
+        }
+        if (bs == 1 && A->nblk > 0 && !A->win)
+        {
+          // read for every row block, of a matrix without entries too
+          // (cols16 is then null: no block is narrow, none has entries)
+          A->rbase = static_cast<std::int32_t*>(dmalloc(sizeof(std::int32_t) * A->nblk));
+          stream_cols_k<<<A->nblk, kBlock, 0, stream()>>>(row_blocks(*A), A->row_ptr, A->cols,
+                                                          A->rbase, A->cols16);
         }
         if (nrows > 0)
           diag_pos_k<<<(nrows + kBlock - 1) / kBlock, kBlock, 0, stream()>>>(nrows, A->row_ptr, A->cols, A->diag);

@@ -5,7 +5,7 @@ import numpy as np
 import pytest
 import scipy.sparse as sps
 
-from dolfinx_amd import la
+from dolfinx_amd import la, solvers
 
 pytestmark = pytest.mark.gpu
 
@@ -70,3 +70,33 @@ def test_row_lanes_rectangular():
     """Fewer columns than rows; the last rows are empty."""
     rp, cols, vals = banded((1 << 18) + 5, 1 << 18, range(0, 5), 1.0, 3)
     check(rp, cols, vals, 1 << 18, np.float32)
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("n", [1, 255, 257, (1 << 18) + 3])
+def test_no_entries(dtype, n):
+    """Rows without any entry: the product adds nothing, whatever the kernel,
+    and CG of b = 0 stops at once with x as it was."""
+    def matrix():
+        return la.MatrixCSR(np.zeros(n + 1, np.int64), np.zeros(0, np.int32), dtype=dtype)
+
+    rng = np.random.default_rng(n)
+    x = la.Vector.from_array(rng.standard_normal(n).astype(dtype))
+    y0 = rng.standard_normal(n).astype(dtype)
+    A = matrix()
+    for lanes in (0, 1, 2, 64):
+        A.set_lanes(lanes)
+        y = la.Vector.from_array(y0)
+        A.mult(x, y)
+        assert np.array_equal(y.array, y0)
+    A.autotune()
+    y = la.Vector.from_array(y0)
+    A.mult(x, y)
+    assert np.array_equal(y.array, y0)
+    S = la.MatrixCSR.shared(A, dtype)
+    S.mult(x, y)
+    assert np.array_equal(y.array, y0)
+    for classic in (False, True):
+        z = la.Vector.from_array(y0)
+        r = solvers.cg(matrix(), la.Vector(n, dtype), z, classic=classic)
+        assert r.converged and r.iterations == 0 and np.array_equal(z.array, y0)
