@@ -900,16 +900,6 @@ __device__ inline void load_factors(const T* __restrict__ cd, std::int64_t c, T 
   }
 }
 
-/// Orders the LDS accesses of the lanes of one wavefront around it
-/// (release and acquire fences at wavefront scope and a wave barrier): a
-/// value one lane writes before it is seen by the others reading after it.
-__device__ inline void wave_sync()
-{
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 /// a[sl[j]] += v[j] for the unmasked j of one incidence. The K slots of an
 /// incidence are distinct columns of its row, so every value is read
 /// before any is written: the K LDS reads are in flight together instead

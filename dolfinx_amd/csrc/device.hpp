@@ -133,6 +133,16 @@ __device__ inline double wave_sum(double v)
   return v;
 }
 
+/// Orders the LDS accesses of the lanes of one wavefront around it
+/// (release and acquire fences at wavefront scope and a wave barrier): a
+/// value one lane writes before it is seen by the others reading after it.
+__device__ inline void wave_sync()
+{
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 /// Sum over a 256-thread block (4 wavefronts of 64); result valid in
 /// thread 0. Fixed order, so deterministic.
 __device__ inline double block_sum_256(double v, double* lds /*[4]*/)

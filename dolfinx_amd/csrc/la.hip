@@ -626,6 +626,9 @@ __global__ void __launch_bounds__(kBlock)
     block_partials<1>(d, partials);
 }
 
+/// A 16-bit half of a word that was stored whole.
+typedef std::uint16_t __attribute__((may_alias)) AliasU16;
+
 /// Rows of a wavefront in the row-lane SpMV, and its longest row.
 constexpr int kRowGroup = 64;
 constexpr int kRowLaneMax = 32;
@@ -717,7 +720,7 @@ __global__ void __launch_bounds__(2 * kRowGroup)
   __shared__ double red[2];
   const int wave = threadIdx.x / kRowGroup, lane = threadIdx.x % kRowGroup;
   const T* val = reinterpret_cast<const T*>(sval[wave]);
-  const std::uint16_t* col = reinterpret_cast<const std::uint16_t*>(scol[wave]);
+  const AliasU16* col = reinterpret_cast<const AliasU16*>(scol[wave]);
   double d = 0.0;
   const int stopped
       = stop ? __hip_atomic_load(stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
@@ -770,7 +773,7 @@ __global__ void __launch_bounds__(2 * kRowGroup)
     const std::int32_t r = g * kRowGroup + lane, n = len, k0 = kb;
     const int4 b = w;
     const T y0 = yold, d0 = dv;
-    __builtin_amdgcn_wave_barrier();
+    wave_sync(); // the lanes read each other's stores
     T xv[NI];
 #pragma unroll
     for (int k = 0; k < NI; ++k)
@@ -796,7 +799,7 @@ __global__ void __launch_bounds__(2 * kRowGroup)
       if (dotv)
         d += double(yr) * double(d0);
     }
-    __builtin_amdgcn_wave_barrier();
+    wave_sync(); // before the next group's stores
   }
   if (partials)
   {
