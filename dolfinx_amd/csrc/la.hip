@@ -5,6 +5,7 @@
 #include "device.hpp"
 
 #include <algorithm>
+#include <array>
 #include <atomic>
 #include <chrono>
 #include <cmath>
@@ -2137,15 +2138,6 @@ __global__ void __launch_bounds__(kBlock)
   }
 }
 
-/// LDS of the cooperative CG that keeps its rows there, or 0 when they do not
-/// fit a workgroup's LDS (maxrow entries per row, rpt rows per thread).
-template <typename T>
-std::size_t coop_rows_lds(std::int32_t maxrow, int rpt)
-{
-  const std::size_t need = (sizeof(T) + 2) * std::size_t(maxrow) * rpt * kBlock;
-  return need <= ctx().lds_per_block ? need : 0;
-}
-
 /// The cooperative CG kernel for rpt rows per thread.
 template <typename T>
 const void* coop_kernel(int rpt, bool lds)
@@ -2158,6 +2150,35 @@ const void* coop_kernel(int rpt, bool lds)
   return rpt == 1   ? k(cg_coop_k<T, 1, false>)
          : rpt == 2 ? k(cg_coop_k<T, 2, false>)
                     : k(cg_coop_k<T, 4, false>);
+}
+
+/// Bytes of LDS that the cooperative CG with its rows in LDS takes for its
+/// own arrays.
+template <typename T>
+std::size_t coop_fixed_lds(int rpt)
+{
+  static const std::array<std::size_t, 3> known = []
+  {
+    std::array<std::size_t, 3> b{};
+    for (int i = 0; i < 3; ++i)
+    {
+      hipFuncAttributes at{};
+      DFX_HIP(hipFuncGetAttributes(&at, coop_kernel<T>(1 << i, true)));
+      b[i] = at.sharedSizeBytes;
+    }
+    return b;
+  }();
+  return known[rpt == 1 ? 0 : rpt == 2 ? 1 : 2];
+}
+
+/// LDS for the rows of the cooperative CG that keeps them there, or 0 when
+/// they do not fit a workgroup's LDS beside the kernel's own arrays (maxrow
+/// entries per row, rpt rows per thread).
+template <typename T>
+std::size_t coop_rows_lds(std::int32_t maxrow, int rpt)
+{
+  const std::size_t need = (sizeof(T) + 2) * std::size_t(maxrow) * rpt * kBlock;
+  return need + coop_fixed_lds<T>(rpt) <= ctx().lds_per_block ? need : 0;
 }
 
 /// Rows per thread and blocks of the cooperative CG for A, or 0 when the

@@ -27,18 +27,27 @@ def ragged(n, longest, dtype):
         vals += [w, w]
     S = sp.csr_matrix((np.concatenate(vals), (np.concatenate(rows), np.concatenate(cols))),
                       shape=(n, n))
+    if longest % 2 == 0:  # one row of exactly `longest` entries
+        length = np.diff(S.indptr)
+        p = int(np.argmax(length[:n - longest]))
+        more = [q for q in range(p + half + 1, n) if q % 37 != 5][:longest - length[p]]
+        E = sp.csr_matrix((np.full(len(more), 0.1 / longest), ([p] * len(more), more)), (n, n))
+        S = (S + E + E.T).tocsr()
+        assert np.diff(S.indptr).max() == longest
     S.sort_indices()
     A = la.MatrixCSR(S.indptr.astype(np.int64), S.indices.astype(np.int32), dtype=dtype)
     A.data = S.data.astype(dtype)
     return A, S.astype(dtype).astype(np.float64)
 
 
-# rows per workgroup: one per thread up to 16,384 rows, then two; an LDS of
-# 160 KiB holds 64 (FP64) or 106 (FP32) entries per thread
+# rows per workgroup: one per thread up to 16,384 rows, then two; beside the
+# kernel's own arrays an LDS of 160 KiB holds 63 (FP64) or 106 (FP32) entries
+# per thread: 64 (and 32 with two rows) would fill it to the last byte
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 @pytest.mark.parametrize("n,longest", [(1, 1), (255, 15), (257, 17), (700, 33), (511, 63),
-                                       (600, 65), (600, 105), (600, 107), (16384, 15),
-                                       (16385, 31), (20000, 35), (65536, 17)])
+                                       (511, 64), (600, 65), (600, 105), (600, 106), (600, 107), (16384, 15),
+                                       (16385, 31), (16385, 32), (20000, 35),
+                                       (65536, 17)])
 def test_coop_rows(n, longest, dtype):
     A, S = ragged(n, longest, dtype)
     b = np.random.default_rng(3).standard_normal(n).astype(dtype)
