@@ -7031,8 +7031,10 @@ bool system_cell_pass(dfx_form& a, dfx_form& L, const dfx_bc* bc, bool want_lift
       return false;
     a.same_geometry_as = L.id;
   }
+  // the parts are numbered by a's dofmap and summed through L's incidences:
+  // both forms on the vertex map (a is, and the vertex maps agree)
   const bool lift = want_lift && ka == DFX_K_P1TET_A && bc && bc->g && bc->ndofs > 0
-                    && (a.lift_vec || !capturing());
+                    && L.dofmap == L.x_dofmap && (a.lift_vec || !capturing());
   if (lift && !a.lift_vec)
     a.lift_vec = static_cast<double*>(dmalloc(sizeof(double) * 4 * a.d.num_cells));
   if (a.d.dtype == DFX_F64)

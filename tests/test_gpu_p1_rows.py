@@ -1,6 +1,8 @@
 """P1 rows by 16 lanes (variant 18, the default on tetrahedra), the default
 variants, the lifting and the system call's stored vector, against the oracle."""
 
+import copy
+
 import numpy as np
 import pytest
 
@@ -94,3 +96,28 @@ def test_defaults_lift_from_the_assemblys_records(cell, n, name):
         assert rel_err(b.array, b1.array) <= 1e-14
         ref = ref or (A.data, b.array)
         assert rel_err(A.data, ref[0]) <= 1e-13 and rel_err(b.array, ref[1]) <= 1e-13
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_source_form_of_another_numbering(dtype):
+    """A source form whose dofs are numbered otherwise than the stiffness
+    form's, on the same geometry: the lifting of a system call goes to the
+    stiffness form's rows, as in the separate calls."""
+    pm = mesh.create_box([[0, 0, 0], [1, 1, 1]], (5, 4, 3), mesh.CellType.tetrahedron)
+    V = fem.functionspace(pm, ("Lagrange", 1))
+    rng = np.random.default_rng(6)
+    nc = pm.topology.cells.shape[0]
+    W = copy.copy(V)
+    W._h = None
+    W.dofmap = copy.copy(V.dofmap)
+    W.dofmap.list = rng.permutation(V.num_dofs).astype(np.int32)[V.dofmap.list]
+    a = fem.form("p1_stiffness_reaction", V, rng.uniform(0.5, 2.0, (nc, 1)), [0.7], dtype)
+    L = fem.form("p1_source", W, rng.standard_normal((nc, 4)), None, dtype)
+    bc = fem.dirichletbc(V, fem.locate_boundary_dofs(V), rng.standard_normal(V.num_dofs))
+    parts = fem.assemble_vector(L)
+    fem.apply_lifting(parts, [a], [[bc]])
+    fem.set_bc(parts, [bc])
+    A, b = fem.assemble_system(a, L, [bc])
+    for _ in range(2):
+        assert np.array_equal(b.array, parts.array)
+        fem.assemble_system(a, L, [bc], 1.0, A, b)
