@@ -7008,6 +7008,10 @@ bool system_cell_pass(dfx_form& a, dfx_form& L, const dfx_bc* bc, bool want_lift
       || !row_path(a) || a.row_variant == 10 || a.d.num_cells == 0 || !a.cell_data
       || !L.cell_vec || (bc && !a.cell_mask))
     return false;
+  // (a BC of another size is refused by the matrix assembly that follows; the
+  // cell pass reads its markers)
+  if (bc && bc->n_total <= a.max_dof)
+    return false;
   if (a.same_geometry_as != L.id)
   {
     if (capturing())

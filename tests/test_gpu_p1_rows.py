@@ -8,6 +8,7 @@ import pytest
 
 import oracle as O
 from dolfinx_amd import fem, la, mesh
+from dolfinx_amd._lib import DfxError
 
 from conftest import rel_err
 from test_mesh_create import bicone, box_input
@@ -121,3 +122,22 @@ def test_source_form_of_another_numbering(dtype):
     for _ in range(2):
         assert np.array_equal(b.array, parts.array)
         fem.assemble_system(a, L, [bc], 1.0, A, b)
+
+
+@pytest.mark.parametrize("cell,name", [(mesh.CellType.tetrahedron, "p1"),
+                                       (mesh.CellType.hexahedron, "q1")])
+def test_condition_of_another_space_is_refused(cell, name):
+    """Dirichlet data for fewer dofs than the forms have: the system call
+    refuses it before any kernel reads it."""
+    V, W = (fem.functionspace(mesh.create_box([[0, 0, 0], [1, 1, 1]], n, cell), ("Lagrange", 1))
+            for n in ((9, 8, 7), (2, 2, 2)))
+    nc, k = V.dofmap.list.shape
+    a = fem.form(f"{name}_stiffness_reaction", V, np.ones((nc, 1)), [0.7])
+    L = fem.form(f"{name}_source", V, np.ones((nc, k)))
+    A, b = fem.assemble_system(a, L)
+    small = fem.dirichletbc(W, fem.locate_boundary_dofs(W), np.ones(W.num_dofs))
+    with pytest.raises(DfxError, match="BC size does not match"):
+        fem.assemble_system(a, L, [small], 1.0, A, b)
+    bc = fem.dirichletbc(V, fem.locate_boundary_dofs(V))
+    fem.assemble_system(a, L, [bc], 1.0, A, b)
+    assert np.array_equal(A.data, fem.assemble_matrix(a, [bc]).data)
