@@ -5061,7 +5061,11 @@ void lift_rows(dfx_form& f, const dfx_bc& bc, const T* x0, double alpha, T* b)
   const std::int32_t nplan = f.max_dof + 1;
   const T* cd = static_cast<const T*>(f.cell_data);
   const T* ref = static_cast<const T*>(f.ref_tensors);
-  if (f.d.dofs_per_cell == 4)
+  if (f.d.dofs_per_cell == 4 && !f.lift_vec && capturing())
+    // the cells' parts have no room yet and none can be allocated
+    row_lift_k<T, 4><<<blocks_for(std::int64_t(nplan) * kLiftLanes), kBlock, 0, stream()>>>(
+        nplan, f.inc_off, f.inc, f.dofmap, cd, f.cell_mask, ref, bc.g, x0, alpha, b);
+  else if (f.d.dofs_per_cell == 4)
   {
     if (!f.lift_vec)
       f.lift_vec = static_cast<double*>(

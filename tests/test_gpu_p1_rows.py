@@ -7,7 +7,7 @@ import numpy as np
 import pytest
 
 import oracle as O
-from dolfinx_amd import fem, la, mesh
+from dolfinx_amd import fem, graph, la, mesh
 from dolfinx_amd._lib import DfxError
 
 from conftest import rel_err
@@ -141,3 +141,34 @@ def test_condition_of_another_space_is_refused(cell, name):
     bc = fem.dirichletbc(V, fem.locate_boundary_dofs(V))
     fem.assemble_system(a, L, [bc], 1.0, A, b)
     assert np.array_equal(A.data, fem.assemble_matrix(a, [bc]).data)
+
+
+@pytest.mark.parametrize("dtype,tol", [(np.float64, 1e-14), (np.float32, 1e-6)])
+def test_first_lifting_inside_a_capture(dtype, tol):
+    """A P1 form that never lifted can be recorded doing so."""
+    V = fem.functionspace(mesh.create_box([[0, 0, 0], [1, 1, 1]], (5, 4, 3),
+                                          mesh.CellType.tetrahedron), ("Lagrange", 1))
+    rng = np.random.default_rng(9)
+    nc, k = V.dofmap.list.shape
+    kap, f = rng.uniform(0.5, 2.0, (nc, 1)), rng.standard_normal((nc, k))
+    bc = fem.dirichletbc(V, fem.locate_boundary_dofs(V), rng.standard_normal(V.num_dofs))
+    x0 = la.Vector.from_array(rng.standard_normal(V.num_dofs).astype(dtype))
+
+    def lifted(a, L, b):
+        b.set(0.0)
+        fem.assemble_vector(L, b)
+        fem.apply_lifting(b, [a], [[bc]], [x0], 0.5)
+
+    L = fem.form("p1_source", V, f, None, dtype)
+    ref = la.Vector(V.num_dofs, dtype)
+    lifted(fem.form("p1_stiffness_reaction", V, kap, [0.7], dtype), L, ref)
+    a, b = fem.form("p1_stiffness_reaction", V, kap, [0.7], dtype), la.Vector(V.num_dofs, dtype)
+    g = graph.Graph()
+    with g.capture():
+        lifted(a, L, b)
+    for _ in range(3):
+        b.set(7.0)
+        g.launch()
+        assert rel_err(b.array, ref.array) <= tol
+        lifted(a, L, b)  # (its own kernels, eagerly, between the replays)
+        assert np.array_equal(b.array, ref.array)
