@@ -5002,12 +5002,21 @@ void choose_variant(dfx_form& f, const dfx_csr& A)
   if (!f.default_variant || !row_path(f))
     return;
   ensure_plan(f, A);
+  // inside a capture no plan can be built: without one, the kernels that
+  // need only the slots
+  const bool build = !capturing();
+  const std::uint64_t id = A.pattern_id;
   if (f.d.kernel == DFX_K_P1TET_A)
-    f.row_variant = ensure_p1<T>(f, A) ? 18 : 1;
+    f.row_variant
+        = (build || (f.p1_places && f.p1_pattern == id)) && ensure_p1<T>(f, A) ? 18 : 1;
   else if (f.d.kernel == DFX_K_Q1HEX_A)
-    f.row_variant = ensure_struct(f, A) ? 15 : 1;
+    f.row_variant
+        = (build || (f.struct_ok >= 0 && f.struct_pattern == id)) && ensure_struct(f, A) ? 15 : 1;
   else if (f.d.kernel == DFX_K_P3TET_A)
-    f.row_variant = A.nrows >= 20000 && team_fits<T>(A) ? 16 : 3;
+    f.row_variant = A.nrows >= 20000 && team_fits<T>(A)
+                            && (build || (f.trow && f.trow_pattern == id))
+                        ? 16
+                        : 3;
 }
 
 template <typename T>

@@ -172,3 +172,36 @@ def test_first_lifting_inside_a_capture(dtype, tol):
         assert rel_err(b.array, ref.array) <= tol
         lifted(a, L, b)  # (its own kernels, eagerly, between the replays)
         assert np.array_equal(b.array, ref.array)
+
+
+@pytest.mark.parametrize("cell,name", [(mesh.CellType.tetrahedron, "p1"),
+                                       (mesh.CellType.hexahedron, "q1")])
+def test_first_single_assembly_inside_a_capture(cell, name):
+    """A form assembled so far by the batched call alone (which leaves its
+    slots, not the plan of the default variant) can be recorded by itself;
+    outside of captures it then takes its default variant."""
+    V = fem.functionspace(mesh.create_box([[0, 0, 0], [1, 1, 1]], (5, 4, 3), cell),
+                          ("Lagrange", 1))
+    nc = V.dofmap.list.shape[0]
+    kap = np.random.default_rng(4).uniform(0.5, 2.0, (nc, 1))
+    bc = fem.dirichletbc(V, fem.locate_boundary_dofs(V))
+    a = fem.form(f"{name}_stiffness_reaction", V, kap, [0.7])
+    A = fem.create_matrix(a)
+    fem.assemble_matrix_batched([a], [bc], [A])
+    ref = A.data
+    g = graph.Graph()
+    with g.capture():
+        A.set_value(0.0)
+        fem.assemble_matrix(a, [bc], 1.0, A)
+    for _ in range(3):
+        A.data = np.full(A.nnz, 3.0)
+        g.launch()
+        assert rel_err(A.data, ref) <= 1e-14
+        A.set_value(0.0)
+        fem.assemble_matrix(a, [bc], 1.0, A)
+        assert rel_err(A.data, ref) <= 1e-14
+    a.set_variant(18 if name == "p1" else 15)
+    eager = A.data
+    A.set_value(0.0)
+    fem.assemble_matrix(a, [bc], 1.0, A)
+    assert np.array_equal(A.data, eager)
