@@ -4993,9 +4993,10 @@ void launch_row_assemble(dfx_form& f, dfx_csr& A, const dfx_bc* bc)
 /// Measured (us per matrix, FP64 unless noted): P1, 18 against 1: 8.9 and 18.7
 /// at 720 rows, 18.9 and 28.9 at 36,000, 59 and 90 at 160,000 (FP32 38 and
 /// 58). Q1 on a structured box, 15 against 1: 8.8 and 13.3 at 8^3 cells, 12.6
-/// and 21.8 at 40 x 41 x 42, 174 and 375 at 128^3. P3, 16 against 3: 20.5 and
-/// 12.0 at 4^3 cubes (2,200 rows), 39.0 and 44.4 at 12^3 (51,000), 196 and 288
-/// at 24^3 (FP32 122 and 310).
+/// and 21.8 at 40 x 41 x 42, 174 and 375 at 128^3. P3, 16 against 3: 18.1 and
+/// 9.5 at 4^3 cubes (2,200 rows), 19.8 and 18.3 at 8^3 (15,600), 23.6 and 23.1
+/// at 9^3 (22,000; FP32 21.0 and 25.7), 23.8 and 28.6 at 10^3 (29,800), 196 and
+/// 288 at 24^3 (FP32 122 and 310).
 template <typename T>
 void choose_variant(dfx_form& f, const dfx_csr& A)
 {

@@ -281,8 +281,8 @@ struct dfx_csr
   std::int32_t nblk = 0;
   // 16-bit columns (bs = 1; nnz + 2 places). Row-lane SpMV: window and
   // offset in the windows of the row's 64-row group (win, int4 per group);
-  // otherwise (win null) offsets from the first column of the row block
-  // (rbase per row block, -1 where they do not fit).
+  // otherwise (win null) offsets from the first column of the row block.
+  // rbase: that column per row block, -1 where the stream SpMV reads cols.
   void* win = nullptr;
   std::int32_t* rbase = nullptr;
   std::uint16_t* cols16 = nullptr;

@@ -634,13 +634,15 @@ typedef std::uint16_t __attribute__((may_alias)) AliasU16;
 constexpr int kRowGroup = 64;
 constexpr int kRowLaneMax = 32;
 /// Rows from which a matrix of short rows is served by the row-lane SpMV. It
-/// needs many groups per resident wavefront (8 per CU at FP64): measured
-/// against the stream SpMV, FP64 27-entry rows 146 against 179 us at 2.1 M
-/// rows, but 33.9 against 30.7 us at 523,000 and 24.5 against 19.8 us at
-/// 300,000 (the matrix is then in the on-package cache and the gathers hide
-/// behind five times as many wavefronts); FP64 15-entry rows 14.8 against
-/// 16.5 us at 358,000; FP32 27-entry rows 96 against 146 us at 2.1 M and 16.0
-/// against 17.7 us at 275,000.
+/// needs many groups per resident wavefront (8 per CU at FP64): below, the
+/// matrix is in the on-package cache and the stream SpMV hides its gathers
+/// behind five times as many wavefronts. Measured, row-lane against stream in
+/// us: FP64 rows of 27 entries 32.6 and 29.6 at 531,000 rows, 50.4 and 47.5 at
+/// 913,000, 60.5 and 59.8 at 1.03 M, 75.9 and 76.1 at 1.16 M, 95.7 and 99.3 at
+/// 1.44 M (145 and 176 at 2.1 M with 32-bit columns); FP64 rows of 15 11.6 and
+/// 11.1 at 250,000, 12.1 and 12.3 at 275,000, 14.2 and 15.8 at 358,000; FP32
+/// rows of 27 14.6 and 16.6 at 250,000, 33.5 and 46.8 at 913,000, of 15 8.1 and
+/// 8.4 at 250,000, 10.0 and 11.6 at 358,000.
 inline std::int32_t row_lane_min_rows(int dtype, std::int32_t max_row)
 {
   return dtype == DFX_F64 && max_row > 16 ? 1 << 20 : 1 << 18;
@@ -1394,8 +1396,9 @@ inline bool block_stream(const dfx_csr& A)
 }
 
 /// Whether the row-lane SpMV serves A (rows of at most kRowLaneMax entries
-/// whose groups' columns fit the windows), and its launch.
-inline bool use_rows(const dfx_csr& A) { return A.win && (A.lanes == 0 || A.lanes == 1); }
+/// whose groups' columns fit the windows, no other kernel asked for), and its
+/// launch.
+inline bool use_rows(const dfx_csr& A) { return A.win && A.lanes == 0; }
 
 template <typename T>
 int launch_rows(const dfx_csr& A, const T* x, T* y, int accumulate, const T* dotv,
@@ -2834,9 +2837,10 @@ int autotune_lanes(dfx_csr& A, int reps, float* best_ms)
   DFX_HIP(hipEventCreate(&e1));
   int best = 0;
   float bms = 1e30f;
-  // block matrices: 1 stream, 2 one thread per (block row, component)
+  // block matrices: 1 stream, 2 one thread per (block row, component);
+  // scalar ones: 0 row-lane where its windows are there
   const int gmax = A.bs == 1 ? 64 : 2;
-  for (int G = 1; G <= gmax; G *= 2)
+  for (int G = A.win ? 0 : 1; G <= gmax; G = G ? 2 * G : 1)
   {
     if (G == 1 && A.nblk == 0)
       continue;
@@ -3019,13 +3023,17 @@ dfx_status dfx_csr_create(const int64_t* row_ptr, const int32_t* cols, int32_t n
             }
           }
         }
-        if (bs == 1 && A->nblk > 0 && !A->win)
+        if (bs == 1 && A->nblk > 0)
         {
           // read for every row block, of a matrix without entries too
-          // (cols16 is then null: no block is narrow, none has entries)
+          // (cols16 is then null: no block is narrow, none has entries);
+          // beside windows -1, the stream SpMV reads the 32-bit columns
           A->rbase = static_cast<std::int32_t*>(dmalloc(sizeof(std::int32_t) * A->nblk));
-          stream_cols_k<<<A->nblk, kBlock, 0, stream()>>>(row_blocks(*A), A->row_ptr, A->cols,
-                                                          A->rbase, A->cols16);
+          if (A->win)
+            DFX_HIP(hipMemsetAsync(A->rbase, 0xff, sizeof(std::int32_t) * A->nblk, stream()));
+          else
+            stream_cols_k<<<A->nblk, kBlock, 0, stream()>>>(row_blocks(*A), A->row_ptr, A->cols,
+                                                            A->rbase, A->cols16);
         }
         if (nrows > 0)
           diag_pos_k<<<(nrows + kBlock - 1) / kBlock, kBlock, 0, stream()>>>(nrows, A->row_ptr, A->cols, A->diag);
@@ -3063,6 +3071,8 @@ dfx_status dfx_csr_create_shared(const dfx_csr* P, int dtype, dfx_csr** out)
           A->rblk = nullptr;
           A->nblk = 0;
           A->rbase = nullptr;
+          if (A->win && A->nrows < row_lane_min_rows(dtype, A->max_row))
+            A->win = nullptr;
           if (!A->win)
             A->cols16 = nullptr;
         }

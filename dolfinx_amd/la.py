@@ -110,8 +110,9 @@ class MatrixCSR:
         return rp, ci
 
     def autotune(self):
-        """Pick the SpMV lanes per row for this matrix by timing (kept for
-        every later SpMV and CG on it). Returns (lanes, ms per SpMV)."""
+        """Pick the SpMV kernel for this matrix by timing (kept for every
+        later SpMV and CG on it). Returns (lanes as of set_lanes, ms per
+        SpMV)."""
         lanes, ms = C.c_int32(), C.c_float()
         _lib.call("dfx_csr_autotune", self._h, C.byref(lanes), C.byref(ms))
         return lanes.value, ms.value
@@ -132,10 +133,10 @@ class MatrixCSR:
                   _lib.ptr(cols), _lib.ptr(v))
 
     def set_lanes(self, lanes):
-        """SpMV kernel of mult: 0 default, 1 row-block stream (or,
-        where the matrix is large enough, a lane per row), 2..64 lanes
-        per row, -1 the solvers' sliced-ELL copy of the values as they are
-        now (set again after the values change)."""
+        """SpMV kernel of mult: 0 default (a lane per row of a large matrix
+        of short rows, otherwise the row-block stream), 1 row-block stream,
+        2..64 lanes per row, -1 the solvers' sliced-ELL copy of the values as
+        they are now (set again after the values change)."""
         _lib.call("dfx_csr_set_lanes", self._h, int(lanes))
 
     def mult(self, x, y):

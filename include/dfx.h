@@ -188,8 +188,8 @@ dfx_status dfx_csr_get_pattern(const dfx_csr* A, int64_t* row_ptr,
 
 /* SpMV autotuner (no counterpart in the reference): times the SpMV
  * variants on this matrix and keeps the fastest for every later SpMV/CG on
- * it: 1 the row-block stream kernel (or the row-lane kernel, where a scalar
- * matrix is large enough for it), 2..64 lanes per row (scalar CSR), 2 one
+ * it: 0 the row-lane kernel (where a scalar matrix is large enough for it),
+ * 1 the row-block stream kernel, 2..64 lanes per row (scalar CSR), 2 one
  * thread per (block row, component) (block CSR). Returns the choice
  * and its time per SpMV. */
 dfx_status dfx_csr_autotune(dfx_csr* A, int32_t* lanes, float* ms);

@@ -100,3 +100,53 @@ def test_no_entries(dtype, n):
         z = la.Vector.from_array(y0)
         r = solvers.cg(matrix(), la.Vector(n, dtype), z, classic=classic)
         assert r.converged and r.iterations == 0 and np.array_equal(z.array, y0)
+
+
+def product(A, x):
+    y = la.Vector(A.shape[0], A.dtype)
+    A.mult(x, y)
+    return y.array
+
+
+def test_kernel_of_a_large_matrix():
+    """set_lanes(1) and the autotuner reach the row-block stream on a matrix
+    that the row-lane kernel serves by default (the bits of its first rows are
+    those of a smaller matrix, which the stream serves), and a copy of the
+    pattern in the other precision takes the kernel of its own size rule."""
+    n, cut = (1 << 18) + 37, 100000
+    rp, cols, vals = banded(n, n, range(-520, 521, 40), 0.97, 7)
+    A = la.MatrixCSR(rp, cols, dtype=np.float32)
+    A.data = vals
+    B = la.MatrixCSR(rp[:cut + 1], cols[:rp[cut]], ncols=n, dtype=np.float32)
+    B.data = vals[:rp[cut]]
+    x = la.Vector.from_array(np.random.default_rng(1).standard_normal(n).astype(np.float32))
+    rows, few = product(A, x), product(B, x)[:cut - 256]
+    A.set_lanes(1)
+    assert np.array_equal(product(A, x)[:cut - 256], few)
+    assert not np.array_equal(rows[:cut - 256], few)
+    assert A.autotune()[0] in (0, 1, 2, 4, 8, 16, 32, 64)
+    A.set_lanes(0)
+    assert np.array_equal(product(A, x), rows)
+    # FP64 rows of this length need 2^20 rows: 8 lanes per row (27 entries)
+    D = la.MatrixCSR.shared(A, np.float64)
+    D.data = vals
+    xd = la.Vector.from_array(x.array.astype(np.float64))
+    default = product(D, xd)
+    D.set_lanes(8)
+    assert np.array_equal(default, product(D, xd))
+
+
+def test_shared_pattern_of_the_other_precision():
+    """FP32 values on a large FP64 pattern: the autotuner times the row-lane
+    kernel too and its choice gives the same product."""
+    n = (1 << 20) + 1
+    rp, cols, vals = banded(n, n, range(-520, 521, 40), 1.0, 11)
+    A = la.MatrixCSR.shared(la.MatrixCSR(rp, cols), np.float32)
+    A.data = vals
+    x = la.Vector.from_array(np.random.default_rng(1).standard_normal(n).astype(np.float32))
+    S = sps.csr_matrix((vals.astype(np.float32).astype(np.float64), cols, rp), shape=(n, n))
+    xd = x.array.astype(np.float64)
+    bound = 30 * np.finfo(np.float32).eps * (abs(S) @ abs(xd))
+    assert (np.abs(product(A, x) - S @ xd) <= bound).all()
+    assert A.autotune()[0] == 0  # (38 us; 2 to 64 lanes per row 60 or more)
+    assert (np.abs(product(A, x) - S @ xd) <= bound).all()
