@@ -633,20 +633,49 @@ typedef std::uint16_t __attribute__((may_alias)) AliasU16;
 /// Rows of a wavefront in the row-lane SpMV, and its longest row.
 constexpr int kRowGroup = 64;
 constexpr int kRowLaneMax = 32;
-/// Rows from which a matrix of short rows is served by the row-lane SpMV. It
-/// needs many groups per resident wavefront (8 per CU at FP64): below, the
-/// matrix is in the on-package cache and the stream SpMV hides its gathers
-/// behind five times as many wavefronts. Measured, row-lane against stream in
-/// us: FP64 rows of 27 entries 32.6 and 29.6 at 531,000 rows, 50.4 and 47.5 at
-/// 913,000, 60.5 and 59.8 at 1.03 M, 75.9 and 76.1 at 1.16 M, 95.7 and 99.3 at
-/// 1.44 M (145 and 176 at 2.1 M with 32-bit columns); FP64 rows of 15 11.6 and
-/// 11.1 at 250,000, 12.1 and 12.3 at 275,000, 14.2 and 15.8 at 358,000; FP32
-/// rows of 27 14.6 and 16.6 at 250,000, 33.5 and 46.8 at 913,000, of 15 8.1 and
-/// 8.4 at 250,000, 10.0 and 11.6 at 358,000.
+/// Rows from which a matrix of short rows may be served by the row-lane SpMV
+/// (row_lane_pays decides). It needs many groups per resident wavefront (8
+/// per CU at FP64): below, the matrix is in the on-package cache and the
+/// stream SpMV hides its gathers behind five times as many wavefronts.
+/// Measured, row-lane against stream in us: FP64 hexahedral rows of 27 entries
+/// 32.6 and 29.6 at 531,000 rows, 50.4 and 47.5 at 913,000, 60.5 and 59.8 at
+/// 1.03 M, 75.9 and 76.1 at 1.16 M, 95.7 and 99.3 at 1.44 M (145 and 176 at
+/// 2.1 M with 32-bit columns); FP64 tetrahedral rows of 15 never gain (14.2
+/// and 15.8 at 358,000, but 21.5 and 20.2 at 531,000, 39.0 and 36.0 at 1.03 M,
+/// 98.9 and 86.6 at 2.1 M); FP32 rows of 27 14.6 and 16.6 at 250,000, 33.5 and
+/// 46.8 at 913,000, of 15 8.1 and 8.4 at 250,000, 42.1 and 58.3 at 2.1 M.
 inline std::int32_t row_lane_min_rows(int dtype, std::int32_t max_row)
 {
-  return dtype == DFX_F64 && max_row > 16 ? 1 << 20 : 1 << 18;
+  if (dtype == DFX_F64)
+    return max_row > 16 ? 1 << 20 : 0x7fffffff;
+  return 1 << 18;
 }
+
+/// Entries that the row-lane SpMV walks per row: what its kernels are made
+/// for.
+constexpr int row_lane_steps(std::int32_t max_row)
+{
+  return max_row <= 16 ? 16 : max_row <= 27 ? 27 : kRowLaneMax;
+}
+
+/// Cache lines of x that the gathers of a product touch: 64 consecutive
+/// entries at a time, as the stream SpMV gathers, and one step of 64 rows at a
+/// time.
+struct GatherLines
+{
+  unsigned long long entries, rows;
+};
+
+/// Whether the row-lane order halves the lines: the stream SpMV's gathers then
+/// bound it. Rows in few runs of columns have no lines to save and the
+/// row-lane kernel is slower, by its padding to row_lane_steps and its few
+/// wavefronts. Ratio and us, row-lane against stream: FP64 hexahedra 2.7, 95.7
+/// and 99.3 at 1.44 M rows; FP32 tetrahedra 2.2, 8.5 and 9.6 at 275,000, and
+/// 2.5, 23.4 and 30.3 at 1.03 M; FP32 seven-point rows 0.95, 20.2 and 20.2
+/// (12.8 and 12.3 at 600,000); random columns 1.0, FP64 rows of 30 176 and 154;
+/// 31-entry bands 0.5, FP64 82.5 and 61.3, FP32 44.2 and 37.4; tridiagonal 0.1,
+/// FP64 30.9 and 13.7, FP32 19.3 and 13.5.
+inline bool row_lane_pays(const GatherLines& g) { return g.entries >= 2 * g.rows; }
 
 /// 16-bit columns of the row-lane SpMV: the wavefront of 64-row group g
 /// covers the group's columns by up to four windows of 2^14 columns, each
@@ -655,11 +684,13 @@ inline std::int32_t row_lane_min_rows(int dtype, std::int32_t max_row)
 /// ordering couple a few narrow bands (the breadth-first levels) far apart:
 /// of the 64-row groups of the 128^3 hexahedral matrix 43 % span more than
 /// 2^16 columns, and all are covered by the windows. *wide is set when a
-/// group needs more.
+/// group needs more. The gathers' lines of 128 bytes (2^shift columns) are
+/// added to *lines.
 __global__ void __launch_bounds__(kBlock)
     row_windows_k(std::int32_t nrows, std::int32_t ngroups, const std::int32_t* __restrict__ rp,
                   const std::int32_t* __restrict__ ci, int4* __restrict__ win,
-                  std::uint16_t* __restrict__ c16, int* wide)
+                  std::uint16_t* __restrict__ c16, int* wide, int steps, int shift,
+                  GatherLines* lines)
 {
   const std::int32_t g = blockIdx.x * (kBlock / kRowGroup) + threadIdx.x / kRowGroup;
   if (g >= ngroups)
@@ -694,11 +725,35 @@ __global__ void __launch_bounds__(kBlock)
   }
   if (out)
     *wide = 1;
+  // lines by entries, then by rows (as spmv_rows_k walks them: past a row's
+  // end its last entry again)
+  auto differ = [&](std::int32_t c)
+  {
+    const std::int32_t l = c >> shift;
+    unsigned int n = 0;
+    for (unsigned long long left = ~0ull; left; ++n)
+      left &= ~__ballot(l == __shfl(l, __ffsll(left) - 1, 64));
+    return n;
+  };
+  unsigned int by_entries = 0, by_rows = 0;
+  const std::int32_t r = min(g * kRowGroup + lane, nrows - 1), r0 = rp[r], r1 = rp[r + 1];
+  if (j1 > j0)
+  {
+    for (std::int32_t j = j0; j < j1; j += kRowGroup)
+      by_entries += differ(ci[min(j + lane, j1 - 1)]);
+    for (int k = 0; k < steps; ++k)
+      by_rows += differ(ci[max(min(r0 + k, r1 - 1), j0)]);
+  }
   if (lane == 0)
+  {
     win[g] = make_int4(base[0], base[1], base[2], base[3]);
+    atomicAdd(&lines->entries, static_cast<unsigned long long>(by_entries));
+    atomicAdd(&lines->rows, static_cast<unsigned long long>(by_rows));
+  }
 }
 
-/// Row-lane SpMV for matrices of short rows (at most NI entries), y (+)= A x.
+/// Row-lane SpMV for large matrices of short rows (at most NI entries) in
+/// scattered columns (row_lane_min_rows, row_lane_pays), y (+)= A x.
 /// A wavefront takes 64 consecutive rows: their entries are loaded in aligned
 /// pairs with coalesced loads, turned over in LDS, and lane l then walks row
 /// l. Neighbouring rows have neighbouring columns, so the x gathers of one
@@ -1395,9 +1450,8 @@ inline bool block_stream(const dfx_csr& A)
   return A.nblk > 0 && A.lanes <= 1 && (A.bs == 2 || A.bs == 3);
 }
 
-/// Whether the row-lane SpMV serves A (rows of at most kRowLaneMax entries
-/// whose groups' columns fit the windows, no other kernel asked for), and its
-/// launch.
+/// Whether the row-lane SpMV serves A (its windows were kept when it was
+/// created, and no other kernel was asked for), and its launch.
 inline bool use_rows(const dfx_csr& A) { return A.win && A.lanes == 0; }
 
 template <typename T>
@@ -1417,9 +1471,11 @@ int launch_rows(const dfx_csr& A, const T* x, T* y, int accumulate, const T* dot
                                              dotv, partials, stop);
     return nb;
   };
-  return A.max_row <= 16   ? go(spmv_rows_k<T, 16>)
-         : A.max_row <= 27 ? go(spmv_rows_k<T, 27>)
-                           : go(spmv_rows_k<T, kRowLaneMax>);
+  if constexpr (sizeof(T) == 4)
+    if (A.max_row <= 16)
+      return go(spmv_rows_k<T, row_lane_steps(16)>);
+  return A.max_row <= 27 ? go(spmv_rows_k<T, row_lane_steps(27)>)
+                         : go(spmv_rows_k<T, kRowLaneMax>);
 }
 
 template <typename T>
@@ -3007,16 +3063,21 @@ dfx_status dfx_csr_create(const int64_t* row_ptr, const int32_t* cols, int32_t n
           if (maxrow <= kRowLaneMax && nrows >= row_lane_min_rows(dtype, maxrow))
           {
             const std::int32_t ng = (nrows + kRowGroup - 1) / kRowGroup;
-            int4* win = static_cast<int4*>(dmalloc(sizeof(int4) * ng + sizeof(int)));
-            int* wide = reinterpret_cast<int*>(win + ng);
-            DFX_HIP(hipMemsetAsync(wide, 0, sizeof(int), stream()));
-            row_windows_k<<<(ng + 3) / 4, kBlock, 0, stream()>>>(nrows, ng, A->row_ptr, A->cols,
-                                                                win, A->cols16, wide);
+            struct Seen
+            {
+              GatherLines lines;
+              int wide;
+            } seen{};
+            int4* win = static_cast<int4*>(dmalloc(sizeof(int4) * ng + sizeof(Seen)));
+            Seen* d = reinterpret_cast<Seen*>(win + ng);
+            h2d(d, &seen, sizeof(Seen));
+            row_windows_k<<<(ng + 3) / 4, kBlock, 0, stream()>>>(
+                nrows, ng, A->row_ptr, A->cols, win, A->cols16, &d->wide, row_lane_steps(maxrow),
+                dtype == DFX_F64 ? 4 : 5, &d->lines);
             check_launch("row_windows");
-            int h = 0;
-            d2h(&h, wide, sizeof(int));
+            d2h(&seen, d, sizeof(Seen));
             A->win = win;
-            if (h)
+            if (seen.wide || !row_lane_pays(seen.lines))
             {
               dfree(win);
               A->win = nullptr;

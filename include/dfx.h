@@ -188,7 +188,7 @@ dfx_status dfx_csr_get_pattern(const dfx_csr* A, int64_t* row_ptr,
 
 /* SpMV autotuner (no counterpart in the reference): times the SpMV
  * variants on this matrix and keeps the fastest for every later SpMV/CG on
- * it: 0 the row-lane kernel (where a scalar matrix is large enough for it),
+ * it: 0 the row-lane kernel (large scalar matrices of short, scattered rows),
  * 1 the row-block stream kernel, 2..64 lanes per row (scalar CSR), 2 one
  * thread per (block row, component) (block CSR). Returns the choice
  * and its time per SpMV. */

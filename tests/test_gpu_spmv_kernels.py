@@ -10,12 +10,14 @@ from dolfinx_amd import la, solvers
 pytestmark = pytest.mark.gpu
 
 
-def banded(nrows, ncols, offsets, keep, seed):
+def banded(nrows, ncols, offsets, keep, seed, empty=0):
     """Pattern with the columns r + offset of each row r that exist, each kept
-    with probability keep; random values."""
+    with probability keep (every `empty`-th row without any); random values."""
     rng = np.random.default_rng(seed)
     c = np.arange(nrows)[:, None] + np.asarray(offsets)[None, :]
     on = (c >= 0) & (c < ncols) & (rng.random(c.shape) < keep)
+    if empty:
+        on[::empty] = False
     rp = np.concatenate([[0], np.cumsum(on.sum(1))])
     return rp, c[on].astype(np.int32), rng.standard_normal(int(rp[-1]))
 
@@ -66,6 +68,35 @@ def test_row_lanes(dtype, n, offsets, keep):
     check(rp, cols, vals, n, dtype)
 
 
+SPACED = {16: range(-320, 320, 40), 27: range(-520, 521, 40)}
+BANDS = {27: sorted([b + 40 * i for b in (-30000, 0, 30000) for i in range(-4, 5)]),
+         32: [-60000, -30000] + list(range(-420, 420, 30)) + [30000, 30040]}
+
+
+@pytest.mark.parametrize("dtype,n", [(np.float32, (1 << 18) + 37), (np.float64, (1 << 20) + 1)])
+@pytest.mark.parametrize("offsets,keep,empty,rows", [
+    (BANDS[32], 1.0, 0, True), (BANDS[27], 0.995, 0, True), (SPACED[27], 1.0, 5, True),
+    (SPACED[16], 1.0, 3, np.float32),         # FP64 rows of 16 stay on the stream
+    (range(-1, 2), 1.0, 0, False), (range(-13, 14), 1.0, 0, False),  # few lines per row
+    ([-10000, -100, -1, 0, 1, 100, 10000], 1.0, 0, False),
+    (SPACED[27], 0.5, 0, False),              # the same columns never side by side
+])
+def test_row_lane_choice(dtype, n, offsets, keep, empty, rows):
+    """Large matrices whose gathers touch half the lines in row order are
+    served by the row-lane kernel (its bits differ from the stream's), others
+    of any size by the stream."""
+    rp, cols, vals = banded(n, n, offsets, keep, 13, empty)
+    A = la.MatrixCSR(rp, cols, dtype=dtype)
+    A.data = vals
+    x = la.Vector.from_array(np.random.default_rng(1).standard_normal(n).astype(dtype))
+    y = product(A, x)
+    A.set_lanes(1)
+    assert np.array_equal(product(A, x), y) == (rows not in (True, dtype))
+    S = sps.csr_matrix((vals.astype(dtype).astype(np.float64), cols, rp), shape=(n, n))
+    xd = x.array.astype(np.float64)
+    assert (np.abs(y - S @ xd) <= 35 * np.finfo(dtype).eps * (abs(S) @ abs(xd))).all()
+
+
 def test_row_lanes_rectangular():
     """Fewer columns than rows; the last rows are empty."""
     rp, cols, vals = banded((1 << 18) + 5, 1 << 18, range(0, 5), 1.0, 3)
@@ -114,7 +145,7 @@ def test_kernel_of_a_large_matrix():
     those of a smaller matrix, which the stream serves), and a copy of the
     pattern in the other precision takes the kernel of its own size rule."""
     n, cut = (1 << 18) + 37, 100000
-    rp, cols, vals = banded(n, n, range(-520, 521, 40), 0.97, 7)
+    rp, cols, vals = banded(n, n, range(-520, 521, 40), 0.995, 7)
     A = la.MatrixCSR(rp, cols, dtype=np.float32)
     A.data = vals
     B = la.MatrixCSR(rp[:cut + 1], cols[:rp[cut]], ncols=n, dtype=np.float32)
