@@ -25,6 +25,9 @@ constexpr int kBlock = 256;
 // LDS slices that end a group of elasticity rows: on the box meshes four edge
 // rows of 27 blocks of 72 bytes, four vertex rows of 65
 constexpr std::size_t kTeamEdge = 8 * 1024, kTeamVertex = 20 * 1024;
+// LDS per CU of all groups up to which the elasticity rows go in one launch:
+// five rounds of resident groups
+constexpr std::size_t kTeamTogether = 5 * 160 * 1024;
 
 /// Two values of T as one aligned vector access (double2 or float2).
 template <typename T>
@@ -3791,16 +3794,16 @@ __device__ inline float row_bcast(float v)
 /// wavefronts that prefetch the next group were slower (1.24 ms), so were
 /// plain stores (1.02 ms; non-temporal ones keep the records in the L2).
 template <typename T, typename O, int KIND>
-__global__ void __launch_bounds__(64)
-    elast_team_k(const int4* __restrict__ erow, const std::int32_t* __restrict__ inc,
-                 const O* __restrict__ islots, const T* __restrict__ cd,
-                 const std::int8_t* __restrict__ bc, T* __restrict__ vals, int accumulate)
+__device__ __forceinline__ void
+elast_team(std::int32_t group, const int4* __restrict__ erow, const std::int32_t* __restrict__ inc,
+           const O* __restrict__ islots, const T* __restrict__ cd,
+           const std::int8_t* __restrict__ bc, T* __restrict__ vals, int accumulate)
 {
   constexpr int K = 10;
   extern __shared__ unsigned char smem_raw[];
   T* acc = reinterpret_cast<T*>(smem_raw);
   const int lane = threadIdx.x, team = lane >> 4, j = lane & 15, jc = min(j, K - 1);
-  const std::int64_t at = 4 * std::int64_t(xcd_contiguous(blockIdx.x, gridDim.x)) + team;
+  const std::int64_t at = 4 * std::int64_t(group) + team;
   const int4 ro = erow[2 * at];
   const int2 rs = *reinterpret_cast<const int2*>(erow + 2 * at + 1);
   const std::int32_t r = ro.x, p0 = ro.y, n = ro.z;
@@ -3999,6 +4002,42 @@ __global__ void __launch_bounds__(64)
         }
     }
   }
+}
+
+/// The groups of one kind.
+template <typename T, typename O, int KIND>
+__global__ void __launch_bounds__(64)
+    elast_team_k(const int4* __restrict__ erow, const std::int32_t* __restrict__ inc,
+                 const O* __restrict__ islots, const T* __restrict__ cd,
+                 const std::int8_t* __restrict__ bc, T* __restrict__ vals, int accumulate)
+{
+  elast_team<T, O, KIND>(xcd_contiguous(blockIdx.x, gridDim.x), erow, inc, islots, cd, bc, vals,
+                         accumulate);
+}
+
+/// The groups of all kinds (edge rows' up to end0, vertex rows' up to end1,
+/// then those that are both) in one launch, the vertex rows' first: they walk
+/// up to 24 cells where an edge row has 6. On small meshes a launch per kind
+/// waits twice for the longest row of its kind; on large ones the edge rows
+/// should not be held to the vertex rows' LDS (kTeamTogether). One launch
+/// against one per kind, us per matrix: FP64 22.7 and 29.2 on 6^3 cubes, 25.2
+/// and 33.6 on 10^3, 45.6 and 51.0 on 16^3 (9,000 groups), 59.4 and 56.9 on
+/// 18^3, 119.9 and 105.2 on 24^3; FP32 22.8 and 29.4 on 10^3, 47.1 and 51.2 on
+/// 20^3 (17,000 groups), 71.9 and 69.2 on 24^3.
+template <typename T, typename O>
+__global__ void __launch_bounds__(64)
+    elast_teams_k(std::int32_t end0, std::int32_t end1, const int4* __restrict__ erow,
+                  const std::int32_t* __restrict__ inc, const O* __restrict__ islots,
+                  const T* __restrict__ cd, const std::int8_t* __restrict__ bc,
+                  T* __restrict__ vals, int accumulate)
+{
+  const std::int32_t n = gridDim.x, q = blockIdx.x + end0, g = q < n ? q : q - n;
+  if (g < end0)
+    elast_team<T, O, 0>(g, erow, inc, islots, cd, bc, vals, accumulate);
+  else if (g < end1)
+    elast_team<T, O, 1>(g, erow, inc, islots, cd, bc, vals, accumulate);
+  else
+    elast_team<T, O, 2>(g, erow, inc, islots, cd, bc, vals, accumulate);
 }
 
 /// Lifting of the P2 elasticity form, b[(r, c)] -= alpha sum over the
@@ -4478,18 +4517,31 @@ void launch_elast(dfx_form& f, dfx_csr& A, const dfx_bc* bc)
               && std::int64_t(nc) * 100 * std::int64_t(sizeof(O)) <= 0xffffffffLL,
           "mesh too large for the elasticity row kernel (cell records above 4 GiB)");
   ensure_teams(f, A, sizeof(T));
-  auto go = [&](auto kern, int kind)
+  const int4* rows = reinterpret_cast<const int4*>(f.team_rows);
+  const O* slots = static_cast<const O*>(f.islots);
+  const T* cd = static_cast<const T*>(f.cell_data);
+  const std::int8_t* mark = bc ? bc->marker : nullptr;
+  T* vals = static_cast<T*>(A.values);
+  const int accumulate = A.zeroed ? 0 : 1;
+  const std::int32_t* end = f.team_end;
+  const std::size_t lds
+      = sizeof(T) * std::max({f.team_lds[0], f.team_lds[1], f.team_lds[2]});
+  if (end[2] > 0 && end[2] * lds <= kTeamTogether * ctx().num_cu)
+    elast_teams_k<T, O><<<end[2], 64, lds, stream()>>>(end[0], end[1], rows, f.inc, slots, cd,
+                                                       mark, vals, accumulate);
+  else
   {
-    const std::int32_t first = kind ? f.team_end[kind - 1] : 0, count = f.team_end[kind] - first;
-    if (count > 0)
-      kern<<<count, 64, sizeof(T) * f.team_lds[kind], stream()>>>(
-          reinterpret_cast<const int4*>(f.team_rows) + 8 * std::int64_t(first), f.inc,
-          static_cast<const O*>(f.islots), static_cast<const T*>(f.cell_data),
-          bc ? bc->marker : nullptr, static_cast<T*>(A.values), A.zeroed ? 0 : 1);
-  };
-  go(elast_team_k<T, O, 1>, 1);
-  go(elast_team_k<T, O, 0>, 0);
-  go(elast_team_k<T, O, 2>, 2);
+    auto go = [&](auto kern, int kind)
+    {
+      const std::int32_t first = kind ? end[kind - 1] : 0, count = end[kind] - first;
+      if (count > 0)
+        kern<<<count, 64, sizeof(T) * f.team_lds[kind], stream()>>>(
+            rows + 8 * std::int64_t(first), f.inc, slots, cd, mark, vals, accumulate);
+    };
+    go(elast_team_k<T, O, 1>, 1);
+    go(elast_team_k<T, O, 0>, 0);
+    go(elast_team_k<T, O, 2>, 2);
+  }
   check_launch("elasticity assembly");
 }
 

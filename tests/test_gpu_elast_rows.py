@@ -72,3 +72,30 @@ def test_rows_of_both_kinds():
     ref = O.assemble_matrix(O.K_P2TET_ELAST_A, pm.geometry.x, pm.geometry.dofmap, dm, 3, co, None,
                             None, None, rp, cols)
     assert rel_err(A.data, ref) <= 1e-12
+
+
+@pytest.mark.parametrize("mixed", [False, True])
+@pytest.mark.parametrize("dtype,n,tol", [(np.float64, (19, 18, 18), 1e-12),
+                                         (np.float32, (23, 23, 23), 5e-6)])
+def test_a_launch_per_kind(dtype, n, tol, mixed):
+    """Meshes above the line up to which all rows go in one launch (53,000
+    rows FP64, 104,000 FP32), in the Lagrange dofmap and with rows of both
+    kinds."""
+    pm = mesh.create_box([[0, 0, 0], [1, 1, 1]], n, mesh.CellType.tetrahedron)
+    V = fem.functionspace(pm, ("Lagrange", 2, (3,)))
+    nn, dm = V.dofmap.index_map_size, V.dofmap.list
+    if mixed:
+        dm[1::2] = dm[1::2, ::-1]
+    rng = np.random.default_rng(5)
+    co = np.stack(problems.lame_from_E(rng.uniform(0.5, 2.0, len(dm))), 1)
+    a = fem.form("p2_elasticity", V, co, None, dtype)
+    rp, cols = O.sparsity(dm, dm, nn)
+    bdofs = np.nonzero(rng.random(3 * nn) < 0.1)[0].astype(np.int32)
+    mark = np.zeros(3 * nn, np.int8)
+    mark[bdofs] = 1
+    A = fem.assemble_matrix(a, [fem.dirichletbc(V, bdofs)], 1.0,
+                            la.MatrixCSR(rp, cols, bs=3, dtype=dtype))
+    ref = O.assemble_matrix(O.K_P2TET_ELAST_A, pm.geometry.x, pm.geometry.dofmap, dm, 3, co, None,
+                            mark, mark, rp, cols)
+    O.set_diagonal(ref, bdofs, 3, 1.0, rp, cols)
+    assert rel_err(A.data, ref) <= tol
