@@ -2499,10 +2499,17 @@ int launch_cg_spmv(const dfx_csr& A, const T* p, T* q, CGState* st, bool sell)
 /// Per iteration, SpMV + the rest: FP32 Q1 of 880,000 rows 30.1 + 7.9 us
 /// against 26.5 + 16.1; P3 of 389,000 rows 38.7 + 8.9 against 36.2 + 15.6;
 /// 3 x 3 blocks of 67,000 rows 28.7 + 6.5 against 24.9 + 13.1; but FP64 Q1 of
-/// 2.1 M rows 155 + 28.7 against 142 + 39.1 (its vectors come from HBM).
+/// 2.1 M rows 155 + 28.7 against 142 + 39.1 (its vectors come from HBM). Block
+/// matrices gather bs pairs per block and need their values in that cache
+/// too: us per iteration, two kernels against three, 33.5 and 34.5 at 117 MB
+/// (3 x 3, 27 blocks per row, FP64), 39.4 and 40.0 at 156 MB (2 x 2, 81 per
+/// row), 46.1 and 44.0 at 175 MB (3 x 3, 81 per row, FP32), 79.6 and 75.2 at
+/// 259 MB, 98.2 and 90.3 at 292 MB, 169 and 163 at 583 MB.
 inline bool pair_cg(const dfx_csr& A, bool sell)
 {
   if (std::int64_t(A.nrows) * A.bs > (1 << 20))
+    return false;
+  if (A.bs > 1 && dtype_size(A.dtype) * A.nnz * A.bs * A.bs > (std::size_t(160) << 20))
     return false;
   return sell || block_stream(A)
          || (A.bs == 1 && A.nblk > 0 && lanes_per_row(A) == 1 && !use_rows(A));

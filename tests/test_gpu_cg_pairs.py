@@ -3,6 +3,7 @@ against the three-kernel one (lanes-per-row SpMV) and a direct solve."""
 
 import numpy as np
 import pytest
+import scipy.sparse as sps
 import scipy.sparse.linalg as spla
 
 from dolfinx_amd import la, problems, solvers
@@ -62,3 +63,27 @@ def test_pairs(kind, jacobi):
     assert solvers.cg(A, b, y, rtol=1e-3, classic=True, jacobi=jacobi).true_rel_residual <= 1e-10
     z = la.Vector(n)
     assert solvers.cg(A, la.Vector(n), z, classic=True, jacobi=jacobi).iterations == 0
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+def test_large_blocks(dtype):
+    """3 x 3 blocks whose values pass the line of the two-kernel iteration in
+    FP64 (175 MB) and not in FP32, against the residual on the host."""
+    n, half = 30000, 40
+    c = np.arange(n)[:, None] + np.arange(-half, half + 1)[None, :]
+    on = (c >= 0) & (c < n)
+    rp, cols = np.concatenate([[0], np.cumsum(on.sum(1))]), c[on].astype(np.int32)
+    rng = np.random.default_rng(2)
+    B = np.full((len(cols), 3, 3), -0.5 / (6 * half))
+    B[cols == np.repeat(np.arange(n), np.diff(rp))] = np.diag([1.0, 2.0, 3.0])
+    A = la.MatrixCSR(rp, cols, bs=3, dtype=dtype)
+    A.data = B.ravel()
+    b = rng.standard_normal(3 * n).astype(dtype)
+    x = la.Vector(3 * n, dtype)
+    rtol = 1e-10 if dtype == np.float64 else 1e-5
+    r = solvers.cg(A, la.Vector.from_array(b), x, rtol=rtol)
+    S = sps.bsr_matrix((B.astype(dtype).astype(np.float64), cols, rp), shape=(3 * n, 3 * n))
+    res = b.astype(np.float64) - S @ x.array.astype(np.float64)
+    # the recurrence's residual, and the rounding of 30 iterations on x
+    assert r.converged and r.iterations < 30
+    assert np.linalg.norm(res) <= (2 * rtol + 100 * np.finfo(dtype).eps) * np.linalg.norm(b)
