@@ -61,7 +61,7 @@ def test_assemble_system_matches_oracle(cell, n, dtype):
 
 
 @pytest.mark.parametrize("cell,n", CASES)
-@pytest.mark.parametrize("variant", list(range(18)))
+@pytest.mark.parametrize("variant", list(range(19)))
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
 def test_every_row_kernel_variant_matches_oracle(cell, n, variant, dtype):
     """Variants 0-3 use the reference tensors, 4-6 closed-form entries for
@@ -72,10 +72,11 @@ def test_every_row_kernel_variant_matches_oracle(cell, n, variant, dtype):
     Q1 rows with their plan at fixed positions, 15 structured rows in
     registers through an LDS slice (hexahedra only), 16 a team of lanes per
     row forming the entries from the cell records, 17 such teams gathering
-    the element matrices of the matrix-core product."""
+    the element matrices of the matrix-core product, 18 P1 rows by 16 lanes
+    (tetrahedra only)."""
     p = build(cell, n, dtype)
     p.a.set_variant(variant)
-    if variant in (9, 12, 13, 14, 15) and cell == O.TET:
+    if variant in ((9, 12, 13, 14, 15) if cell == O.TET else (18,)):
         with pytest.raises(DfxError, match="not available"):
             problems.assemble_system(p)
         return
@@ -91,7 +92,7 @@ def test_autotune_keeps_results():
     p = build(O.HEX, (20, 20, 20), np.float64)
     A = fem.create_matrix(p.a)
     variant, ms = p.a.autotune(A, p.bc)
-    assert 0 <= variant <= 17 and ms > 0
+    assert 0 <= variant <= 18 and ms > 0
     assert np.all(A.data == 0)
     fem.assemble_matrix(p.a, [p.bc], 1.0, A)
     ref = oracle_system(p, (20, 20, 20))

@@ -68,6 +68,27 @@ def test_rows_and_lifting(name, dtype, tol):
     assert np.array_equal(parts.array, b.array)
 
 
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("name", list(MESHES))
+def test_entries_are_those_of_variant_1(name, dtype):
+    """Variant 18 forms and adds the entries in the order and with the
+    rounding of the thread-per-row kernel: the same bits."""
+    cells, x = MESHES[name]
+    V = fem.functionspace(mesh.create_mesh(mesh.CellType.tetrahedron, cells, x), ("Lagrange", 1))
+    rng = np.random.default_rng(12)
+    kap = rng.uniform(0.5, 2.0, (V.dofmap.list.shape[0], 1))
+    a = fem.form("p1_stiffness_reaction", V, kap, [0.7], dtype)
+    bdofs = np.nonzero(rng.random(V.num_dofs) < 0.3)[0].astype(np.int32)
+    for bcs in ([], [fem.dirichletbc(V, bdofs)]):
+        out = []
+        for variant in (1, 18):
+            a.set_variant(variant)
+            A = fem.assemble_matrix(a, bcs)
+            fem.assemble_matrix(a, bcs, 1.0, A)  # added to what is there
+            out.append(A.data)
+        assert np.array_equal(*out)
+
+
 @pytest.mark.parametrize("cell,n,name", [
     (O.HEX, (6, 5, 4), "q1"), (O.TET, (4, 3, 3), "p3"), (O.TET, (11, 9, 8), "p3")])
 def test_defaults_lift_from_the_assemblys_records(cell, n, name):
