@@ -1,11 +1,13 @@
 """SpMV kernels at the edges of their chunks, pairs, row groups and column
 encodings, against scipy in FP64."""
 
+import ctypes as C
+
 import numpy as np
 import pytest
 import scipy.sparse as sps
 
-from dolfinx_amd import la, solvers
+from dolfinx_amd import _lib, la, solvers
 
 pytestmark = pytest.mark.gpu
 
@@ -181,3 +183,40 @@ def test_shared_pattern_of_the_other_precision():
     assert (np.abs(product(A, x) - S @ xd) <= bound).all()
     assert A.autotune()[0] == 0  # (38 us; 2 to 64 lanes per row 60 or more)
     assert (np.abs(product(A, x) - S @ xd) <= bound).all()
+
+
+@pytest.mark.parametrize("dtype,n", [(np.float32, (1 << 18) + 37), (np.float64, (1 << 20) + 37)])
+def test_cg_through_the_row_lane_kernel(dtype, n):
+    """CG whose product is the row-lane kernel (its partial sums and stop flag;
+    an odd number of groups, the last of 37 rows): rows of 27 scattered entries
+    with every fifth its diagonal alone, which the sliced-ELL copy would pad by
+    a quarter. The residual is checked on the host, the iterations against the
+    stream's, and the no-allocation solve where it takes the size."""
+    rp, cols, _ = banded(n, n, range(-520, 521, 40), 1.0, 3)
+    row = np.repeat(np.arange(n), np.diff(rp))
+    on = (row % 5 != 0) | (cols == row)       # (40 k keeps the remainder: symmetric)
+    row, cols = row[on], cols[on]
+    rp = np.concatenate([[0], np.cumsum(np.bincount(row, minlength=n))])
+    vals = np.where(cols == row, 1.0 + row % 3, -0.5 / 26).astype(dtype)
+    b = np.random.default_rng(5).standard_normal(n).astype(dtype)
+    S = sps.csr_matrix((vals.astype(np.float64), cols, rp), shape=(n, n))
+    rtol = 1e-10 if dtype == np.float64 else 1e-5
+    A = la.MatrixCSR(rp, cols, dtype=dtype)
+    A.data = vals
+    bv, its, ys = la.Vector.from_array(b), [], []
+
+    def solve(name):
+        x, opts, res = la.Vector(n, dtype), _lib.CGOpts(200, rtol, 1, 7, 0, 0), _lib.CGResult()
+        _lib.call(name, A.handle, bv.handle, x.handle, C.byref(opts), C.byref(res))
+        r = b.astype(np.float64) - S @ x.array.astype(np.float64)
+        assert np.linalg.norm(r) <= (2 * rtol + 100 * np.finfo(dtype).eps) * np.linalg.norm(b)
+        return res.iterations
+
+    for lanes in (0, 1):
+        A.set_lanes(lanes)
+        its.append(solve("dfx_cg_solve"))
+        ys.append(product(A, bv))
+        if n <= 1 << 20:
+            its.append(solve("dfx_cg_solve_noalloc"))
+    assert max(its) - min(its) <= 1 and 3 < its[0] < 60
+    assert not np.array_equal(*ys)            # (two kernels)
