@@ -3432,9 +3432,11 @@ __global__ void __launch_bounds__(kBlock)
 /// Eight incidences per group, loads at clamped positions so that all
 /// sixteen loads of a group are in flight together. LIFT: minus the lifting
 /// parts that cell_system_k left for the cells with a Dirichlet column, summed
-/// in FP64 and subtracted once. 61 x 47 x 53 P1 FP32: 30 us for both, against
-/// 16 us and a lifting pass of 37 us (nearly every wavefront of that pass had a
-/// row beside the boundary, and formed its entries for a few lanes).
+/// in FP64 and subtracted once. 61 x 47 x 53 P1 FP32: 31 us for both and 26 us
+/// for the cell pass that leaves the parts, against 16, 17 and a lifting pass
+/// of 37 us (nearly every wavefront of that pass had a row beside the boundary,
+/// and formed its entries for a few lanes); over buffers that change from call
+/// to call the whole call gains less, 94.3 us against 96.8.
 template <typename T, int K, int BS, bool LIFT = false>
 __global__ void __launch_bounds__(kBlock)
     row_vector_k(std::int32_t nplan, std::int32_t nc, const std::int32_t* __restrict__ inc_off,
@@ -3788,9 +3790,11 @@ __device__ inline float row_bcast(float v)
 /// mask) is one value per lane, handed on by row broadcasts.
 /// Teams of 10 lanes that each loaded the whole record and S (176 bytes per
 /// lane and step) kept the data return of the vector memory path busy 97 % of
-/// the time; now the vector ALU is busy half of the time and the LDS adds 44 %,
+/// the time; it still is 96 % (edge rows) and 94 % (vertex rows), for 0.58 of
+/// the load instructions, the vector ALU 52 and 34 % and the LDS 43 and 49 %,
 /// with 20 wavefronts per CU by LDS and registers. 48^3 cubes (25.8 M blocks,
-/// 1.85 GB): 0.90 ms for both kinds of rows against 1.27 ms. Resident
+/// 1.85 GB): 0.54 ms for the edge rows and 0.34 ms for the vertex rows against
+/// 1.27 ms. Resident
 /// wavefronts that prefetch the next group were slower (1.24 ms), so were
 /// plain stores (1.02 ms; non-temporal ones keep the records in the L2).
 template <typename T, typename O, int KIND>
@@ -4389,6 +4393,7 @@ void ensure_teams(dfx_form& f, const dfx_csr& A, std::size_t tsize)
     e = 0;
   if (A.nrows == 0)
     return;
+  // (rows are accepted up to this length, at ten values a block; nine are used)
   require(10 * std::int64_t(A.max_row) <= most, "row too long for the LDS slice");
   const std::int32_t nplan = f.max_dof + 1;
   std::vector<std::int32_t> off(nplan + 1), rp(A.nrows + 1);

@@ -1350,8 +1350,10 @@ void materialize_zero(const dfx_csr& A)
 /// The stream SpMV row blocks of A as (first row, first entry) pairs.
 inline const int2* row_blocks(const dfx_csr& A) { return reinterpret_cast<const int2*>(A.rblk); }
 
-/// Queries the resident grids of the stream SpMV kernels once, at matrix
-/// creation, so that no solve pays for the first occupancy query.
+/// Queries the resident grids of the row-lane and stream SpMV kernels once, at
+/// matrix creation, so that no solve pays for the first occupancy query (the
+/// block stream kernels of rows longer than bsr_chunk's 1024 tasks make theirs
+/// at their first product).
 void prime_stream_grids()
 {
   static std::once_flag once;
@@ -1372,6 +1374,14 @@ void prime_stream_grids()
                                       reinterpret_cast<const void*>(bsr_stream_k<float, 2, 1024, true>)};
                    for (const void* f : k)
                      resident_blocks(f, kBlock, 0);
+                   const void* rows[]
+                       = {reinterpret_cast<const void*>(spmv_rows_k<double, row_lane_steps(27)>),
+                          reinterpret_cast<const void*>(spmv_rows_k<double, kRowLaneMax>),
+                          reinterpret_cast<const void*>(spmv_rows_k<float, row_lane_steps(16)>),
+                          reinterpret_cast<const void*>(spmv_rows_k<float, row_lane_steps(27)>),
+                          reinterpret_cast<const void*>(spmv_rows_k<float, kRowLaneMax>)};
+                   for (const void* f : rows)
+                     resident_blocks(f, 2 * kRowGroup, 0);
                  });
 }
 
