@@ -3791,7 +3791,7 @@ __device__ inline float row_bcast(float v)
 /// Teams of 10 lanes that each loaded the whole record and S (176 bytes per
 /// lane and step) kept the data return of the vector memory path busy 97 % of
 /// the time; it still is 96 % (edge rows) and 94 % (vertex rows), for 0.58 of
-/// the load instructions, the vector ALU 52 and 34 % and the LDS 43 and 49 %,
+/// the load instructions, the vector ALU 52 and 34 % and the LDS 44 and 50 %,
 /// with 20 wavefronts per CU by LDS and registers. 48^3 cubes (25.8 M blocks,
 /// 1.85 GB): 0.54 ms for the edge rows and 0.34 ms for the vertex rows against
 /// 1.27 ms. Resident

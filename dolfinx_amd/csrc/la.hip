@@ -1931,7 +1931,7 @@ int pair_blocks(std::int64_t n)
 // always drains. Same stop test and FP64 reductions as the other
 // paths; sums are grouped differently, so the last bits (and
 // at most an iteration) may differ from it. P1 on 32^3 cubes (36,000 rows, 71
-// workgroups): 13.9 us per iteration, 18.2 us with the rows read again in
+// workgroups): 13.2 us per iteration, 18.4 us with the rows read again in
 // every iteration.
 // ---------------------------------------------------------------------
 
