@@ -134,9 +134,10 @@ class MatrixCSR:
 
     def set_lanes(self, lanes):
         """SpMV kernel of mult: 0 default (a lane per row of a large matrix
-        of short, scattered rows, otherwise the row-block stream), 1 row-block stream,
-        2..64 lanes per row, -1 the solvers' sliced-ELL copy of the values as
-        they are now (set again after the values change)."""
+        of short, scattered rows, otherwise the row-block stream), 1
+        row-block stream, 2..64 lanes per row, -1 the solvers' sliced-ELL
+        copy of the values as they are now (set again after the values
+        change)."""
         _lib.call("dfx_csr_set_lanes", self._h, int(lanes))
 
     def mult(self, x, y):

@@ -370,8 +370,9 @@ dfx_status dfx_form_autotune(dfx_form* a, dfx_csr* A, const dfx_bc* bc,
  * cell factors; 17 such teams gathering the matrix-core element matrices
  * of 7; 18 P1 rows by 16 lanes, a lane per incidence and then per entry.
  * Without a call the library chooses a variant for the element, the mesh and
- * the number of rows. The P2 elasticity form has a single row kernel and
- * ignores the variant. */
+ * the number of rows (inside a graph capture, where no plan can be built, one
+ * that needs only what earlier calls left). The P2 elasticity form has a
+ * single row kernel and ignores the variant. */
 dfx_status dfx_form_set_variant(dfx_form* a, int32_t variant);
 /* fem::assemble_matrix / fem::assemble_vector with a custom kernel
  * (cpp/demo/custom_kernel/main.cpp:73-118): the form (kernel
